@@ -115,15 +115,12 @@ __device__ __forceinline__ bool rebuild_pending(const uint32_t* flags) {
   return __hip_atomic_load(flags + RUMDX_FLAG_REBUILD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
 }
 
-// Called by every block of the final build kernel after its work: the block
-// that finishes last clears the rebuild request and counts the build.
-__device__ __forceinline__ void finish_build(uint32_t* flags) {
-  if (last_to_arrive(flags + RUMDX_FLAG_DONE, gridDim.x) && threadIdx.x == 0) {
-    flags[RUMDX_FLAG_REBUILD] = 0u;
-    flags[RUMDX_FLAG_BUILDS] += 1u;
-    flags[RUMDX_FLAG_EXCL_PENDING] = 1u;
-    flags[RUMDX_FLAG_PRUNE] = 1u;
-  }
+// Clears the rebuild request and counts the build (one thread of the launch).
+__device__ __forceinline__ void complete_build(uint32_t* flags) {
+  flags[RUMDX_FLAG_REBUILD] = 0u;
+  flags[RUMDX_FLAG_BUILDS] += 1u;
+  flags[RUMDX_FLAG_EXCL_PENDING] = 1u;
+  flags[RUMDX_FLAG_PRUNE] = 1u;
 }
 
 // ------------------------------------------------------------------ skin check
@@ -143,51 +140,83 @@ __global__ void k_request_rebuild(uint32_t* flags) {
 }
 
 // ------------------------------------------------------------------ N2 build
-// All pairs in slot order, positions staged through LDS.  List entries come out
-// in ascending j (RUMD's atomicInc order is unspecified; only sets compare).
-__global__ __launch_bounds__(kBlock) void k_build_n2(const float4* __restrict__ r, float4* __restrict__ last_r,
-                                                     uint32_t* __restrict__ nbl, uint32_t* __restrict__ num_nbrs,
-                                                     uint32_t* __restrict__ flags, const float* __restrict__ cut_skin2,
-                                                     uint32_t nt, Box bx, uint32_t n, uint32_t nvp,
-                                                     uint32_t max_nbrs, Exclusions ex) {
+// All pairs, list entries in ascending j (RUMD's atomicInc order is
+// unspecified; only sets compare).  A wave owns one particle and tests it
+// against 64 candidates at a time, one per lane: a ballot places the accepted
+// ones in candidate order, so the list needs no serial append.  The candidates
+// pass through LDS kN2Block at a time, shared by the workgroup's sixteen
+// waves; the next ones are read while these are tested.  Bound by the VALU
+// work of the n^2 tests; with a thread per particle it was the serial walk of
+// n / 256 workgroups over all n candidates (207 -> 10 us at n = 1000,
+// 845 -> 36 us at n = 5001).  Two or four particles per wave share each LDS
+// read but leave too few waves in flight (47 and 80 us at n = 5001).
+//
+// Arrivals are counted at the block's start, after its request read, so the
+// atomic's round trip overlaps the work; the block that starts last completes
+// the build.
+constexpr uint32_t kN2Block = 1024;
+
+__global__ __launch_bounds__(kN2Block) void k_build_n2(const float4* __restrict__ r, float4* __restrict__ last_r,
+                                                       uint32_t* __restrict__ nbl, uint32_t* __restrict__ num_nbrs,
+                                                       uint32_t* __restrict__ flags,
+                                                       const float* __restrict__ cut_skin2, uint32_t nt, Box bx,
+                                                       uint32_t n, uint32_t nvp, uint32_t max_nbrs, Exclusions ex) {
   if (!rebuild_pending(flags)) return;
-  extern __shared__ float4 s_dyn[];
-  float4* s_r = s_dyn;
-  float* s_cut = reinterpret_cast<float*>(s_dyn + kBlock);
-  for (uint32_t k = threadIdx.x; k < nt * nt; k += kBlock) s_cut[k] = cut_skin2[k];
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  extern __shared__ float s_cut[];
+  __shared__ float4 s_r[kN2Block];
+  __shared__ uint32_t s_max[kN2Block / 64];
+  for (uint32_t k = threadIdx.x; k < nt * nt; k += kN2Block) s_cut[k] = cut_skin2[k];
+  const uint32_t lane = threadIdx.x & 63u;
+  // this wave's particle (wave-uniform); the last workgroup's spare waves
+  // stage candidates and test none
+  const uint32_t i = __builtin_amdgcn_readfirstlane(blockIdx.x * (kN2Block / 64) + (threadIdx.x >> 6));
   const bool live = i < n;
-  const float4 ri = live ? r[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-  const uint32_t ti = __float_as_uint(ri.w);
-  const ExclusionRange er = live ? ex.of(i) : ExclusionRange{};
+  const float4 ri = r[live ? i : n - 1u];
+  const float* cut = s_cut + nt * __float_as_uint(ri.w);
+  const ExclusionRange er = ex.of(live ? i : n - 1u);
+  const uint64_t below = (1ull << lane) - 1ull;
   uint32_t cnt = 0;
-  for (uint32_t base = 0; base < n; base += kBlock) {
+  bool last = false;
+  float4 next = r[threadIdx.x < n ? threadIdx.x : n - 1u];
+  for (uint32_t base = 0; base < n; base += kN2Block) {
+    __syncthreads();  // the first one: every wave of the block has read the request
+    if (base == 0 && threadIdx.x == 0)
+      last = __hip_atomic_fetch_add(flags + RUMDX_FLAG_DONE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+             gridDim.x - 1;
+    s_r[threadIdx.x] = next;
     __syncthreads();
-    if (base + threadIdx.x < n) s_r[threadIdx.x] = r[base + threadIdx.x];
-    __syncthreads();
-    const uint32_t m = (n - base) < kBlock ? (n - base) : kBlock;
-    if (live) {
-      for (uint32_t k = 0; k < m; ++k) {
-        const uint32_t j = base + k;
-        if (j == i) continue;
-        const float4 rj = s_r[k];
-        const float d2 = min_image_d2_f32(ri, rj, bx);
-        if (d2 < s_cut[ti * nt + __float_as_uint(rj.w)] && !ex.excludes(er, j)) {
-          if (cnt < max_nbrs) nbl[static_cast<size_t>(cnt) * nvp + i] = j;
-          ++cnt;  // keeps counting past capacity: the true length sizes the regrowth
-        }
+    const uint32_t jn = base + kN2Block + threadIdx.x;
+    next = r[jn < n ? jn : n - 1u];
+    const uint32_t m = live ? min(n - base, kN2Block) : 0u;
+    for (uint32_t q = 0; q < m; q += 64u) {
+      const uint32_t j = base + q + lane;
+      const float4 rj = s_r[q + lane];
+      bool in = j < n && j != i && min_image_d2_f32(ri, rj, bx) < cut[__float_as_uint(rj.w)];
+      if (in) in = !ex.excludes(er, j);
+      const uint64_t hit = __builtin_amdgcn_ballot_w64(in);
+      if (in) {
+        const uint32_t k = cnt + static_cast<uint32_t>(__builtin_popcountll(hit & below));
+        if (k < max_nbrs) nbl[static_cast<size_t>(k) * nvp + i] = j;
       }
+      // keeps counting past capacity: the true length sizes the regrowth
+      cnt += static_cast<uint32_t>(__builtin_popcountll(hit));
     }
   }
-  if (live) {
+  if (live && lane == 0) {
     last_r[i] = ri;
     num_nbrs[i] = cnt < max_nbrs ? cnt : max_nbrs;  // == max_nbrs marks an overflowed list
     if (cnt >= max_nbrs) flags[RUMDX_FLAG_OVERFLOW] = 1u;
   }
-  __shared__ uint32_t s_max[kBlock / 64];
-  const uint32_t longest = block_max_u32(live ? cnt : 0u, s_max);
-  if (threadIdx.x == 0) atomicMax(flags + RUMDX_FLAG_MAXLEN, longest);
-  finish_build(flags);
+  const uint32_t longest = block_max_u32(cnt, s_max);
+  if (threadIdx.x == 0) {
+    // an atomic only where the block raises the figure: rarely after the first build
+    if (longest > __hip_atomic_load(flags + RUMDX_FLAG_MAXLEN, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(flags + RUMDX_FLAG_MAXLEN, longest);
+    if (last) {
+      flags[RUMDX_FLAG_DONE] = 0u;
+      complete_build(flags);
+    }
+  }
 }
 
 // ------------------------------------------------------------------ sorted build
@@ -1108,10 +1137,7 @@ __global__ __launch_bounds__(kBuildBlock) void k_build_tiles(uint32_t* __restric
     // waits on a same-address atomic
     s.tile_max[t] = longest;
     if (last) {
-      flags[RUMDX_FLAG_REBUILD] = 0u;
-      flags[RUMDX_FLAG_BUILDS] += 1u;
-      flags[RUMDX_FLAG_EXCL_PENDING] = 1u;
-      flags[RUMDX_FLAG_PRUNE] = 1u;
+      complete_build(flags);
       flags[RUMDX_FLAG_STATS] = 1u;
     }
     if (h.npart > 65535u) atomicOr(flags + RUMDX_FLAG_ERROR, RUMDX_BUILD_ERR_HALO);
@@ -1299,8 +1325,8 @@ extern "C" int rumdx_nblist_build_n2(const rumdx_particles* p, rumdx_nblist* nb,
   if (nb->excl_start_dev != nullptr && (nb->excl_ids_dev == nullptr || p->unsorted_index_dev == nullptr))
     return fail(RUMDX_E_INVALID, "rumdx_nblist_build_n2: exclusions need the exclusion ids and the unsorted index");
   if (p->n == 0) return RUMDX_OK;
-  const size_t lds = sizeof(float4) * kBlock + sizeof(float) * nb->ntypes * nb->ntypes;
-  hipLaunchKernelGGL(k_build_n2, dim3(blocks_for(p->n)), dim3(kBlock), lds, as_stream(stream),
+  const size_t lds = sizeof(float) * nb->ntypes * nb->ntypes;
+  hipLaunchKernelGGL(k_build_n2, dim3(blocks_for(p->n, kN2Block / 64)), dim3(kN2Block), lds, as_stream(stream),
                      reinterpret_cast<const float4*>(p->r_dev), reinterpret_cast<float4*>(nb->last_r_dev),
                      nb->nbl_dev, nb->num_nbrs_dev, nb->flags_dev, nb->cut_skin2_dev, nb->ntypes, make_box(box), p->n,
                      p->nvp, nb->max_nbrs, Exclusions{p->unsorted_index_dev, nb->excl_start_dev, nb->excl_ids_dev});

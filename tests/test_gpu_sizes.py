@@ -1,0 +1,55 @@
+"""Kernels at the sizes where their work split changes: remainders of a wave or
+workgroup, both sides of a size rule, the smallest and larger samples."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle
+from capi import GpuSystem, check, gpu_available, lib
+from helpers import FORCE_TOL_GUARDED, force_errors, ka_table, unsort
+from rumd_amd import configs
+
+pytestmark = pytest.mark.gpu
+
+SP, SF, NS = 1, 2, 0
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _need_gpu():
+    if not gpu_available():
+        pytest.fail("no GPU visible: the gpu tests must run on an MI355X")
+
+
+def _ka(n, seed=7, jitter=0.02, density=1.2):
+    s = configs.ka_random_lattice(n, density=density, seed=seed)
+    rng = np.random.default_rng(seed + 1)
+    pos = s.positions + rng.uniform(-jitter, jitter, size=s.positions.shape)
+    pos -= s.box * np.rint(pos / s.box)
+    return s, configs.pack_pos4(pos.astype(np.float32), s.types)
+
+
+def _gpu(s, pos4, method, **kw):
+    return GpuSystem(pos4, configs.pack_vel4(s.velocities, s.types, s.masses), configs.box8(s.box), 2, ka_table(),
+                     method=method, **kw)
+
+
+# a wave per particle, sixteen per workgroup, candidates 1,024 at a time
+@pytest.mark.parametrize("n", [2, 16, 17, 1023, 1024, 1025, 4099])
+def test_n2_lists_at_the_edges_of_the_wave_split(n):
+    s, pos4 = _ka(n)
+    g = _gpu(s, pos4, "n2", max_nbrs=n + 1)
+    print(f"[case] n2 lists n={n}", flush=True)
+    g.update_nblist()
+    # a second build starts from the counters the first one left
+    check(lib().rumdx_nblist_request_rebuild(C.byref(g.nb), None))
+    g.update_nblist()
+    cnt, nbl = g.neighbor_lists()
+    off, idx = oracle.nblist_brute_f32(pos4, configs.box8(s.box), 2, configs.cut_skin2_table(ka_table(), 0.3))
+    for i in range(n):
+        assert np.array_equal(nbl[: cnt[i], i], np.sort(idx[off[i]:off[i + 1]])), i
+    flags = g.flags_host()
+    # (no rebuild pending, no overflow, two builds, the longest list, counter at zero)
+    assert flags[:5].tolist() == [0, 0, 2, cnt.max(), 0]
