@@ -53,3 +53,18 @@ def test_n2_lists_at_the_edges_of_the_wave_split(n):
     flags = g.flags_host()
     # (no rebuild pending, no overflow, two builds, the longest list, counter at zero)
     assert flags[:5].tolist() == [0, 0, 2, cnt.max(), 0]
+
+
+# a wave per particle, four per workgroup, partners 512 at a time
+@pytest.mark.parametrize("n", [2, 3, 65, 511, 513, 1027])
+@pytest.mark.parametrize("stress", [False, True])
+def test_all_pairs_at_the_edges_of_the_partner_tiles(n, stress):
+    s, pos4 = _ka(n)
+    g = _gpu(s, pos4, "none", with_sts=stress)
+    print(f"[case] all pairs n={n} stress={stress}", flush=True)
+    f_ref, _ = oracle.forces_brute(pos4, s.box, 2, ka_table(), SF)
+    g.calc_f(SF, stress=stress)
+    f = g.get("f")[:n]
+    assert force_errors(f[:, :3], f_ref[:, :3])["guarded_max"] <= FORCE_TOL_GUARDED
+    g.calc_f(SF, initialize=False, stress=stress)  # added to the first call's
+    np.testing.assert_allclose(g.get("f")[:n], 2 * f, rtol=0, atol=2e-6 * np.abs(f).max())
