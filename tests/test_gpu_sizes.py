@@ -68,3 +68,36 @@ def test_all_pairs_at_the_edges_of_the_partner_tiles(n, stress):
     assert force_errors(f[:, :3], f_ref[:, :3])["guarded_max"] <= FORCE_TOL_GUARDED
     g.calc_f(SF, initialize=False, stress=stress)  # added to the first call's
     np.testing.assert_allclose(g.get("f")[:n], 2 * f, rtol=0, atol=2e-6 * np.abs(f).max())
+
+
+# one, two and four workgroups per tile (27, 125 and 512 tiles), wrapping tiles
+# with and without the shifted frame, FP64 positions
+@pytest.mark.parametrize("n,cutoff,stress", [(2500, SF, False), (2500, SP, True), (19001, NS, False),
+                                             (19001, SF, True), (95003, SF, False)])
+def test_fp64_tiles_at_each_split(n, cutoff, stress):
+    s, pos4 = _ka(n)
+    g = _gpu(s, pos4, "sorted", max_nbrs=200, with_sts=stress)
+    print(f"[case] fp64 tiles n={n} tiles={g.nb.ntiles} cutoff={cutoff} stress={stress}", flush=True)
+    g.calc_f(cutoff, fp64=True, stress=stress)
+    uidx = g.unsorted_index()
+    f = unsort(g.get("f"), uidx)
+    f_ref, _ = oracle.forces_cells(pos4, s.box, 2, ka_table(), cutoff)
+    # the output's rounding (2^-24) and the float parameters the oracle shares
+    assert force_errors(f[:, :3], f_ref[:, :3])["guarded_max"] <= 2e-7
+    if stress:
+        sts = unsort(g.get("sts"), uidx)
+        sts_ref = oracle.stress_brute(pos4, s.box, 2, ka_table(), cutoff) if n < 5000 else None
+        if sts_ref is not None:
+            np.testing.assert_allclose(sts[:, :3], sts_ref[:, :3], rtol=0, atol=2e-7 * np.abs(sts_ref).max())
+
+
+# list lanes and the all-pairs wave of the FP64 slot kernel
+@pytest.mark.parametrize("method,n", [("n2", 3), ("n2", 17), ("n2", 1003), ("none", 3), ("none", 333)])
+def test_fp64_slots_with_shared_lanes(method, n):
+    s, pos4 = _ka(n)
+    g = _gpu(s, pos4, method)
+    print(f"[case] fp64 slots {method} n={n}", flush=True)
+    g.calc_f(SF, fp64=True)
+    f = unsort(g.get("f"), g.unsorted_index())
+    f_ref, _ = oracle.forces_brute(pos4, s.box, 2, ka_table(), SF)
+    assert force_errors(f[:, :3], f_ref[:, :3])["guarded_max"] <= 2e-7
