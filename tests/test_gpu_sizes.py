@@ -9,7 +9,8 @@ import pytest
 
 import oracle
 from capi import GpuSystem, check, gpu_available, lib
-from helpers import FORCE_TOL_GUARDED, force_errors, ka_table, unsort
+from helpers import FORCE_TOL_GUARDED, force_errors, ka_table, load_golden, unsort
+from test_gpu_potentials import PE_ATOL, _forms, _table
 from rumd_amd import configs
 
 pytestmark = pytest.mark.gpu
@@ -101,3 +102,23 @@ def test_fp64_slots_with_shared_lanes(method, n):
     f = unsort(g.get("f"), g.unsorted_index())
     f_ref, _ = oracle.forces_brute(pos4, s.box, 2, ka_table(), SF)
     assert force_errors(f[:, :3], f_ref[:, :3])["guarded_max"] <= 2e-7
+
+
+# the kernels compiled per form (no stresses, initialising), every cut-off and list method
+@pytest.mark.parametrize("case", _forms(), ids=lambda c: c[0])
+def test_forms_without_stresses(golden_dir, case):
+    name, form, make, rows = case
+    c = load_golden(golden_dir / "KA_N1000_T0.466.xyz.gz")
+    pos4 = configs.pack_pos4(c.positions, c.types)
+    for cutoff in (NS, SP, SF):
+        table = _table(make, cutoff, rows)
+        f_ref, _ = oracle.forces_form_brute(pos4, c.box, 2, table, form, cutoff)
+        for method in ("sorted", "n2", "none"):
+            g = GpuSystem(pos4, configs.pack_vel4(c.velocities, c.types, c.masses), configs.box8(c.box), 2, table,
+                          method=method)
+            print(f"[case] form {name} cutoff={cutoff} method={method}", flush=True)
+            g.calc_f(cutoff, form=form)
+            f = unsort(g.get("f"), g.unsorted_index())
+            assert force_errors(f[:, :3], f_ref[:, :3])["guarded_max"] <= FORCE_TOL_GUARDED
+            pe_tol = max(PE_ATOL, 2e-6 * np.abs(f_ref[:, 3]).max())
+            np.testing.assert_allclose(f[:, 3], f_ref[:, 3], rtol=0, atol=pe_tol)
