@@ -28,9 +28,13 @@ void Sample::SetPB_TP(unsigned pb, unsigned tp) {
   if (GetNumberOfParticles()) {
     // reallocate with the new padding, keeping the configuration
     const unsigned n = GetNumberOfParticles();
-    std::vector<float> r(4ull * n), v(4ull * n), im(4ull * n);
+    std::vector<float> r(4ull * n), v(4ull * n), im(4ull * n), lo;
     std::vector<int32_t> t(n);
     pd_.Get("r", r.data(), stream_);
+    if (pd_.MixedPositions()) {
+      lo.resize(4ull * n);
+      pd_.Get("rlo", lo.data(), stream_);
+    }
     pd_.Get("v", v.data(), stream_);
     pd_.Get("im", im.data(), stream_);
     pd_.GetTypes(t.data(), stream_);
@@ -43,7 +47,15 @@ void Sample::SetPB_TP(unsigned pb, unsigned tp) {
     std::vector<float> x3(3ull * n);
     for (unsigned i = 0; i < n; ++i)
       for (int k = 0; k < 3; ++k) x3[3ull * i + k] = r[4ull * i + k];
-    pd_.SetPositions(x3.data(), stream_);
+    if (!lo.empty() && mixed_) {
+      std::vector<double> x64(3ull * n);
+      for (unsigned i = 0; i < n; ++i)
+        for (int k = 0; k < 3; ++k)
+          x64[3ull * i + k] = static_cast<double>(r[4ull * i + k]) + static_cast<double>(lo[4ull * i + k]);
+      pd_.SetPositionsFP64(x64.data(), stream_);
+    } else {
+      pd_.SetPositions(x3.data(), stream_);
+    }
     for (unsigned i = 0; i < n; ++i)
       for (int k = 0; k < 3; ++k) x3[3ull * i + k] = v[4ull * i + k];
     pd_.SetVelocities(x3.data(), stream_);

@@ -11,7 +11,7 @@ import oracle
 from capi import GpuSystem, check, gpu_available, lib
 from helpers import FORCE_TOL_GUARDED, force_errors, ka_table, load_golden, unsort
 from test_gpu_potentials import PE_ATOL, _forms, _table
-from rumd_amd import configs
+from rumd_amd import conf_io, configs, rumd
 
 pytestmark = pytest.mark.gpu
 
@@ -122,3 +122,21 @@ def test_forms_without_stresses(golden_dir, case):
             assert force_errors(f[:, :3], f_ref[:, :3])["guarded_max"] <= FORCE_TOL_GUARDED
             pe_tol = max(PE_ATOL, 2e-6 * np.abs(f_ref[:, 3]).max())
             np.testing.assert_allclose(f[:, 3], f_ref[:, 3], rtol=0, atol=pe_tol)
+
+
+def test_new_padding_keeps_the_fp64_positions():
+    """SetPB_TP reallocates the particle arrays; in mixed-precision mode the
+    low-order position parts stay with the configuration."""
+    s, _ = _ka(500)
+    sample = rumd.Sample(0, 0)
+    sample.SetVerbose(False)
+    sample.SetMixedPrecisionPositions(True)
+    sample.SetConfiguration(conf_io.Configuration(
+        n=s.n, box=s.box, types=s.types, positions=s.positions, masses=s.masses, velocities=s.velocities,
+        images=np.zeros_like(s.positions)))
+    pos64 = s.positions.astype(np.float64) * (1.0 + 1e-8)
+    sample.SetPositionsFP64(pos64)
+    before = sample.GetPositionsFP64()
+    assert np.abs(before - pos64).max() < 1e-12
+    sample.SetPB_TP(64, 8)
+    np.testing.assert_array_equal(sample.GetPositionsFP64(), before)
