@@ -83,11 +83,14 @@ extern "C" {
 #define RUMDX_FLAG_MAXTILE 8   /* most particles in one cell tile, last sorted build, after rumdx_nblist_build_stats */
 #define RUMDX_FLAG_PRUNE 9     /* != 0: the next rumdx_nblist_prune rebuilds the inner lists */
 #define RUMDX_FLAG_STATS 10    /* internal: set by a completed sorted build, cleared by rumdx_nblist_build_stats */
+#define RUMDX_FLAG_CHAIN 12    /* internal: three words of rumdx_pair_lj_small_step, zero between chains */
 /* Bits of flags[RUMDX_FLAG_ERROR]. */
 #define RUMDX_BUILD_ERR_HALO 1u     /* a tile halo held more than 65535 particles */
 #define RUMDX_BUILD_ERR_MOVED 2u    /* rebuild_sorted: a particle moved more than one cell since the last build */
 #define RUMDX_BUILD_ERR_WAIT 4u     /* rebuild_sorted: a tile's wait for the tiles before it timed out */
 #define RUMDX_BUILD_ERR_TILE 8u     /* rebuild_sorted: a tile held more than RUMDX_RESORT_TILE_MAX particles */
+/* Largest sample of the one-kernel steps (rumdx_pair_lj_small_step). */
+#define RUMDX_SMALL_STEP_MAX 16384u
 /* Particles one tile may hold for rumdx_nblist_rebuild_sorted. */
 #define RUMDX_RESORT_TILE_MAX 2048u
 
@@ -436,6 +439,26 @@ int rumdx_nvt_step(rumdx_particles* p, rumdx_nh_state* nh_dev, float dt, uint32_
 int rumdx_pair_lj_nvt(const rumdx_particles* p, const rumdx_nblist* nb, const float* params_dev, uint32_t ntypes,
                       const float box[8], int cutoff_method, float* r_out_dev, rumdx_nh_state* nh_dev, float dt,
                       uint32_t thermostat_on_mask, float omega2, uint32_t dof, void* workspace_dev, void* stream);
+
+/* Steps of a small sample (n <= RUMDX_SMALL_STEP_MAX) whose only force term is
+ * a 12-6 pair potential over a list of the N2 method, or over all pairs (nb ==
+ * NULL), one kernel each: rumdx_nblist_build_n2 when flags[REBUILD] asks,
+ * rumdx_pair_lj with initialize = 1, and rumdx_nvt_step.  Called for step = 0,
+ * 1, 2, ... of a chain, the caller swapping p->r_dev and r_out_dev after each,
+ * then once rumdx_small_steps_end with the number of steps; nothing else may
+ * use the list's flags, the thermostat state or the workspace in between (the
+ * thermostat's update and the rebuild request of a step are taken up by the
+ * next one).  f and w are stored when store_forces is nonzero; otherwise they
+ * are left undefined until a later step of the chain stores them.  Positions,
+ * velocities, images, forces, lists and the thermostat state after the end are
+ * the same bits as from the three calls. */
+int rumdx_pair_lj_small_step(const rumdx_particles* p, rumdx_nblist* nb, const float* params_dev, uint32_t ntypes,
+                             const float box[8], int cutoff_method, float* r_out_dev, rumdx_nh_state* nh_dev, float dt,
+                             uint32_t thermostat_on_mask, float omega2, uint32_t dof, uint32_t step, int store_forces,
+                             void* workspace_dev, void* stream);
+int rumdx_small_steps_end(const rumdx_particles* p, rumdx_nblist* nb, rumdx_nh_state* nh_dev, float dt,
+                          uint32_t thermostat_on_mask, float omega2, uint32_t dof, uint32_t steps,
+                          void* workspace_dev, void* stream);
 
 /* IntegratorNVT::SetMomentumToZero (src/IntegratorNVT.cu:176-183, 444-472):
  * subtracts the centre-of-mass velocity, with the momentum sum in FP64. */

@@ -83,8 +83,13 @@ __global__ __launch_bounds__(kBlock) void k_nvt(NvtArgs a, Box bx) {
     }
   }
   if (THERMO) {
-    const double s = block_sum(static_cast<double>(ke2), s_red);
-    if (threadIdx.x == 0) a.partials[b] = s;
+    if (a.n <= kSmallStepMax) {
+      const double s = group_sum(static_cast<double>(ke2));
+      if (i < a.n && i % kSmallGroup == 0) a.partials[i / kSmallGroup] = s;
+    } else {
+      const double s = block_sum(static_cast<double>(ke2), s_red);
+      if (threadIdx.x == 0) a.partials[b] = s;
+    }
   }
 }
 
@@ -183,7 +188,7 @@ void launch_nvt(const NvtArgs& a, const Box& bx, hipStream_t st) {
   const uint32_t nb = blocks_for(a.n);
   hipLaunchKernelGGL((k_nvt<THERMO, HILO, SKIN>), dim3(nb), dim3(kBlock), 0, st, a, bx);
   if (THERMO)
-    hipLaunchKernelGGL(k_nvt_finish, dim3(1), dim3(kBlock), 0, st, a.partials, nb, a.nh, a.dt, a.omega2, a.dof);
+    hipLaunchKernelGGL(k_nvt_finish, dim3(1), dim3(kBlock), 0, st, a.partials, ke_partials(a.n), a.nh, a.dt, a.omega2, a.dof);
 }
 
 }  // namespace
@@ -196,7 +201,7 @@ extern "C" int rumdx_version(void) { return RUMDX_VERSION; }
 extern "C" const char* rumdx_last_error(void) { return g_last_error.c_str(); }
 
 extern "C" size_t rumdx_workspace_bytes(uint32_t n) {
-  return Workspace::kPartials + sizeof(double) * 4 * static_cast<size_t>(blocks_for(n > 0 ? n : 1));
+  return Workspace::kPartials + sizeof(double) * Workspace::partial_doubles(n);
 }
 
 extern "C" int rumdx_nvt_step(rumdx_particles* p, rumdx_nh_state* nh_dev, float dt, uint32_t thermostat_on_mask,

@@ -103,12 +103,13 @@ __device__ __forceinline__ NvtIn nvt_fused_load(uint32_t i, const float4* __rest
   return in;
 }
 
-// One particle of the fused step: the update of k_nvt for slot i from its
-// force fi and state `in`; returns m v^2 when the particle is thermostatted,
-// else 0.
-__device__ __forceinline__ float nvt_fused(uint32_t i, float4 fi, NvtIn in, const NvtFuse& z, float ps,
-                                           const Box& bx) {
-  float4 ri = in.r;
+// One particle of a fused step: the update of k_nvt for slot i from its force
+// fi and state `in`; returns m v^2 when the particle is thermostatted, else 0.
+// With skin, `moved` tells whether it is beyond half the skin from the last
+// build.
+__device__ __forceinline__ float nvt_advance(uint32_t i, float4 fi, NvtIn in, const NvtFuse& z, float ps,
+                                             const Box& bx, float4& ri, bool& moved, bool skin) {
+  ri = in.r;
   const bool apply = z.nh != nullptr && ((z.on_mask >> (__float_as_uint(ri.w) & 31u)) & 1u);
   float3 shift;
   float ke;
@@ -121,26 +122,45 @@ __device__ __forceinline__ float nvt_fused(uint32_t i, float4 fi, NvtIn in, cons
   z.r_out[i] = ri;
   z.v[i] = in.v;
   add_image_shift(z.im, i, shift);
-  if (min_image_d2_f32(ri, in.last_r, bx) > z.skin2_over_4) z.nb_flags[RUMDX_FLAG_REBUILD] = 1u;
-  if (z.prune_r != nullptr && min_image_d2_f32(ri, z.prune_r[i], bx) > z.inner2) z.nb_flags[RUMDX_FLAG_PRUNE] = 1u;
+  moved = skin && min_image_d2_f32(ri, in.last_r, bx) > z.skin2_over_4;
   return apply ? ke : 0.f;
+}
+
+// The same with the flags of a list (rebuild, and prune of its inner lists)
+// raised as the particle's new position asks.
+__device__ __forceinline__ float nvt_fused(uint32_t i, float4 fi, NvtIn in, const NvtFuse& z, float ps,
+                                           const Box& bx) {
+  float4 ri;
+  bool moved;
+  const float ke = nvt_advance(i, fi, in, z, ps, bx, ri, moved, true);
+  if (moved) z.nb_flags[RUMDX_FLAG_REBUILD] = 1u;
+  if (z.prune_r != nullptr && min_image_d2_f32(ri, z.prune_r[i], bx) > z.inner2) z.nb_flags[RUMDX_FLAG_PRUNE] = 1u;
+  return ke;
+}
+
+// Ps += dt omega^2 min(KE2 / (dof T) - 1, 10) and the T ramp, from the sum of
+// m v^2 (UpdateThermostatState) in FP64.
+__device__ __forceinline__ void nh_advance(rumdx_nh_state& nh, double ke2, float dt, float omega2, uint32_t dof) {
+  double dev = ke2 / (static_cast<double>(dof) * nh.target_T) - 1.0;
+  if (dev > 10.0) dev = 10.0;  // runaway clamp (src/IntegratorNVT.cu:432-434)
+  nh.ps += static_cast<double>(dt) * static_cast<double>(omega2) * dev;
+  nh.ke2_sum = ke2;
+  nh.target_T += nh.dT_per_step;
 }
 
 namespace {
 
-// UpdateThermostatState in FP64: fixed-order sum of the block partials of
-// the integrator, then Ps += dt omega^2 min(KE2 / (dof T) - 1, 10) and the T
-// ramp.  One workgroup; the kernel boundary makes the partials visible.
+// UpdateThermostatState: fixed-order sum of the integrator's partials, then
+// the state's update.  One workgroup; the kernel boundary makes the partials
+// visible.
 __global__ __launch_bounds__(kBlock) void k_nvt_finish(const double* __restrict__ partials, uint32_t np,
                                                        rumdx_nh_state* nh, float dt, float omega2, uint32_t dof) {
   __shared__ double s_red[kBlock / 64];
   const double tot = sum_partials(partials, np, 1, s_red);
   if (threadIdx.x == 0) {
-    double dev = tot / (static_cast<double>(dof) * nh->target_T) - 1.0;
-    if (dev > 10.0) dev = 10.0;  // runaway clamp (src/IntegratorNVT.cu:432-434)
-    nh->ps += static_cast<double>(dt) * static_cast<double>(omega2) * dev;
-    nh->ke2_sum = tot;
-    nh->target_T += nh->dT_per_step;
+    rumdx_nh_state st = *nh;
+    nh_advance(st, tot, dt, omega2, dof);
+    *nh = st;
   }
 }
 

@@ -157,6 +157,13 @@ __device__ __forceinline__ double block_sum(double v, double* lds4) {
   return s;
 }
 
+// Sum of v over each 16 consecutive lanes, in every one of them.
+__device__ __forceinline__ double group_sum(double v) {
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
 // Maximum of v over the workgroup (lds4: blockDim.x / 64 entries), valid in thread 0.  Flags
 // that collect a maximum (the longest list) take one atomic per workgroup:
 // one per particle on a single address serialises at the memory side.
@@ -213,12 +220,31 @@ __device__ __forceinline__ double sum_partials(const double* partials, uint32_t 
 }
 
 // ------------------------------------------------------------------ workspace
+// Samples of at most kSmallStepMax particles keep one kinetic-energy partial
+// per kSmallGroup consecutive particles (larger ones per kBlock): the grain of
+// the one-kernel steps (small_step.h), so that every way of stepping a small
+// sample adds in one order.
+constexpr uint32_t kSmallGroup = 16;
+constexpr uint32_t kSmallStepMax = RUMDX_SMALL_STEP_MAX;
+inline __host__ __device__ uint32_t ke_partials(uint32_t n) {
+  const uint32_t g = n <= kSmallStepMax ? kSmallGroup : kBlock;
+  return (n + g - 1u) / g;
+}
+
 // Layout of the caller's reduction workspace.
 struct Workspace {
-  static constexpr size_t kCounters = 0;    // uint32[16]
   static constexpr size_t kScalars = 64;    // double[8] scratch results
-  static constexpr size_t kPartials = 256;  // double[4 * nblocks]
-  static uint32_t* counters(void* ws) { return reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + kCounters); }
+  static constexpr size_t kStates = 128;    // rumdx_nh_state[2]: the thermostat inside a chain of one-kernel steps
+  static constexpr size_t kPartials = 256;  // double[partial_doubles(n)]
+  // four sums per kBlock particles, or two sets of a small sample's partials
+  static size_t partial_doubles(uint32_t n) {
+    const size_t four = 4 * static_cast<size_t>(blocks_for(n > 0 ? n : 1));
+    const size_t two = n <= kSmallStepMax ? 2 * static_cast<size_t>(ke_partials(n > 0 ? n : 1)) : 0;
+    return four > two ? four : two;
+  }
+  static rumdx_nh_state* states(void* ws) {
+    return reinterpret_cast<rumdx_nh_state*>(static_cast<char*>(ws) + kStates);
+  }
   static double* scalars(void* ws) { return reinterpret_cast<double*>(static_cast<char*>(ws) + kScalars); }
   static double* partials(void* ws) { return reinterpret_cast<double*>(static_cast<char*>(ws) + kPartials); }
 };

@@ -9,9 +9,10 @@
 // (src/IntegratorNVT.cu:364-437).
 //
 // A small sample's step is bound by launches and by the chain of dependent
-// kernels, not by work: four kernels (build, forces, integrator, thermostat)
-// took 13-20 us at n = 500 to 4,099, most of it between them.  None of them
-// needs a grid-wide barrier inside a step:
+// reads, not by work: four kernels (build, forces, integrator, thermostat) took
+// 13 us a step at n = 500 without a list, 18 at n = 1000 and 19 at n = 4099,
+// most of it between them; one takes 7.5, 8.4 and 12 (rebuilds included).
+// None of the four needs a grid-wide barrier inside a step:
 //  - a list of the N2 method belongs to one particle and is built from the
 //    positions alone, so the workgroup that owns the particle rebuilds it when
 //    a rebuild is due and goes on to its forces;

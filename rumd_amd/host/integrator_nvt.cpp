@@ -65,10 +65,8 @@ void IntegratorNVT::PullState() {
 void IntegratorNVT::Integrate() {
   if (!S || !S->GetNumberOfParticles()) throw RUMD_Error("IntegratorNVT", "Integrate", kNoSample);
   if (!S->GetSimulationBox()) throw RUMD_Error("IntegratorNVT", "Integrate", "no simulation box");
-  // omega^2 = 4 pi^2 / tau^2 formed in double, passed as float (src/IntegratorNVT.cu:88)
-  const float omega2 = static_cast<float>(4. * M_PI * M_PI / (static_cast<double>(relaxation_time_) * relaxation_time_));
   NeighborList* nl = S->FusedCheckList();
-  rumdx_check(rumdx_nvt_step(S->GetParticleData().Descriptor(), d_state_.get(), timeStep, thermostat_on_, omega2,
+  rumdx_check(rumdx_nvt_step(S->GetParticleData().Descriptor(), d_state_.get(), timeStep, thermostat_on_, Omega2(),
                              S->GetNumberOfDOFs(), S->GetSimulationBox()->GetBox8(), nl ? nl->Descriptor() : nullptr,
                              S->Workspace(), S->GetStream()),
               "IntegratorNVT", "Integrate");
@@ -78,9 +76,19 @@ void IntegratorNVT::Integrate() {
 void IntegratorNVT::IntegrateFused(PairPotential& pp) {
   if (!S || !S->GetNumberOfParticles()) throw RUMD_Error("IntegratorNVT", "Integrate", kNoSample);
   if (!S->GetSimulationBox()) throw RUMD_Error("IntegratorNVT", "Integrate", "no simulation box");
-  const float omega2 = static_cast<float>(4. * M_PI * M_PI / (static_cast<double>(relaxation_time_) * relaxation_time_));
-  pp.CalcFIntegrateNVT(d_state_.get(), timeStep, thermostat_on_, omega2, S->GetNumberOfDOFs());
+  pp.CalcFIntegrateNVT(d_state_.get(), timeStep, thermostat_on_, Omega2(), S->GetNumberOfDOFs());
   pp.GetNeighborList().NoteFusedCheck();
+}
+
+void IntegratorNVT::IntegrateChain(PairPotential& pp, unsigned nsteps) {
+  // the forces of the inner steps are replaced before anything reads them
+  for (unsigned k = 0; k < nsteps; ++k)
+    pp.ChainStep(d_state_.get(), timeStep, thermostat_on_, Omega2(), S->GetNumberOfDOFs(), k, k + 1 == nsteps);
+  pp.EndChain(d_state_.get(), timeStep, thermostat_on_, Omega2(), S->GetNumberOfDOFs(), nsteps);
+}
+
+float IntegratorNVT::Omega2() const {
+  return static_cast<float>(4. * M_PI * M_PI / (static_cast<double>(relaxation_time_) * relaxation_time_));
 }
 
 std::string IntegratorNVT::GetInfoString(unsigned precision) const {

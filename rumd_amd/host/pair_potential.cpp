@@ -639,6 +639,35 @@ void PairPotential::CalcFIntegrateNVT(rumdx_nh_state* nh_dev, float dt, unsigned
   pd.SwapPositions();
 }
 
+bool PairPotential::CanChainSteps() {
+  return sample != nullptr && GetPotentialForm() == 0 && !fp64_forces_ &&
+         neighborList.GetResolvedMethod() != NeighborList::SORT &&
+         sample->GetNumberOfParticles() <= RUMDX_SMALL_STEP_MAX;
+}
+
+void PairPotential::ChainStep(rumdx_nh_state* nh_dev, float dt, unsigned thermostat_on_mask, float omega2, unsigned dof,
+                              unsigned step, bool store_forces) {
+  ParticleData& pd = sample->GetParticleData();
+  rumdx_nblist* nb = neighborList.GetResolvedMethod() == NeighborList::NONE ? nullptr : neighborList.Descriptor();
+  const float* box = sample->GetSimulationBox()->GetBox8();
+  const hipStream_t st = sample->GetStream();
+  if (step == 0 && nb != nullptr)
+    rumdx_check(rumdx_nblist_check(pd.Descriptor(), nb, box, st), GetID_String().c_str(), "ChainStep");
+  rumdx_check(rumdx_pair_lj_small_step(pd.Descriptor(), nb, d_params_.get(), table_types_, box, cutoff_method_,
+                                       pd.NextPositions(), nh_dev, dt, thermostat_on_mask, omega2, dof, step,
+                                       store_forces ? 1 : 0, sample->Workspace(), st),
+              GetID_String().c_str(), "ChainStep");
+  pd.SwapPositions();
+}
+
+void PairPotential::EndChain(rumdx_nh_state* nh_dev, float dt, unsigned thermostat_on_mask, float omega2, unsigned dof,
+                             unsigned steps) {
+  rumdx_nblist* nb = neighborList.GetResolvedMethod() == NeighborList::NONE ? nullptr : neighborList.Descriptor();
+  rumdx_check(rumdx_small_steps_end(sample->GetParticleData().Descriptor(), nb, nh_dev, dt, thermostat_on_mask, omega2,
+                                    dof, steps, sample->Workspace(), sample->GetStream()),
+              GetID_String().c_str(), "EndChain");
+}
+
 void PairPotential::SetFP64Forces(bool on) {
   if (on && GetPotentialForm() != 0)
     throw RUMD_Error(GetID_String(), "SetFP64Forces", "the all-FP64 comparison path serves the 12-6 potentials only");

@@ -311,6 +311,16 @@ class PairPotential : public Potential {
   // comparison path; FP32 pair arithmetic otherwise.
   void SetFP64Forces(bool on);
   bool GetFP64Forces() const { return fp64_forces_; }
+  // True when the steps of a captured block of a small sample whose only force
+  // term is this potential can run as one kernel each
+  // (rumdx_pair_lj_small_step): the 12-6 form in FP32 over an N2 list or over
+  // all pairs, at most RUMDX_SMALL_STEP_MAX particles.  ChainStep records step
+  // `step` of a block and swaps the position arrays; EndChain closes it.
+  bool CanChainSteps();
+  void ChainStep(rumdx_nh_state* nh_dev, float dt, unsigned thermostat_on_mask, float omega2, unsigned dof,
+                 unsigned step, bool store_forces);
+  void EndChain(rumdx_nh_state* nh_dev, float dt, unsigned thermostat_on_mask, float omega2, unsigned dof,
+                unsigned steps);
   // True when a step of a sample whose only force term is this potential can
   // run as one kernel (rumdx_pair_lj_nvt): the 12-6 form in FP32 over an
   // allocated list of the sorted method whose tiles fit the sample's
@@ -745,10 +755,14 @@ class IntegratorNVT : public Integrator {
   // The step with the forces of `pp` computed in the same kernel
   // (PairPotential::CalcFIntegrateNVT): CalcF and Integrate of Simulation.Run.
   void IntegrateFused(PairPotential& pp);
+  // nsteps steps as a chain of one-kernel steps (PairPotential::ChainStep).
+  void IntegrateChain(PairPotential& pp, unsigned nsteps);
 
  private:
   void PushState();
   void PullState();
+  // omega^2 = 4 pi^2 / tau^2 formed in double, passed as float (src/IntegratorNVT.cu:88)
+  float Omega2() const;
   unsigned thermostat_on_ = 0;
   float relaxation_time_ = 0.2f;
   rumdx_nh_state host_state_{0.0, 0.0, 0.0, 0.0};
@@ -900,6 +914,7 @@ class Sample {
     float* r_home;
   };
   void PrepareRun();
+  PairPotential* ChainPotential();
   void StepOnce(bool zero_momentum);
   Block CaptureBlock(unsigned nsteps, bool reset_first);
   unsigned pb_ = 0, tp_ = 0;

@@ -243,6 +243,14 @@ PairPotential* Sample::FusedStepPotential() {
   return (pp != nullptr && pp->CanFuseStep()) ? pp : nullptr;
 }
 
+// The potential whose steps run as chains of one kernel each inside captured
+// blocks (small samples), or null.
+PairPotential* Sample::ChainPotential() {
+  if (!fused_steps_ || potentials_.size() != 1 || dynamic_cast<IntegratorNVT*>(itg_) == nullptr) return nullptr;
+  auto* pp = dynamic_cast<PairPotential*>(potentials_.front());
+  return (pp != nullptr && pp->CanChainSteps()) ? pp : nullptr;
+}
+
 void Sample::PrepareRun() {
   if (!box_) throw RUMD_Error("Sample", "Run", "No simulation box has been set");
   if (!itg_) throw RUMD_Error("Sample", "Run", "Integrator has not been set");
@@ -257,7 +265,7 @@ void Sample::PrepareRun() {
       // re-sort of skin-triggered rebuilds (the build settles its capacities)
       if (nl.NeedsFullSort()) nl.UpdateNBlist();
     }
-  if (FusedStepPotential() != nullptr) pd_.EnsureNextPositions();
+  if (FusedStepPotential() != nullptr || ChainPotential() != nullptr) pd_.EnsureNextPositions();
 }
 
 void Sample::StepOnce(bool zero_momentum) {
@@ -302,7 +310,12 @@ Sample::Block Sample::CaptureBlock(unsigned nsteps, bool reset_first) {
     // the first step re-checks the skin explicitly; later steps use the
     // check fused into the previous integrator step
     if (nl) nl->ResetFusedCheck();
-    for (unsigned k = 0; k < nsteps; ++k) StepOnce(k == 0 && reset_first);
+    if (PairPotential* chain = ChainPotential()) {
+      if (reset_first) itg_->SetMomentumToZero();
+      static_cast<IntegratorNVT*>(itg_)->IntegrateChain(*chain, nsteps);
+    } else {
+      for (unsigned k = 0; k < nsteps; ++k) StepOnce(k == 0 && reset_first);
+    }
     // fused steps alternate the two position arrays: the graph ends in the
     // one it starts from (a copy after an odd number of them)
     pd_.MovePositionsTo(home, stream_);

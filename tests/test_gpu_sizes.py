@@ -140,3 +140,68 @@ def test_new_padding_keeps_the_fp64_positions():
     assert np.abs(before - pos64).max() < 1e-12
     sample.SetPB_TP(64, 8)
     np.testing.assert_array_equal(sample.GetPositionsFP64(), before)
+
+
+def _stepping_sample(n, method, thermo, mixed, T=2.0):
+    s, _ = _ka(n, jitter=0.0)
+    sample = rumd.Sample(0, 0)
+    sample.SetVerbose(False)
+    sample.SetMixedPrecisionPositions(mixed)
+    sample.SetConfiguration(conf_io.Configuration(
+        n=s.n, box=s.box, types=s.types, positions=s.positions, masses=s.masses,
+        velocities=2.0 * s.velocities, images=np.zeros_like(s.positions)))
+    pot = rumd.Pot_LJ_12_6(cutoff_method=rumd.ShiftedForce)
+    pot.SetVerbose(False)
+    for (i, j, sg, ep, rc) in configs.ka_params(2.5):
+        pot.SetParams(i, j, Sigma=sg, Epsilon=ep, Rcut=rc)
+    pot.SetNbListSkin(0.3)
+    pot.SetNB_Method(method)
+    sample.SetPotential(pot)
+    itg = rumd.IntegratorNVT(timeStep=0.0025, targetTemperature=T, thermostatRelaxationTime=0.2) if thermo else \
+        rumd.IntegratorNVE(timeStep=0.0025)
+    if thermo:
+        itg.SetTemperatureChangePerTimeStep(1e-4)
+    sample.SetIntegrator(itg)
+    return sample, pot, itg
+
+
+# one-kernel steps in chains of 7, 1, 2 and more against CalcF and Integrate:
+# remainders of the 16-particle groups, the largest size, rebuilds inside chains
+@pytest.mark.parametrize("n,method,thermo,mixed", [(40, "none", True, False), (531, "none", False, True),
+                                                   (203, "n2", True, False), (1003, "n2", False, False),
+                                                   (4099, "n2", True, True), (16384, "n2", True, False)])
+def test_one_kernel_steps_equal_the_separate_calls(n, method, thermo, mixed):
+    print(f"[case] small steps n={n} {method} thermo={thermo} mixed={mixed}", flush=True)
+    a, pot_a, itg_a = _stepping_sample(n, method, thermo, mixed)
+    b, pot_b, itg_b = _stepping_sample(n, method, thermo, mixed)
+    i = 0
+    for steps, block in ((7, 7), (1, 5), (2, 2), (23, 8)):
+        a.RunSteps(i, steps, block, 20)
+        for k in range(i, i + steps):
+            if k % 20 == 0:
+                itg_b.SetMomentumToZero()
+            b.CalcF()
+            itg_b.Integrate()
+        i += steps
+        for get in ("GetPositionsFP64", "GetVelocities", "GetImages", "GetForcesAndEnergies", "GetVirials"):
+            np.testing.assert_array_equal(getattr(a, get)(), getattr(b, get)(), err_msg=f"{get} after {i} steps")
+        assert itg_a.GetThermostatState() == itg_b.GetThermostatState()
+        assert itg_a.GetKineticEnergy() == itg_b.GetKineticEnergy()
+    if thermo:
+        assert itg_a.GetTargetTemperature() == itg_b.GetTargetTemperature()
+    if method == "n2":
+        assert pot_a.GetNumberOfNbListBuilds() == pot_b.GetNumberOfNbListBuilds() > 1
+
+
+def test_one_kernel_steps_with_an_overflowed_list():
+    """Lists that overflow inside a chain take all pairs, and grow afterwards."""
+    a, pot_a, _ = _stepping_sample(1003, "n2", True, False)
+    b, _, _ = _stepping_sample(1003, "n2", True, False)
+    pot_a.SetNbMaxNumNbrs(40)
+    print("[case] small steps, overflowed lists", flush=True)
+    a.RunSteps(0, 10, 10, 0)
+    b.RunSteps(0, 10, 10, 0)
+    # the overflowed particles' sums run in another order: rounding apart after ten steps
+    np.testing.assert_allclose(a.GetVelocities(), b.GetVelocities(), rtol=0, atol=1e-4)
+    a.CalcF()  # builds in the grown lists
+    assert pot_a.GetActualMaxNumNbrs() > 40
