@@ -151,7 +151,7 @@ typedef struct rumdx_nblist {
   uint16_t* nbl16_dev;      /* sorted method: (max_nbrs rounded up to 8) x nvp halo offsets */
   uint32_t ntiles;          /* from rumdx_tile_table() */
   const uint32_t* tile_first_rank_dev; /* ntiles + 1 */
-  const uint32_t* tile_origin_dev;     /* ntiles: cx0 | cy0 << 10 | cz0 << 20 */
+  const uint32_t* tile_origin_dev;     /* ntiles: cx0 | cy0 << 10 | cz0 << 20 | shape << 30 */
   uint32_t halo_cap;        /* halo particles a tile stages in LDS (<= RUMDX_HALO_CAP_MAX) */
   uint16_t* lane_order_dev; /* sorted method: nvp, written by the build */
   uint32_t* tile_halo_dev;  /* sorted method: ntiles x halo_cap slots of each tile's halo, written by the build */
@@ -193,7 +193,8 @@ typedef struct rumdx_nblist {
 /* tile_info_dev[4 t + 1] of a sorted build: bit 0 set when the tile's halo
  * was staged and every pair takes the plain FP32 difference (in the shifted
  * frame where the halo wraps); bits 1-6 mark, per axis, a halo wrapping below
- * (bit 2a+1) or above (bit 2a+2) the tile; bits 16-31 hold the halo capacity
+ * (bit 2a+1) or above (bit 2a+2) the tile; bits 7-15 hold the longest list in
+ * groups of 8 rounded up (at most 511); bits 16-31 hold the halo capacity
  * the build used.  tile_info_dev[4 t] is the tile's halo size, [4 t + 2] and
  * [4 t + 3] its slot range. */
 #define RUMDX_TILE_FAST 1u
@@ -228,13 +229,21 @@ int rumdx_cell_rank_table(const int32_t nc[3], uint32_t* rank_out);
  * origin cell, packed cx | cy << 10 | cz << 20).  rank is the table of
  * rumdx_cell_rank_table.  Host only; returns a negative code on error. */
 int rumdx_tile_table(const int32_t nc[3], const uint32_t* rank, uint32_t* first_rank_out, uint32_t* origin_out);
+/* The same for smaller tiles: shape 0 (4 x 4 x 4 cells), 1 (4 x 4 x 2), 2 (4 x
+ * 2 x 2) or 3 (2 x 2 x 2), recorded in bits 30-31 of the origin words.
+ * rumdx_tile_shape(nc) gives the shape that suits a grid: a small one has too
+ * few 4^3 tiles for one workgroup each. */
+int rumdx_tile_shape(const int32_t nc[3]);
+int rumdx_tile_table_shaped(const int32_t nc[3], const uint32_t* rank, int shape, uint32_t* first_rank_out,
+                            uint32_t* origin_out);
 /* Halo capacity (particles) to request for a grid of nc cells holding n
- * particles: the mean 8^3-cell halo plus 8 % and 64, rounded up to 64, at
+ * particles: the mean halo (8^3 cells for tiles of 4^3) plus 8 % and 64, rounded up to 64, at
  * most RUMDX_HALO_CAP_MAX.  The force kernel's LDS is 16 bytes per halo
  * particle, so a smaller capacity lets more tiles share a CU.  Tiles whose
  * halo is larger still compute exactly, reading positions from global
  * memory. */
 uint32_t rumdx_halo_cap_estimate(const int32_t nc[3], uint32_t n);
+uint32_t rumdx_halo_cap_estimate_shaped(const int32_t nc[3], uint32_t n, int shape);
 
 /* ---------------------------------------------------------------- neighbour list
  * NeighborList::CheckRebuildRequired / displacement_since_nb_build
@@ -432,8 +441,8 @@ int rumdx_nvt_step(rumdx_particles* p, rumdx_nh_state* nh_dev, float dt, uint32_
  * place and f, w hold the forces, energies and virials at the old positions.
  * The caller swaps p->r_dev and r_out_dev afterwards.  With the thermostat on,
  * the kinetic-energy sum is taken per cell tile (one double per tile in the
- * workspace of rumdx_workspace_bytes(n), which must hold nb->ntiles of them:
- * RUMDX_E_INVALID otherwise) and then in tile order, so Ps agrees with
+ * workspace of rumdx_workspace_bytes(n), which must hold nb->ntiles of them
+ * after its first 256 bytes: RUMDX_E_INVALID otherwise) and then in tile order, so Ps agrees with
  * rumdx_nvt_step's to rounding; forces, velocities and positions of a step
  * are bit-identical to the two calls'. */
 int rumdx_pair_lj_nvt(const rumdx_particles* p, const rumdx_nblist* nb, const float* params_dev, uint32_t ntypes,

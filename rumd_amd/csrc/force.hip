@@ -40,8 +40,10 @@ struct LjPair {
   // ComputeInteraction inlined): u = A12 r^-12 + A6 r^-6, s = -u'(r)/r,
   // shifted as the cut-off method asks (SP: u - u(rc); SF: s - s(rc) rc/r and
   // u - u(rc) + s(rc) rc (r - rc)).  Branch-free; pairs at or beyond rc are
-  // masked.
-  template <bool STR>
+  // masked.  FINE refines 1/r^2 from the squared rsq by one Newton step (two
+  // operations): the seventh power of its error enters the force, and the
+  // callers that form displacements in FP64 are not bound by the arithmetic.
+  template <bool STR, bool FINE>
   __device__ __forceinline__ void core(float dx, float dy, float dz, float d2, uint32_t tj, const float4* prow,
                                        Acc& a) const {
     const float4 pa = prow[2 * tj];
@@ -51,6 +53,7 @@ struct LjPair {
     if (CUT == RUMDX_CUTOFF_SF) {
       rinv = __builtin_amdgcn_rsqf(d2);
       inv2 = rinv * rinv;
+      if (FINE) inv2 = fmaf(inv2, fmaf(-d2, inv2, 1.f), inv2);
     } else {
       inv2 = __builtin_amdgcn_rcpf(d2);
     }
@@ -127,8 +130,8 @@ extern "C" int rumdx_pair_lj_nvt(const rumdx_particles* p, const rumdx_nblist* n
     return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: thermostat state and workspace required");
   if (thermo && dof == 0) return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: zero degrees of freedom");
   // one kinetic-energy partial per tile in the workspace's partials
-  if (thermo && static_cast<size_t>(nb->ntiles) > 4u * static_cast<size_t>(blocks_for(p->n > 0 ? p->n : 1)))
-    return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: more tiles than the workspace holds partials (4 per 256 particles)");
+  if (thermo && static_cast<size_t>(nb->ntiles) > Workspace::partial_doubles(p->n))
+    return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: more tiles than the workspace holds partials");
   if (p->n == 0) return RUMDX_OK;
   NvtFuse fz{};
   fz.r_out = reinterpret_cast<float4*>(r_out_dev);

@@ -63,7 +63,7 @@ struct FormPair {
   // u(rc); SF: s - s(rc) rc / r, u + s(rc) rc (r - rc) - u(rc), the last two
   // terms as s(rc) rc r - (s(rc) rc^2 + u(rc))); pairs at or beyond rc are
   // masked.
-  template <bool STR>
+  template <bool STR, bool FINE>
   __device__ __forceinline__ void core(float dx, float dy, float dz, float d2, uint32_t tj, const float4* prow,
                                        Acc& a) const {
     const float4 c0 = prow[3 * tj];

@@ -19,8 +19,9 @@
 // A pair policy PP supplies the potential: kRow float4 per type pair in LDS,
 // kWavesPerEU (the tile kernel's occupancy target; kTunedWaves: the
 // stepping variant also exists for 4 and 6 waves, rumdx_nblist.tile_waves_per_eu),
-// load_table (RUMD's 12-float rows -> that LDS table) and core<STR> (the
-// masked pair term for a displacement, accumulated into Acc).  The 12-6
+// load_table (RUMD's 12-float rows -> that LDS table) and core<STR, FINE> (the
+// masked pair term for a displacement, accumulated into Acc; FINE where the
+// displacement was formed in FP64).  The 12-6
 // policy lives in force.hip, the other potential forms in force_generic.hip.
 #pragma once
 
@@ -78,7 +79,7 @@ __device__ __forceinline__ void pair_term(const PP& pp, double xi, double yi, do
   x -= bx.Ld[0] * rint(x * bx.iLd[0]);
   y -= bx.Ld[1] * rint(y * bx.iLd[1]);
   z -= bx.Ld[2] * rint(z * bx.iLd[2]);
-  pp.template core<STR>(static_cast<float>(x), static_cast<float>(y), static_cast<float>(z),
+  pp.template core<STR, true>(static_cast<float>(x), static_cast<float>(y), static_cast<float>(z),
                         static_cast<float>(x * x + y * y + z * z), __float_as_uint(rj.w), prow, a);
 }
 
@@ -87,7 +88,7 @@ __device__ __forceinline__ void pair_term(const PP& pp, double xi, double yi, do
 template <bool STR, class PP>
 __device__ __forceinline__ void pair_term_direct(const PP& pp, float4 ri, float4 rj, const float4* prow, Acc& a) {
   const float dx = ri.x - rj.x, dy = ri.y - rj.y, dz = ri.z - rj.z;
-  pp.template core<STR>(dx, dy, dz, dx * dx + dy * dy + dz * dz, __float_as_uint(rj.w), prow, a);
+  pp.template core<STR, false>(dx, dy, dz, dx * dx + dy * dy + dz * dz, __float_as_uint(rj.w), prow, a);
 }
 
 // Forces on particle i from the 5x5x5 cell stencil around the cell it was
@@ -296,8 +297,11 @@ __device__ __forceinline__ void tile_particles(const PP& pp, uint32_t slot0, uin
                                                const uint16_t* __restrict__ lane_order, const float4* s_pos,
                                                const float4* s_tab, uint32_t nt, const Box& bx,
                                                const CellFallback& fb, uint32_t nvp, uint32_t max_nbrs,
-                                               uint32_t lgp) {
+                                               uint32_t lgp, uint32_t longest) {
   const uint32_t np = slot1 - slot0;
+  // a small tile's lists are spread over as many lanes as its workgroup has,
+  // while the longest still gives each lane a group
+  while (lgp < 3u && (np << (lgp + 1u)) <= kBlock && (8u << lgp) < longest) ++lgp;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t per_wave = 64u >> lgp;  // particles per wave and chunk: 2^lgp lanes each
   for (uint32_t c0 = (threadIdx.x >> 6) * per_wave; c0 < np; c0 += (kBlock / 64) * per_wave) {
@@ -408,6 +412,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
   pp.load_table(s_tab, params, nt);
   const bool staged = (info.y >> 16) == halo_cap && info.x <= halo_cap;
   const bool fast = (info.y & kTileFast) != 0u;
+  const uint32_t longest = tile_longest(info.y);
   // the fused step's state of this thread's first particle, read now so that
   // the reads overlap the staging and the pair loop
   const uint32_t i_own = info.z + threadIdx.x;
@@ -444,10 +449,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
   __syncthreads();
   if (staged && fast)
     tile_particles<PP, STR, INIT, true>(pp, info.z, info.w, true, info.y, r, f, w, sts, nbl16, num_nbrs, lane_order,
-                                         s_pos, s_tab, nt, bx, fb, nvp, max_nbrs, lgp);
+                                         s_pos, s_tab, nt, bx, fb, nvp, max_nbrs, lgp, longest);
   else
     tile_particles<PP, STR, INIT, false>(pp, info.z, info.w, staged, 0u, r, f, w, sts, nbl16, num_nbrs, lane_order,
-                                          s_pos, s_tab, nt, bx, fb, nvp, max_nbrs, lgp);
+                                          s_pos, s_tab, nt, bx, fb, nvp, max_nbrs, lgp, longest);
   if (FUSE) {
     // the tile's forces are stored (and read back from L2 in slot order);
     // the halo is no longer read, so its LDS holds the reduction

@@ -517,7 +517,8 @@ __global__ __launch_bounds__(kBlock) void k_tile_resort(uint32_t* __restrict__ f
     const int c0[3] = {static_cast<int>(org & 1023u), static_cast<int>((org >> 10) & 1023u),
                        static_cast<int>((org >> 20) & 1023u)};
     for (int a = 0; a < 3; ++a) {
-      const int own = (nc[a] - c0[a]) < kTileEdge ? (nc[a] - c0[a]) : kTileEdge;
+      const int edge = tile_edge(org >> 30, a);
+      const int own = (nc[a] - c0[a]) < edge ? (nc[a] - c0[a]) : edge;
       L.c0[a] = c0[a];
       L.own[a] = own;
       L.ext[a] = (own + 2) < nc[a] ? (own + 2) : nc[a];
@@ -711,7 +712,7 @@ __global__ __launch_bounds__(kBlock) void k_build_stats(uint32_t* __restrict__ f
 // order) and the staged lists of the two particles tested together.  A staged
 // list holds as many entries as the window, so appends need no bounds check.
 constexpr uint32_t kCandWindow = 512;
-constexpr uint32_t kStageMax = 256;  // longest list the staged path writes (max_nbrs bound)
+static_assert(kCandWindow <= 64 * 8, "one 16-byte group of a staged list per lane");
 struct WaveBuild {
   uint16_t cand[kCandWindow];
   uint16_t seg_start[128];  // LDS offset of the segment's first particle
@@ -919,7 +920,7 @@ __device__ __forceinline__ void build_cell_wave(const Halo& h, const HaloLds& L,
   }
   const uint32_t total = __builtin_amdgcn_readfirstlane(carry);
   wave_lds_sync();
-  if (bytes && total <= kCandWindow && max_nbrs <= kStageMax) {
+  if (bytes && total <= kCandWindow) {
     build_cell_staged<WRAPS>(s_pos, s_cut, nt, bx, coff, m, gstart, nseg, total, tg.halo_cap << 4, wb,
                              s_cnt + (gstart - h.slot0), nbl16, nvp, max_nbrs);
     return;
@@ -1144,7 +1145,11 @@ __global__ __launch_bounds__(kBuildBlock) void k_build_tiles(uint32_t* __restric
     // wrapping axes, and whether the shifted frame serves them
     const int nc[3] = {tg.nc0, tg.nc1, tg.nc2};
     uint32_t fl = 0;
-    bool shiftable = true;
+    // A small box in small tiles (shape above 0) keeps FP64 displacements for
+    // every tile: in 4^3 tiles nearly all of them wrapped and had them, and at
+    // these sizes they are not what the force kernel's time goes into.
+    const bool small_box = (tg.origin[t] >> 30) != 0u && min(min(nc[0], nc[1]), nc[2]) < kShiftMinCells;
+    bool shiftable = !small_box;
     for (int a = 0; a < 3; ++a) {
       const bool below = h.base[a] < 0, above = h.base[a] + h.ext[a] > nc[a];
       if (below) fl |= kTileShiftDown << (2 * a);
@@ -1153,6 +1158,7 @@ __global__ __launch_bounds__(kBuildBlock) void k_build_tiles(uint32_t* __restric
                                                        !(below && above) && shift_exact(bx.L[a], nc[a])));
     }
     if (staged && shiftable) fl |= kTileFast;
+    fl |= tile_longest_bits(longest);
     tg.tile_info[t] = make_uint4(h.npart, fl | (tg.halo_cap << 16), h.slot0, h.slot1);
   }
   // the cell starts of this build, home for the force kernels' rescans and
@@ -1598,28 +1604,56 @@ extern "C" int rumdx_nblist_build_stats(const rumdx_particles* p, rumdx_nblist* 
   return check_launch("rumdx_nblist_build_stats");
 }
 
+extern "C" int rumdx_tile_shape(const int32_t nc[3]) {
+  if (nc == nullptr) return fail(RUMDX_E_INVALID, "rumdx_tile_shape: null argument");
+  // The smallest tiles that do not exceed kTilesWanted.  The re-sort, build and
+  // force kernels run one workgroup per tile, up to five to a CU (256 CUs):
+  // with fewer tiles CUs idle and a tile's serial work is the kernel's time,
+  // with more the halo staged per particle grows (2.1 times the tile's own
+  // cells per halved axis at worst).  us per step at N = 12,000, shapes 0-3: 36
+  // (64 tiles), 26, 24, 22 (512); 32,768: 40 (216), 34, 30 (726), 33 (1331);
+  // 65,536: 37 (343), 32 (686), 36 (1372), 45; 200,000: 51 (1000), 58 (2000), 71.
+  constexpr uint64_t kTilesWanted = 900;
+  for (int shape = kTileShapes - 1; shape > 0; --shape) {
+    uint64_t tiles = 1;
+    for (int a = 0; a < 3; ++a) {
+      const int edge = tile_edge(static_cast<uint32_t>(shape), a);
+      tiles *= static_cast<uint64_t>((nc[a] + edge - 1) / edge);
+    }
+    if (tiles <= kTilesWanted) return shape;
+  }
+  return 0;
+}
+
 extern "C" int rumdx_tile_table(const int32_t nc[3], const uint32_t* rank, uint32_t* first_rank_out,
                                 uint32_t* origin_out) {
+  return rumdx_tile_table_shaped(nc, rank, 0, first_rank_out, origin_out);
+}
+
+extern "C" int rumdx_tile_table_shaped(const int32_t nc[3], const uint32_t* rank, int shape, uint32_t* first_rank_out,
+                                       uint32_t* origin_out) {
   if (nc == nullptr) return fail(RUMDX_E_INVALID, "rumdx_tile_table: null argument");
-  int nb[3];
+  if (shape < 0 || shape >= kTileShapes) return fail(RUMDX_E_INVALID, "rumdx_tile_table: shape out of range");
+  int nb[3], edge[3];
   for (int a = 0; a < 3; ++a) {
     if (nc[a] < 1 || nc[a] > 1023) return fail(RUMDX_E_INVALID, "rumdx_tile_table: cells per axis out of range");
-    nb[a] = (nc[a] + kTileEdge - 1) / kTileEdge;
+    edge[a] = tile_edge(static_cast<uint32_t>(shape), a);
+    nb[a] = (nc[a] + edge[a] - 1) / edge[a];
   }
   const uint64_t ntiles = static_cast<uint64_t>(nb[0]) * nb[1] * nb[2];
   if (first_rank_out == nullptr && origin_out == nullptr) return static_cast<int>(ntiles);
   if (rank == nullptr || first_rank_out == nullptr || origin_out == nullptr)
     return fail(RUMDX_E_INVALID, "rumdx_tile_table: null output");
-  // The origin cell of an aligned brick has the smallest Morton code (hence
-  // rank) of the brick, and bricks occupy disjoint code ranges.
+  // The origin cell of an aligned brick (or half, ...) has the smallest Morton
+  // code (hence rank) of the brick, and bricks occupy disjoint code ranges.
   std::vector<std::pair<uint32_t, uint32_t>> t;
   t.reserve(ntiles);
   for (int z = 0; z < nb[2]; ++z)
     for (int y = 0; y < nb[1]; ++y)
       for (int x = 0; x < nb[0]; ++x) {
-        const uint32_t cx = x * kTileEdge, cy = y * kTileEdge, cz = z * kTileEdge;
+        const uint32_t cx = x * edge[0], cy = y * edge[1], cz = z * edge[2];
         const uint32_t lin = cx + cy * nc[0] + cz * static_cast<uint32_t>(nc[0]) * nc[1];
-        t.emplace_back(rank[lin], cx | (cy << 10) | (cz << 20));
+        t.emplace_back(rank[lin], cx | (cy << 10) | (cz << 20) | (static_cast<uint32_t>(shape) << 30));
       }
   std::sort(t.begin(), t.end());
   for (uint64_t k = 0; k < ntiles; ++k) {
@@ -1631,9 +1665,14 @@ extern "C" int rumdx_tile_table(const int32_t nc[3], const uint32_t* rank, uint3
 }
 
 extern "C" uint32_t rumdx_halo_cap_estimate(const int32_t nc[3], uint32_t n) {
-  if (nc == nullptr) return 0;
+  return rumdx_halo_cap_estimate_shaped(nc, n, 0);
+}
+
+extern "C" uint32_t rumdx_halo_cap_estimate_shaped(const int32_t nc[3], uint32_t n, int shape) {
+  if (nc == nullptr || shape < 0 || shape >= kTileShapes) return 0;
   const double ncells = static_cast<double>(nc[0]) * nc[1] * nc[2];
-  const double halo = static_cast<double>(kHaloCellsMax) * n / ncells;
+  double halo = static_cast<double>(n) / ncells;
+  for (int a = 0; a < 3; ++a) halo *= tile_edge(static_cast<uint32_t>(shape), a) + 4;
   uint32_t cap = static_cast<uint32_t>(1.08 * halo + 64.0);
   cap = (cap + 63u) & ~63u;
   return cap > RUMDX_HALO_CAP_MAX ? RUMDX_HALO_CAP_MAX : cap;

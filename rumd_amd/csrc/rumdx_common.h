@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <string>
 
 #include "rumdx.h"
@@ -236,11 +237,13 @@ struct Workspace {
   static constexpr size_t kScalars = 64;    // double[8] scratch results
   static constexpr size_t kStates = 128;    // rumdx_nh_state[2]: the thermostat inside a chain of one-kernel steps
   static constexpr size_t kPartials = 256;  // double[partial_doubles(n)]
-  // four sums per kBlock particles, or two sets of a small sample's partials
+  // four sums per kBlock particles, two sets of a small sample's partials, or
+  // the small tiles of a medium one (some 27 particles each in a liquid)
   static size_t partial_doubles(uint32_t n) {
     const size_t four = 4 * static_cast<size_t>(blocks_for(n > 0 ? n : 1));
     const size_t two = n <= kSmallStepMax ? 2 * static_cast<size_t>(ke_partials(n > 0 ? n : 1)) : 0;
-    return four > two ? four : two;
+    const size_t tiles = n <= 262144u ? blocks_for(n, 16u) : 0u;
+    return std::max(four, std::max(two, tiles));
   }
   static rumdx_nh_state* states(void* ws) {
     return reinterpret_cast<rumdx_nh_state*>(static_cast<char*>(ws) + kStates);

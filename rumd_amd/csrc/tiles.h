@@ -3,8 +3,8 @@
 //
 // Cells are stored in Morton order of their coordinates, so an aligned
 // kTileEdge^3 brick of cells is a contiguous run of ranks and therefore of
-// particle slots.  One workgroup owns one brick ("tile") and stages its halo
-// -- the bricks's cells dilated by the 2-cell stencil, at most 8^3 cells -- into
+// particle slots (as are its halves, see tile_edge).  One workgroup owns one
+// brick ("tile") and stages its halo -- the brick's cells dilated by the 2-cell stencil, at most 8^3 cells -- into
 // LDS: a per-halo-cell table (global first slot, LDS offset) and, when it fits,
 // the halo particles' positions.  List entries of the tile format are LDS
 // offsets into that halo (16 bit), so the force kernel reads neighbour
@@ -15,7 +15,16 @@
 
 namespace rumdx {
 
-constexpr int kTileEdge = 4;                            // cells per tile edge (a power of two)
+// Cells per tile edge (a power of two).  A grid of few cells has too few 4^3
+// bricks for the chip, so it is cut into halves, quarters or eighths of them,
+// which are contiguous rank ranges too (z is the top bit of a Morton code, then
+// y, then x): the tile's shape s halves the edges of its last s axes, and bits
+// 30-31 of its origin word hold s.  tile_shape gives the rule.
+constexpr int kTileEdge = 4;
+constexpr int kTileShapes = 4;
+__host__ __device__ inline int tile_edge(uint32_t shape, int axis) {
+  return shape > static_cast<uint32_t>(2 - axis) ? kTileEdge / 2 : kTileEdge;
+}
 constexpr int kHaloEdgeMax = kTileEdge + 4;             // 2-cell stencil on each side
 constexpr uint32_t kHaloCellsMax = kHaloEdgeMax * kHaloEdgeMax * kHaloEdgeMax;  // 512
 
@@ -24,7 +33,7 @@ struct TileGeom {
   const uint32_t* cell_rank;   // linear cell -> rank
   const uint32_t* cell_start;  // rank -> first slot (ncells + 1)
   const uint32_t* first_rank;  // tile -> first rank (ntiles + 1)
-  const uint32_t* origin;      // tile -> cx0 | cy0 << 10 | cz0 << 20
+  const uint32_t* origin;      // tile -> cx0 | cy0 << 10 | cz0 << 20 | shape << 30
   uint32_t ntiles;
   uint32_t halo_cap;           // particles the LDS position buffer holds
   uint32_t* halo_slots;        // tile t's halo slots at [t * halo_cap, ...) (build output)
@@ -39,6 +48,14 @@ struct TileGeom {
 constexpr uint32_t kTileFast = 1u;
 constexpr uint32_t kTileShiftDown = 2u;
 constexpr uint32_t kTileShiftUp = 4u;
+// Bits 7-15: the tile's longest list at the build, in groups of 8 rounded up.
+constexpr uint32_t kTileLongShift = 7, kTileLongMax = 511;
+__device__ __forceinline__ uint32_t tile_longest_bits(uint32_t longest) {
+  const uint32_t groups = (longest + 7u) >> 3;
+  return (groups < kTileLongMax ? groups : kTileLongMax) << kTileLongShift;
+}
+// At least the longest list (up to its last, partial group).
+__device__ __forceinline__ uint32_t tile_longest(uint32_t fl) { return ((fl >> kTileLongShift) & kTileLongMax) << 3; }
 static_assert(kTileFast == RUMDX_TILE_FAST, "tile flag bits of the header");
 static_assert((((kTileShiftDown | kTileShiftUp) << 0) | ((kTileShiftDown | kTileShiftUp) << 2) |
                ((kTileShiftDown | kTileShiftUp) << 4)) == RUMDX_TILE_SHIFT_MASK,
@@ -149,7 +166,8 @@ __device__ __forceinline__ void stage_halo(uint32_t t, const TileGeom& g, const 
     bool wraps = false;
     uint32_t ncell = 1;
     for (int a = 0; a < 3; ++a) {
-      const int bw = (nc[a] - c0[a]) < kTileEdge ? (nc[a] - c0[a]) : kTileEdge;
+      const int edge = tile_edge(o >> 30, a);
+      const int bw = (nc[a] - c0[a]) < edge ? (nc[a] - c0[a]) : edge;
       const int ext = (bw + 4) < nc[a] ? (bw + 4) : nc[a];
       L.h.base[a] = c0[a] - 2;
       L.h.ext[a] = ext;

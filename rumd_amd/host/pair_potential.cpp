@@ -265,16 +265,17 @@ void NeighborList::Allocate() {
     desc_.sort_scratch_dev = sort_scratch_.get();
     desc_.lane_order_dev = lane_order_.get();
     // cell tiles of the LDS-staged build and force kernels
-    const int ntiles = rumdx_tile_table(nc, rank.data(), nullptr, nullptr);
+    const int shape = rumdx_tile_shape(nc);
+    const int ntiles = rumdx_tile_table_shaped(nc, rank.data(), shape, nullptr, nullptr);
     if (ntiles <= 0) rumdx_check(ntiles == 0 ? RUMDX_E_INVALID : ntiles, "NeighborList", "Allocate");
     std::vector<uint32_t> first(ntiles + 1), origin(ntiles);
-    const int nt2 = rumdx_tile_table(nc, rank.data(), first.data(), origin.data());
+    const int nt2 = rumdx_tile_table_shaped(nc, rank.data(), shape, first.data(), origin.data());
     if (nt2 != ntiles) rumdx_check(RUMDX_E_INVALID, "NeighborList", "Allocate");
     tile_first_rank_.resize(first.size());
     tile_first_rank_.upload(first.data(), first.size(), st);
     tile_origin_.resize(origin.size());
     tile_origin_.upload(origin.data(), origin.size(), st);
-    if (halo_cap_ == 0) halo_cap_ = rumdx_halo_cap_estimate(nc, n);
+    if (halo_cap_ == 0) halo_cap_ = rumdx_halo_cap_estimate_shaped(nc, n, shape);
     tile_info_.resize(4ull * ntiles);
     desc_.nbl16_dev = nbl16_.get();
     desc_.ntiles = static_cast<uint32_t>(ntiles);
@@ -619,9 +620,8 @@ bool PairPotential::CanFuseStep() {
   if (neighborList.GetResolvedMethod() != NeighborList::SORT) return false;
   const rumdx_nblist* nb = neighborList.Descriptor();
   if (nb->nbl16_dev == nullptr || nb->ntiles == 0) return false;
-  // the workspace of rumdx_workspace_bytes(n) holds 4 partials per 256 particles
-  const size_t n = sample->GetNumberOfParticles();
-  return static_cast<size_t>(nb->ntiles) <= 4 * ((n + 255) / 256);
+  // the sample's workspace holds a partial sum per tile
+  return 256 + sizeof(double) * static_cast<size_t>(nb->ntiles) <= rumdx_workspace_bytes(sample->GetNumberOfParticles());
 }
 
 void PairPotential::CalcFIntegrateNVT(rumdx_nh_state* nh_dev, float dt, unsigned thermostat_on_mask, float omega2,

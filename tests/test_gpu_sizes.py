@@ -205,3 +205,33 @@ def test_one_kernel_steps_with_an_overflowed_list():
     np.testing.assert_allclose(a.GetVelocities(), b.GetVelocities(), rtol=0, atol=1e-4)
     a.CalcF()  # builds in the grown lists
     assert pot_a.GetActualMaxNumNbrs() > 40
+
+
+# tiles of 2x2x2, 4x2x2, 4x4x2 and 4x4x4 cells
+@pytest.mark.parametrize("n", [9001, 33001, 66001, 130001])
+def test_sorted_lists_and_steps_at_each_tile_shape(n):
+    print(f"[case] tile shapes n={n}", flush=True)
+    a, pot, itg_a = _stepping_sample(n, "sort", True, False)
+    b, _, itg_b = _stepping_sample(n, "sort", True, False)
+    b.SetFusedSteps(False)
+    a.RunSteps(0, 30, 10, 0)  # rebuilds inside
+    b.RunSteps(0, 30, 10, 0)
+    assert pot.GetNumberOfNbListBuilds() > 1
+    # the kinetic-energy sum runs per tile in one and per 256 slots in the
+    # other (Ps agrees to 1e-12), so bits may differ where ps rounds to float
+    np.testing.assert_allclose(itg_a.GetThermostatState(), itg_b.GetThermostatState(), rtol=1e-6)
+    np.testing.assert_allclose(a.GetVelocities(), b.GetVelocities(), rtol=0, atol=2e-4)
+    a.CalcF()
+    off, ids = pot.GetNeighborListCSR(a)
+    pos4 = configs.pack_pos4(a.GetPositions(), a.GetTypes())
+    box = np.array([a.GetSimulationBox().GetLength(k) for k in range(3)])
+    f_ref, _ = oracle.forces_cells(pos4, box, 2, ka_table(), SF)
+    assert force_errors(a.GetForces(), f_ref[:, :3])["guarded_max"] <= FORCE_TOL_GUARDED
+    # the list holds every pair within rc of the current positions (it was
+    # built within half a skin of them): check a sample of particles
+    x = pos4[:, :3].astype(np.float64)
+    for i in range(0, n, n // 50):
+        d = x - x[i]
+        d -= box * np.rint(d / box)
+        near = np.flatnonzero((d * d).sum(axis=1) < (2.5 * 0.8) ** 2)
+        assert set(near) - {i} <= set(ids[off[i]:off[i + 1]].tolist())
