@@ -449,6 +449,35 @@ int rumdx_pair_lj_nvt(const rumdx_particles* p, const rumdx_nblist* nb, const fl
                       const float box[8], int cutoff_method, float* r_out_dev, rumdx_nh_state* nh_dev, float dt,
                       uint32_t thermostat_on_mask, float omega2, uint32_t dof, void* workspace_dev, void* stream);
 
+/* Steps whose thermostat update is left to a later call: rumdx_nvt_step and
+ * rumdx_pair_lj_nvt without UpdateThermostatState, the kinetic-energy partials
+ * staying in the workspace (rumdx_nvt_partials(n), or nb->ntiles of them).  The
+ * caller passes the update on to rumdx_nblist_rebuild_sorted_due or
+ * rumdx_nvt_finish before anything else reads the state or uses the workspace.
+ * With store_forces 0 the fused step leaves energies and virials out: f holds
+ * the forces, w is not written; the next step's forces replace them. */
+typedef struct rumdx_nh_update {
+  rumdx_nh_state* nh_dev;
+  void* workspace_dev;  /* holds the partials */
+  uint32_t npartials;
+  uint32_t dof;
+  float dt;
+  float omega2;
+} rumdx_nh_update;
+uint32_t rumdx_nvt_partials(uint32_t n);
+int rumdx_nvt_step_due(rumdx_particles* p, const rumdx_nh_state* nh_dev, float dt, uint32_t thermostat_on_mask,
+                       const float box[8], rumdx_nblist* nb, void* workspace_dev, void* stream);
+int rumdx_pair_lj_nvt_due(const rumdx_particles* p, const rumdx_nblist* nb, const float* params_dev, uint32_t ntypes,
+                          const float box[8], int cutoff_method, float* r_out_dev, const rumdx_nh_state* nh_dev,
+                          float dt, uint32_t thermostat_on_mask, int store_forces, void* workspace_dev, void* stream);
+int rumdx_nvt_finish(const rumdx_nh_update* due, void* stream);
+/* rumdx_nblist_rebuild_sorted with a thermostat update that is due (due may be
+ * NULL) done by one more workgroup of its first kernel, in every call; with
+ * carry_forces 0 a rebuild leaves f and w behind (the next force call
+ * initialises them). */
+int rumdx_nblist_rebuild_sorted_due(rumdx_particles* p, rumdx_nblist* nb, const float box[8], int carry_forces,
+                                    const rumdx_nh_update* due, void* stream);
+
 /* Steps of a small sample (n <= RUMDX_SMALL_STEP_MAX) whose only force term is
  * a 12-6 pair potential over a list of the N2 method, or over all pairs (nb ==
  * NULL), one kernel each: rumdx_nblist_build_n2 when flags[REBUILD] asks,

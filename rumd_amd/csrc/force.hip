@@ -107,31 +107,33 @@ extern "C" int rumdx_pair_lj(const rumdx_particles* p, const rumdx_nblist* nb, c
 // positions going to r_out_dev; then the thermostat update from the per-tile
 // kinetic-energy sums.  Per particle the arithmetic is that of rumdx_pair_lj
 // followed by rumdx_nvt_step.
-extern "C" int rumdx_pair_lj_nvt(const rumdx_particles* p, const rumdx_nblist* nb, const float* params_dev,
-                                 uint32_t ntypes, const float box[8], int cutoff_method, float* r_out_dev,
-                                 rumdx_nh_state* nh_dev, float dt, uint32_t thermostat_on_mask, float omega2,
-                                 uint32_t dof, void* workspace_dev, void* stream) {
-  using namespace rumdx;
-  const char* entry = "rumdx_pair_lj_nvt";
+namespace rumdx {
+namespace {
+
+// The fused step without the thermostat's update; want: energies and virials
+// are stored too.
+int pair_lj_nvt(const char* entry, const rumdx_particles* p, const rumdx_nblist* nb, const float* params_dev,
+                uint32_t ntypes, const float* box, int cutoff_method, float* r_out_dev, const rumdx_nh_state* nh_dev,
+                float dt, uint32_t thermostat_on_mask, bool want, void* workspace_dev, void* stream) {
+  const std::string e(entry);
   const int rc = check_pair_args(entry, p, nb, params_dev, ntypes, box, 0);
   if (rc != RUMDX_OK) return rc;
   if (nb == nullptr || nb->nbl16_dev == nullptr)
-    return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: needs a list of the sorted method");
+    return fail(RUMDX_E_INVALID, e + ": needs a list of the sorted method");
   if (nb->flags_dev == nullptr || nb->last_r_dev == nullptr)
-    return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: neighbour list not allocated");
+    return fail(RUMDX_E_INVALID, e + ": neighbour list not allocated");
   if (p->v_dev == nullptr || p->im_dev == nullptr || r_out_dev == nullptr)
-    return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: particle arrays not allocated");
+    return fail(RUMDX_E_INVALID, e + ": particle arrays not allocated");
   if (r_out_dev == p->r_dev)
-    return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: r_out_dev must not alias the positions the forces read");
+    return fail(RUMDX_E_INVALID, e + ": r_out_dev must not alias the positions the forces read");
   if (cutoff_method != RUMDX_CUTOFF_NS && cutoff_method != RUMDX_CUTOFF_SP && cutoff_method != RUMDX_CUTOFF_SF)
-    return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: invalid cutoff method");
+    return fail(RUMDX_E_INVALID, e + ": invalid cutoff method");
   const bool thermo = thermostat_on_mask != 0u;
   if (thermo && (nh_dev == nullptr || workspace_dev == nullptr))
-    return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: thermostat state and workspace required");
-  if (thermo && dof == 0) return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: zero degrees of freedom");
+    return fail(RUMDX_E_INVALID, e + ": thermostat state and workspace required");
   // one kinetic-energy partial per tile in the workspace's partials
   if (thermo && static_cast<size_t>(nb->ntiles) > Workspace::partial_doubles(p->n))
-    return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: more tiles than the workspace holds partials");
+    return fail(RUMDX_E_INVALID, e + ": more tiles than the workspace holds partials");
   if (p->n == 0) return RUMDX_OK;
   NvtFuse fz{};
   fz.r_out = reinterpret_cast<float4*>(r_out_dev);
@@ -151,20 +153,44 @@ extern "C" int rumdx_pair_lj_nvt(const rumdx_particles* p, const rumdx_nblist* n
   const hipStream_t st = as_stream(stream);
   const uint32_t lpp = nb->lanes_per_particle;
   const uint32_t lgp = lpp >= 8u ? 3u : lpp >= 4u ? 2u : lpp >= 2u ? 1u : 0u;
+  const auto launch = [&](auto pp) {
+    if (want)
+      launch_tiles<decltype(pp), false, true, kFuseStore>(pp, p, nb, params_dev, ntypes, bx, lgp, fz, st);
+    else
+      launch_tiles<decltype(pp), false, true, kFuseInner>(pp, p, nb, params_dev, ntypes, bx, lgp, fz, st);
+  };
   switch (cutoff_method) {
-    case RUMDX_CUTOFF_NS:
-      launch_tiles<LjPair<RUMDX_CUTOFF_NS>, false, true, true>({}, p, nb, params_dev, ntypes, bx, lgp, fz, st);
-      break;
-    case RUMDX_CUTOFF_SP:
-      launch_tiles<LjPair<RUMDX_CUTOFF_SP>, false, true, true>({}, p, nb, params_dev, ntypes, bx, lgp, fz, st);
-      break;
-    default:
-      launch_tiles<LjPair<RUMDX_CUTOFF_SF>, false, true, true>({}, p, nb, params_dev, ntypes, bx, lgp, fz, st);
-      break;
+    case RUMDX_CUTOFF_NS: launch(LjPair<RUMDX_CUTOFF_NS>{}); break;
+    case RUMDX_CUTOFF_SP: launch(LjPair<RUMDX_CUTOFF_SP>{}); break;
+    default: launch(LjPair<RUMDX_CUTOFF_SF>{}); break;
   }
-  if (thermo)
-    hipLaunchKernelGGL(k_nvt_finish, dim3(1), dim3(kBlock), 0, st, fz.partials, nb->ntiles, nh_dev, dt, omega2, dof);
   return check_launch(entry);
+}
+
+}  // namespace
+}  // namespace rumdx
+
+extern "C" int rumdx_pair_lj_nvt_due(const rumdx_particles* p, const rumdx_nblist* nb, const float* params_dev,
+                                     uint32_t ntypes, const float box[8], int cutoff_method, float* r_out_dev,
+                                     const rumdx_nh_state* nh_dev, float dt, uint32_t thermostat_on_mask,
+                                     int store_forces, void* workspace_dev, void* stream) {
+  return rumdx::pair_lj_nvt("rumdx_pair_lj_nvt_due", p, nb, params_dev, ntypes, box, cutoff_method, r_out_dev, nh_dev,
+                            dt, thermostat_on_mask, store_forces != 0, workspace_dev, stream);
+}
+
+extern "C" int rumdx_pair_lj_nvt(const rumdx_particles* p, const rumdx_nblist* nb, const float* params_dev,
+                                 uint32_t ntypes, const float box[8], int cutoff_method, float* r_out_dev,
+                                 rumdx_nh_state* nh_dev, float dt, uint32_t thermostat_on_mask, float omega2,
+                                 uint32_t dof, void* workspace_dev, void* stream) {
+  using namespace rumdx;
+  const bool thermo = thermostat_on_mask != 0u;
+  if (thermo && nh_dev != nullptr && workspace_dev != nullptr && dof == 0)
+    return fail(RUMDX_E_INVALID, "rumdx_pair_lj_nvt: zero degrees of freedom");
+  const int rc = pair_lj_nvt("rumdx_pair_lj_nvt", p, nb, params_dev, ntypes, box, cutoff_method, r_out_dev, nh_dev, dt,
+                             thermostat_on_mask, true, workspace_dev, stream);
+  if (rc != RUMDX_OK || !thermo || p->n == 0) return rc;
+  const rumdx_nh_update due{nh_dev, workspace_dev, nb->ntiles, dof, dt, omega2};
+  return rumdx_nvt_finish(&due, stream);
 }
 
 namespace rumdx {

@@ -287,7 +287,10 @@ __global__ __launch_bounds__(kBlock) void k_pair_all(PP pp, const float4* __rest
 // FP32 difference; otherwise the halo wraps and displacements are formed in
 // FP64.  An overflowed list, or every list of a tile whose halo was not
 // staged, rescans the particle's build-time cell stencil from global memory.
-template <class PP, bool STR, bool INIT, bool FAST>
+// ENERGY false: the forces alone are stored (the compiler then drops the
+// energy and virial arithmetic, 8 of a pair's 28 operations, and the table's
+// second row).
+template <class PP, bool STR, bool INIT, bool FAST, bool ENERGY>
 __device__ __forceinline__ void tile_particles(const PP& pp, uint32_t slot0, uint32_t slot1, bool staged,
                                                const uint32_t shifts,
                                                const float4* __restrict__ r, float4* __restrict__ f,
@@ -373,7 +376,12 @@ __device__ __forceinline__ void tile_particles(const PP& pp, uint32_t slot0, uin
       }
     }
     combine_lanes<STR>(a, lg);
-    if (live && part == 0) store_result<STR, INIT>(i, a, f, w, sts);
+    if (live && part == 0) {
+      if (ENERGY)
+        store_result<STR, INIT>(i, a, f, w, sts);
+      else
+        f[i] = make_float4(a.fx, a.fy, a.fz, 0.f);
+    }
   }
 }
 
@@ -391,19 +399,24 @@ __device__ __forceinline__ void tile_particles(const PP& pp, uint32_t slot0, uin
 // LDS: its dynamic LDS is the halo capacity and the parameter table, which
 // sets how many workgroups share a CU.
 //
-// With FUSE (initialising, no stresses) the kernel also takes the NVT step:
+// With FUSE (initialising, no stresses) the kernel also takes the NVT step
+// (kFuseInner: without energies and virials, for a step whose forces the next
+// one replaces):
 // once the tile's forces are stored, its particles are advanced in slot order
 // (coalesced; the force loop visits them by list length), the positions into
 // fz.r_out, and the tile's sum of m v^2 goes to fz.partials[tile] for
 // k_nvt_finish.
-template <class PP, bool STR, bool INIT, int WPE = PP::kWavesPerEU, bool FUSE = false>
+constexpr int kFuseNone = 0, kFuseStore = 1, kFuseInner = 2;
+
+template <class PP, bool STR, bool INIT, int WPE = PP::kWavesPerEU, int FUSE = kFuseNone>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) void k_pair_tiles(
     PP pp, const float4* __restrict__ r, float4* __restrict__ f, float4* __restrict__ w, float4* __restrict__ sts,
     const uint16_t* __restrict__ nbl16, const uint32_t* __restrict__ num_nbrs,
     const uint16_t* __restrict__ lane_order, const float* __restrict__ params, uint32_t nt, Box bx,
     const uint4* __restrict__ tile_info, const uint32_t* __restrict__ halo_slots, uint32_t halo_cap,
     CellFallback fb, uint32_t nvp, uint32_t max_nbrs, uint32_t lgp, NvtFuse fz) {
-  static_assert(!FUSE || (INIT && !STR), "the fused step initialises forces and takes no stresses");
+  constexpr bool kEnergy = FUSE != kFuseInner;
+  static_assert(FUSE == kFuseNone || (INIT && !STR), "the fused step initialises forces and takes no stresses");
   extern __shared__ float4 s_dyn[];
   float4* s_pos = s_dyn;
   float4* s_tab = s_dyn + halo_cap;
@@ -417,7 +430,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
   // the reads overlap the staging and the pair loop
   const uint32_t i_own = info.z + threadIdx.x;
   NvtIn own{};
-  if (FUSE && i_own < info.w) own = nvt_fused_load(i_own, r, fz);
+  if (FUSE != kFuseNone && i_own < info.w) own = nvt_fused_load(i_own, r, fz);
   if (staged) {
     // four halo particles per thread and pass: their slot and position loads
     // are issued together, so a pass waits for two round trips, not eight
@@ -448,12 +461,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
   }
   __syncthreads();
   if (staged && fast)
-    tile_particles<PP, STR, INIT, true>(pp, info.z, info.w, true, info.y, r, f, w, sts, nbl16, num_nbrs, lane_order,
+    tile_particles<PP, STR, INIT, true, kEnergy>(pp, info.z, info.w, true, info.y, r, f, w, sts, nbl16, num_nbrs, lane_order,
                                          s_pos, s_tab, nt, bx, fb, nvp, max_nbrs, lgp, longest);
   else
-    tile_particles<PP, STR, INIT, false>(pp, info.z, info.w, staged, 0u, r, f, w, sts, nbl16, num_nbrs, lane_order,
+    tile_particles<PP, STR, INIT, false, kEnergy>(pp, info.z, info.w, staged, 0u, r, f, w, sts, nbl16, num_nbrs, lane_order,
                                           s_pos, s_tab, nt, bx, fb, nvp, max_nbrs, lgp, longest);
-  if (FUSE) {
+  if (FUSE != kFuseNone) {
     // the tile's forces are stored (and read back from L2 in slot order);
     // the halo is no longer read, so its LDS holds the reduction
     __syncthreads();
@@ -473,7 +486,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
 // pairs beyond them are outside rc), and for the stepping variants (no
 // stresses, initialising) of a policy whose occupancy target is tunable, the
 // build compiled for rumdx_nblist.tile_waves_per_eu.
-template <class PP, bool STR, bool INIT, bool FUSE>
+template <class PP, bool STR, bool INIT, int FUSE>
 void launch_tiles(const PP& pp, const rumdx_particles* p, const rumdx_nblist* nb, const float* params, uint32_t nt,
                   const Box& bx, uint32_t lgp, const NvtFuse& fz, hipStream_t st) {
   float4* r = reinterpret_cast<float4*>(p->r_dev);
@@ -496,7 +509,7 @@ void launch_tiles(const PP& pp, const rumdx_particles* p, const rumdx_nblist* nb
     if (nb->tile_waves_per_eu == 4u) return launch(k_pair_tiles<PP, STR, INIT, 4, FUSE>);
     // the fused step's update state does not fit six waves' registers (it
     // would spill), and the tile's LDS allows five workgroups per CU anyway
-    if constexpr (!FUSE)
+    if constexpr (FUSE == kFuseNone)
       if (nb->tile_waves_per_eu == 6u) return launch(k_pair_tiles<PP, STR, INIT, 6, FUSE>);
   }
   launch(k_pair_tiles<PP, STR, INIT, PP::kWavesPerEU, FUSE>);
@@ -513,7 +526,7 @@ int launch_pair(const PP& pp, const char* entry, const rumdx_particles* p, const
   const uint32_t lpp = nb != nullptr ? nb->lanes_per_particle : 1u;
   const uint32_t lgp = lpp >= 8u ? 3u : lpp >= 4u ? 2u : lpp >= 2u ? 1u : 0u;
   if (nb != nullptr && nb->nbl16_dev != nullptr) {
-    launch_tiles<PP, STR, INIT, false>(pp, p, nb, params, nt, bx, lgp, NvtFuse{}, st);
+    launch_tiles<PP, STR, INIT, kFuseNone>(pp, p, nb, params, nt, bx, lgp, NvtFuse{}, st);
   } else if (nb != nullptr) {
     // A small sample does not fill the chip: its lists are spread over 16
     // lanes, whatever lanes_per_particle asks (one pass of dependent reads

@@ -43,7 +43,7 @@ struct NvtArgs {
   const float4* f;
   float4* im;
   float4* rlo;
-  rumdx_nh_state* nh;
+  const rumdx_nh_state* nh;
   double* partials;
   const float4* last_r;  // skin check fused when non-null
   uint32_t* nb_flags;
@@ -51,9 +51,7 @@ struct NvtArgs {
   const float4* prune_r;  // inner-list check fused when non-null
   float inner2;
   float dt;
-  float omega2;
   uint32_t on_mask;
-  uint32_t dof;
   uint32_t n;
 };
 
@@ -185,10 +183,7 @@ __global__ __launch_bounds__(kBlock) void k_reduce_f4(const float4* __restrict__
 
 template <bool THERMO, bool HILO, bool SKIN>
 void launch_nvt(const NvtArgs& a, const Box& bx, hipStream_t st) {
-  const uint32_t nb = blocks_for(a.n);
-  hipLaunchKernelGGL((k_nvt<THERMO, HILO, SKIN>), dim3(nb), dim3(kBlock), 0, st, a, bx);
-  if (THERMO)
-    hipLaunchKernelGGL(k_nvt_finish, dim3(1), dim3(kBlock), 0, st, a.partials, ke_partials(a.n), a.nh, a.dt, a.omega2, a.dof);
+  hipLaunchKernelGGL((k_nvt<THERMO, HILO, SKIN>), dim3(blocks_for(a.n)), dim3(kBlock), 0, st, a, bx);
 }
 
 }  // namespace
@@ -204,18 +199,21 @@ extern "C" size_t rumdx_workspace_bytes(uint32_t n) {
   return Workspace::kPartials + sizeof(double) * Workspace::partial_doubles(n);
 }
 
-extern "C" int rumdx_nvt_step(rumdx_particles* p, rumdx_nh_state* nh_dev, float dt, uint32_t thermostat_on_mask,
-                              float omega2, uint32_t dof, const float box[8], rumdx_nblist* nb, void* workspace_dev,
-                              void* stream) {
-  if (p == nullptr || box == nullptr) return fail(RUMDX_E_INVALID, "rumdx_nvt_step: null argument");
+namespace rumdx {
+namespace {
+
+// The leapfrog step without the thermostat's update.
+int nvt_step(const char* entry, rumdx_particles* p, const rumdx_nh_state* nh_dev, float dt,
+             uint32_t thermostat_on_mask, const float* box, rumdx_nblist* nb, void* workspace_dev, void* stream) {
+  const std::string e(entry);
+  if (p == nullptr || box == nullptr) return fail(RUMDX_E_INVALID, e + ": null argument");
   if (p->r_dev == nullptr || p->v_dev == nullptr || p->f_dev == nullptr || p->im_dev == nullptr)
-    return fail(RUMDX_E_INVALID, "rumdx_nvt_step: particle arrays not allocated");
+    return fail(RUMDX_E_INVALID, e + ": particle arrays not allocated");
   const bool thermo = thermostat_on_mask != 0u;
   if (thermo && (nh_dev == nullptr || workspace_dev == nullptr))
-    return fail(RUMDX_E_INVALID, "rumdx_nvt_step: thermostat state and workspace required");
-  if (thermo && dof == 0) return fail(RUMDX_E_INVALID, "rumdx_nvt_step: zero degrees of freedom");
+    return fail(RUMDX_E_INVALID, e + ": thermostat state and workspace required");
   if (nb != nullptr && (nb->flags_dev == nullptr || nb->last_r_dev == nullptr))
-    return fail(RUMDX_E_INVALID, "rumdx_nvt_step: neighbour list not allocated");
+    return fail(RUMDX_E_INVALID, e + ": neighbour list not allocated");
   if (p->n == 0) return RUMDX_OK;
   NvtArgs a{};
   a.r = reinterpret_cast<float4*>(p->r_dev);
@@ -226,9 +224,7 @@ extern "C" int rumdx_nvt_step(rumdx_particles* p, rumdx_nh_state* nh_dev, float 
   a.nh = nh_dev;
   a.partials = workspace_dev ? Workspace::partials(workspace_dev) : nullptr;
   a.dt = dt;
-  a.omega2 = omega2;
   a.on_mask = thermostat_on_mask;
-  a.dof = dof;
   a.n = p->n;
   if (nb != nullptr) {
     a.last_r = reinterpret_cast<const float4*>(nb->last_r_dev);
@@ -251,7 +247,38 @@ extern "C" int rumdx_nvt_step(rumdx_particles* p, rumdx_nh_state* nh_dev, float 
     case 6: launch_nvt<true, true, false>(a, bx, st); break;
     default: launch_nvt<true, true, true>(a, bx, st); break;
   }
-  return check_launch("rumdx_nvt_step");
+  return check_launch(entry);
+}
+
+}  // namespace
+}  // namespace rumdx
+
+extern "C" uint32_t rumdx_nvt_partials(uint32_t n) { return ke_partials(n); }
+
+extern "C" int rumdx_nvt_step_due(rumdx_particles* p, const rumdx_nh_state* nh_dev, float dt,
+                                  uint32_t thermostat_on_mask, const float box[8], rumdx_nblist* nb,
+                                  void* workspace_dev, void* stream) {
+  return nvt_step("rumdx_nvt_step_due", p, nh_dev, dt, thermostat_on_mask, box, nb, workspace_dev, stream);
+}
+
+extern "C" int rumdx_nvt_finish(const rumdx_nh_update* due, void* stream) {
+  if (due == nullptr || due->nh_dev == nullptr || due->workspace_dev == nullptr)
+    return fail(RUMDX_E_INVALID, "rumdx_nvt_finish: null argument");
+  if (due->dof == 0) return fail(RUMDX_E_INVALID, "rumdx_nvt_finish: zero degrees of freedom");
+  hipLaunchKernelGGL(k_nvt_finish, dim3(1), dim3(kBlock), 0, as_stream(stream), finish_args(*due));
+  return check_launch("rumdx_nvt_finish");
+}
+
+extern "C" int rumdx_nvt_step(rumdx_particles* p, rumdx_nh_state* nh_dev, float dt, uint32_t thermostat_on_mask,
+                              float omega2, uint32_t dof, const float box[8], rumdx_nblist* nb, void* workspace_dev,
+                              void* stream) {
+  const bool thermo = thermostat_on_mask != 0u;
+  if (thermo && nh_dev != nullptr && workspace_dev != nullptr && dof == 0)
+    return fail(RUMDX_E_INVALID, "rumdx_nvt_step: zero degrees of freedom");
+  const int rc = nvt_step("rumdx_nvt_step", p, nh_dev, dt, thermostat_on_mask, box, nb, workspace_dev, stream);
+  if (rc != RUMDX_OK || !thermo || p->n == 0) return rc;
+  const rumdx_nh_update due{nh_dev, workspace_dev, ke_partials(p->n), dof, dt, omega2};
+  return rumdx_nvt_finish(&due, stream);
 }
 
 extern "C" int rumdx_zero_momentum(rumdx_particles* p, void* workspace_dev, void* stream) {

@@ -150,18 +150,34 @@ __device__ __forceinline__ void nh_advance(rumdx_nh_state& nh, double ke2, float
 
 namespace {
 
-// UpdateThermostatState: fixed-order sum of the integrator's partials, then
-// the state's update.  One workgroup; the kernel boundary makes the partials
-// visible.
-__global__ __launch_bounds__(kBlock) void k_nvt_finish(const double* __restrict__ partials, uint32_t np,
-                                                       rumdx_nh_state* nh, float dt, float omega2, uint32_t dof) {
-  __shared__ double s_red[kBlock / 64];
-  const double tot = sum_partials(partials, np, 1, s_red);
+// A thermostat update that is due: UpdateThermostatState from the integrator's
+// partials, added in a fixed order by one workgroup.
+struct NvtFinish {
+  const double* partials;
+  uint32_t np;
+  rumdx_nh_state* nh;  // null: none
+  float dt;
+  float omega2;
+  uint32_t dof;
+};
+
+__device__ __forceinline__ void nvt_finish(const NvtFinish& u, double* s_red) {
+  const double tot = sum_partials(u.partials, u.np, 1, s_red);
   if (threadIdx.x == 0) {
-    rumdx_nh_state st = *nh;
-    nh_advance(st, tot, dt, omega2, dof);
-    *nh = st;
+    rumdx_nh_state st = *u.nh;
+    nh_advance(st, tot, u.dt, u.omega2, u.dof);
+    *u.nh = st;
   }
+}
+
+// The kernel boundary makes the partials visible.
+__global__ __launch_bounds__(kBlock) void k_nvt_finish(NvtFinish u) {
+  __shared__ double s_red[kBlock / 64];
+  nvt_finish(u, s_red);
+}
+
+inline NvtFinish finish_args(const rumdx_nh_update& d) {
+  return NvtFinish{Workspace::partials(d.workspace_dev), d.npartials, d.nh_dev, d.dt, d.omega2, d.dof};
 }
 
 }  // namespace

@@ -23,6 +23,7 @@
 #include <utility>
 #include <vector>
 
+#include "leapfrog.h"
 #include "rumdx_common.h"
 #include "tiles.h"
 
@@ -430,7 +431,7 @@ __global__ __launch_bounds__(kBlock) void k_gather(const uint32_t* __restrict__ 
 struct HomeArrays {
   float4* r;
   float4* v;
-  float4* f;
+  float4* f;  // null: forces and virials stay behind (f and w)
   float4* w;
   float4* im;
   float4* rlo;
@@ -504,9 +505,13 @@ struct ResortLds {
 };
 
 __global__ __launch_bounds__(kBlock) void k_tile_resort(uint32_t* __restrict__ flags, SortScratch s, TileGeom tg,
-                                                        Box bx, ParticleArrays o, uint32_t n) {
-  if (!rebuild_pending(flags)) return;
+                                                        Box bx, ParticleArrays o, uint32_t n, NvtFinish due) {
   __shared__ ResortLds L;
+  if (blockIdx.x == tg.ntiles) {  // the workgroup after the tiles' (launched when due.nh is set)
+    nvt_finish(due, reinterpret_cast<double*>(&L));
+    return;
+  }
+  if (!rebuild_pending(flags)) return;
   // tiles in slot order, in dispatch order: a tile waits only on earlier ones
   const uint32_t t = blockIdx.x;
   const uint32_t epoch = flags[RUMDX_FLAG_BUILDS];  // unchanged during the launch
@@ -671,8 +676,10 @@ __global__ __launch_bounds__(kBlock) void k_tile_resort(uint32_t* __restrict__ f
     if (d < n) {  // in range unless particles were lost (then the build is flagged)
       s.t_r[d] = o.r[my];
       s.t_v[d] = o.v[my];
-      s.t_f[d] = o.f[my];
-      s.t_w[d] = o.w[my];
+      if (o.f != nullptr) {
+        s.t_f[d] = o.f[my];
+        s.t_w[d] = o.w[my];
+      }
       s.t_im[d] = o.im[my];
       if (o.rlo != nullptr) s.t_rlo[d] = o.rlo[my];
       s.t_idx[d] = o.idx[my];
@@ -1026,9 +1033,10 @@ __global__ __launch_bounds__(kBuildBlock) void k_build_tiles(uint32_t* __restric
                                                              uint32_t* __restrict__ num_nbrs, uint32_t nvp,
                                                              uint32_t max_nbrs) {
   if (!rebuild_pending(flags)) return;
-  // Arrival at the start (grouped counters, kArriveGroups): its round trip
-  // overlaps the halo loads, and the block that arrives last (every block has
-  // read the request by then) completes the build at its end.
+  // Arrival at the start (grouped counters, kArriveGroups), once every wave of
+  // the block has read the request: its round trip overlaps the halo loads, and
+  // the block that arrives last completes the build at its end.
+  __syncthreads();
   const bool last = threadIdx.x == 0 && grouped_arrival_last(s.arrive);
   __shared__ HaloLds L;
   __shared__ float s_cut[RUMDX_MAX_TYPES * RUMDX_MAX_TYPES];
@@ -1097,8 +1105,10 @@ __global__ __launch_bounds__(kBuildBlock) void k_build_tiles(uint32_t* __restric
     o.r[i] = ri;
     o.last_r[i] = ri;
     o.v[i] = s.t_v[i];
-    o.f[i] = s.t_f[i];
-    o.w[i] = s.t_w[i];
+    if (o.f != nullptr) {
+      o.f[i] = s.t_f[i];
+      o.w[i] = s.t_w[i];
+    }
     o.im[i] = s.t_im[i];
     if (o.rlo != nullptr) o.rlo[i] = s.t_rlo[i];
     o.idx[i] = s.t_idx[i];
@@ -1511,7 +1521,8 @@ int check_sorted_args(const char* entry, const rumdx_particles* p, const rumdx_n
 // The tile build, its finishing kernel and the exclusion pass: the common
 // end of both sorted builds (the particles are staged in sorted order in s,
 // their cell starts in s.start_next).
-void launch_tile_build(rumdx_particles* p, rumdx_nblist* nb, const Box& bx, const SortScratch& s, hipStream_t st) {
+void launch_tile_build(rumdx_particles* p, rumdx_nblist* nb, const Box& bx, const SortScratch& s, hipStream_t st,
+                       bool carry) {
   const TileGeom tg{nb->nc[0],           nb->nc[1],
                     nb->nc[2],           nb->cell_rank_dev,
                     s.start_next,        nb->tile_first_rank_dev,
@@ -1519,7 +1530,8 @@ void launch_tile_build(rumdx_particles* p, rumdx_nblist* nb, const Box& bx, cons
                     nb->halo_cap,        nb->tile_halo_dev,
                     reinterpret_cast<uint4*>(nb->tile_info_dev)};
   const HomeArrays home{reinterpret_cast<float4*>(p->r_dev), reinterpret_cast<float4*>(p->v_dev),
-                        reinterpret_cast<float4*>(p->f_dev), reinterpret_cast<float4*>(p->w_dev),
+                        carry ? reinterpret_cast<float4*>(p->f_dev) : nullptr,
+                        reinterpret_cast<float4*>(p->w_dev),
                         reinterpret_cast<float4*>(p->im_dev), reinterpret_cast<float4*>(p->rlo_dev),
                         p->unsorted_index_dev, reinterpret_cast<float4*>(nb->last_r_dev), nb->slot_cell_dev,
                         nb->lane_order_dev, nb->cell_start_dev};
@@ -1566,14 +1578,22 @@ extern "C" int rumdx_nblist_build_sorted(rumdx_particles* p, rumdx_nblist* nb, c
                      reinterpret_cast<const float4*>(p->f_dev), reinterpret_cast<const float4*>(p->w_dev),
                      reinterpret_cast<const float4*>(p->im_dev), reinterpret_cast<const float4*>(p->rlo_dev),
                      p->unsorted_index_dev, s, p->n);
-  launch_tile_build(p, nb, bx, s, st);
+  launch_tile_build(p, nb, bx, s, st, true);
   return check_launch("rumdx_nblist_build_sorted");
 }
 
 extern "C" int rumdx_nblist_rebuild_sorted(rumdx_particles* p, rumdx_nblist* nb, const float box[8], void* stream) {
+  return rumdx_nblist_rebuild_sorted_due(p, nb, box, 1, nullptr, stream);
+}
+
+extern "C" int rumdx_nblist_rebuild_sorted_due(rumdx_particles* p, rumdx_nblist* nb, const float box[8],
+                                               int carry_forces, const rumdx_nh_update* due, void* stream) {
   int rc = check_sorted_args("rumdx_nblist_rebuild_sorted", p, nb, box);
   if (rc != RUMDX_OK) return rc;
+  if (due != nullptr && (due->nh_dev == nullptr || due->workspace_dev == nullptr || due->dof == 0))
+    return fail(RUMDX_E_INVALID, "rumdx_nblist_rebuild_sorted: incomplete thermostat update");
   if (p->n == 0) return RUMDX_OK;
+  const bool carry = carry_forces != 0;
   const uint32_t ncells =
       static_cast<uint32_t>(nb->nc[0]) * static_cast<uint32_t>(nb->nc[1]) * static_cast<uint32_t>(nb->nc[2]);
   const Box bx = make_box(box);
@@ -1583,11 +1603,13 @@ extern "C" int rumdx_nblist_rebuild_sorted(rumdx_particles* p, rumdx_nblist* nb,
   const TileGeom tg{nb->nc[0], nb->nc[1], nb->nc[2], nb->cell_rank_dev, nb->cell_start_dev,
                     nb->tile_first_rank_dev, nb->tile_origin_dev, nb->ntiles, nb->halo_cap, nullptr, nullptr};
   const ParticleArrays old{reinterpret_cast<const float4*>(p->r_dev), reinterpret_cast<const float4*>(p->v_dev),
-                           reinterpret_cast<const float4*>(p->f_dev), reinterpret_cast<const float4*>(p->w_dev),
-                           reinterpret_cast<const float4*>(p->im_dev), reinterpret_cast<const float4*>(p->rlo_dev),
+                           carry ? reinterpret_cast<const float4*>(p->f_dev) : nullptr,
+                           reinterpret_cast<const float4*>(p->w_dev), reinterpret_cast<const float4*>(p->im_dev), reinterpret_cast<const float4*>(p->rlo_dev),
                            p->unsorted_index_dev};
-  hipLaunchKernelGGL(k_tile_resort, dim3(nb->ntiles), dim3(kBlock), 0, st, nb->flags_dev, s, tg, bx, old, p->n);
-  launch_tile_build(p, nb, bx, s, st);
+  const NvtFinish fin = due != nullptr ? finish_args(*due) : NvtFinish{};
+  hipLaunchKernelGGL(k_tile_resort, dim3(nb->ntiles + (due != nullptr ? 1u : 0u)), dim3(kBlock), 0, st, nb->flags_dev,
+                     s, tg, bx, old, p->n, fin);
+  launch_tile_build(p, nb, bx, s, st, carry);
   return check_launch("rumdx_nblist_rebuild_sorted");
 }
 

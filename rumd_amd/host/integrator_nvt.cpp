@@ -65,19 +65,45 @@ void IntegratorNVT::PullState() {
 void IntegratorNVT::Integrate() {
   if (!S || !S->GetNumberOfParticles()) throw RUMD_Error("IntegratorNVT", "Integrate", kNoSample);
   if (!S->GetSimulationBox()) throw RUMD_Error("IntegratorNVT", "Integrate", "no simulation box");
+  FinishDue();
   NeighborList* nl = S->FusedCheckList();
-  rumdx_check(rumdx_nvt_step(S->GetParticleData().Descriptor(), d_state_.get(), timeStep, thermostat_on_, Omega2(),
-                             S->GetNumberOfDOFs(), S->GetSimulationBox()->GetBox8(), nl ? nl->Descriptor() : nullptr,
-                             S->Workspace(), S->GetStream()),
+  rumdx_check(rumdx_nvt_step_due(S->GetParticleData().Descriptor(), d_state_.get(), timeStep, thermostat_on_,
+                                 S->GetSimulationBox()->GetBox8(), nl ? nl->Descriptor() : nullptr, S->Workspace(),
+                                 S->GetStream()),
               "IntegratorNVT", "Integrate");
   if (nl) nl->NoteFusedCheck();
+  NoteDue(rumdx_nvt_partials(S->GetNumberOfParticles()));
 }
 
-void IntegratorNVT::IntegrateFused(PairPotential& pp) {
+void IntegratorNVT::IntegrateFused(PairPotential& pp, bool store_forces) {
   if (!S || !S->GetNumberOfParticles()) throw RUMD_Error("IntegratorNVT", "Integrate", kNoSample);
   if (!S->GetSimulationBox()) throw RUMD_Error("IntegratorNVT", "Integrate", "no simulation box");
-  pp.CalcFIntegrateNVT(d_state_.get(), timeStep, thermostat_on_, Omega2(), S->GetNumberOfDOFs());
+  const unsigned np = pp.CalcFIntegrateNVT(d_state_.get(), timeStep, thermostat_on_, store_forces);
   pp.GetNeighborList().NoteFusedCheck();
+  NoteDue(np);
+}
+
+void IntegratorNVT::NoteDue(unsigned npartials) {
+  if (!thermostat_on_) return;
+  due_partials_ = npartials;
+  if (!defer_) FinishDue();
+}
+
+bool IntegratorNVT::TakeDue(rumdx_nh_update* out) {
+  if (due_partials_ == 0) return false;
+  *out = rumdx_nh_update{d_state_.get(), S->Workspace(), due_partials_, S->GetNumberOfDOFs(), timeStep, Omega2()};
+  due_partials_ = 0;
+  return true;
+}
+
+void IntegratorNVT::FinishDue() {
+  rumdx_nh_update u;
+  if (TakeDue(&u)) rumdx_check(rumdx_nvt_finish(&u, S->GetStream()), "IntegratorNVT", "Integrate");
+}
+
+void IntegratorNVT::Defer(bool on) {
+  defer_ = on;
+  if (!on) FinishDue();
 }
 
 void IntegratorNVT::IntegrateChain(PairPotential& pp, unsigned nsteps) {

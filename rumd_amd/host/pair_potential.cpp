@@ -336,7 +336,7 @@ void NeighborList::EnsureAllocated() {
   if (!allocated_ || allocated_nvp_ != sample_->GetNumberOfVirtualParticles()) Allocate();
 }
 
-void NeighborList::UpdateNBlist() {
+void NeighborList::UpdateNBlist(bool forces_follow) {
   if (!sample_) throw RUMD_Error("NeighborList", "UpdateNBlist", "no sample");
   const Method method = GetResolvedMethod();
   if (method == NONE) return;
@@ -350,7 +350,12 @@ void NeighborList::UpdateNBlist() {
     // skin-triggered rebuilds re-sort tile by tile; the first build, and any
     // after the host changed positions or arrays, sorts from scratch
     const bool resort = UseTileResort() && !force_full_sort_;
-    const int rc = resort ? rumdx_nblist_rebuild_sorted(p, &desc_, box, st) : rumdx_nblist_build_sorted(p, &desc_, box, st);
+    rumdx_nh_update due;
+    auto* itg = dynamic_cast<IntegratorNVT*>(sample_->GetIntegrator());
+    if (itg != nullptr && !resort) itg->FinishDue();
+    const bool take = itg != nullptr && itg->TakeDue(&due);
+    const int rc = resort ? rumdx_nblist_rebuild_sorted_due(p, &desc_, box, forces_follow ? 0 : 1, take ? &due : nullptr, st)
+                          : rumdx_nblist_build_sorted(p, &desc_, box, st);
     rumdx_check(rc, "NeighborList", "UpdateNBlist");
     sort_valid_ = true;
     sample_->BumpSlotEpoch();  // the build may have moved particles between slots
@@ -624,19 +629,21 @@ bool PairPotential::CanFuseStep() {
   return 256 + sizeof(double) * static_cast<size_t>(nb->ntiles) <= rumdx_workspace_bytes(sample->GetNumberOfParticles());
 }
 
-void PairPotential::CalcFIntegrateNVT(rumdx_nh_state* nh_dev, float dt, unsigned thermostat_on_mask, float omega2,
-                                      unsigned dof) {
+unsigned PairPotential::CalcFIntegrateNVT(const rumdx_nh_state* nh_dev, float dt, unsigned thermostat_on_mask,
+                                          bool store_forces) {
   if (!sample) throw RUMD_Error(GetID_String(), "CalcF", "no sample");
   if (table_types_ != sample->GetNumberOfTypes()) Initialize();
-  neighborList.UpdateNBlist();
+  neighborList.UpdateNBlist(true);
   ParticleData& pd = sample->GetParticleData();
   if (!pd.HasNextPositions())
     throw RUMD_Error(GetID_String(), "CalcF", "the fused step needs the sample's second position array");
-  rumdx_check(rumdx_pair_lj_nvt(pd.Descriptor(), neighborList.Descriptor(), d_params_.get(), table_types_,
-                                sample->GetSimulationBox()->GetBox8(), cutoff_method_, pd.NextPositions(), nh_dev, dt,
-                                thermostat_on_mask, omega2, dof, sample->Workspace(), sample->GetStream()),
+  rumdx_check(rumdx_pair_lj_nvt_due(pd.Descriptor(), neighborList.Descriptor(), d_params_.get(), table_types_,
+                                    sample->GetSimulationBox()->GetBox8(), cutoff_method_, pd.NextPositions(), nh_dev,
+                                    dt, thermostat_on_mask, store_forces ? 1 : 0, sample->Workspace(),
+                                    sample->GetStream()),
               GetID_String().c_str(), "CalcF");
   pd.SwapPositions();
+  return neighborList.Descriptor()->ntiles;
 }
 
 bool PairPotential::CanChainSteps() {
@@ -678,7 +685,7 @@ void PairPotential::SetFP64Forces(bool on) {
 void PairPotential::CalcF(bool initialize, bool calc_stresses) {
   if (!sample) throw RUMD_Error(GetID_String(), "CalcF", "no sample");
   if (table_types_ != sample->GetNumberOfTypes()) Initialize();
-  neighborList.UpdateNBlist();
+  neighborList.UpdateNBlist(initialize);
   LaunchForce(sample->GetParticleData().Descriptor(), initialize, calc_stresses, sample->GetStream(), "CalcF");
 }
 

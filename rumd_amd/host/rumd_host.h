@@ -179,8 +179,10 @@ class NeighborList {
   unsigned GetNumberOfBuilds();
   // Marks the list stale: the next UpdateNBlist rebuilds (ResetNeighborList).
   void ResetNeighborList();
-  // Launches the device-side check and build chain (UpdateNBlist).
-  void UpdateNBlist();
+  // Launches the device-side check and build chain (UpdateNBlist).  With
+  // forces_follow the caller initialises forces and virials next, so a rebuild
+  // need not move them.
+  void UpdateNBlist(bool forces_follow = false);
   // Allocates buffers now (before a graph capture, which may not allocate).
   void EnsureAllocated();
   // Called after an integrator step that ran this list's skin check fused.
@@ -328,7 +330,9 @@ class PairPotential : public Potential {
   bool CanFuseStep();
   // CalcF(true, false) and the NVT step in one kernel; the new positions go to
   // the sample's second position array, which then becomes the current one.
-  void CalcFIntegrateNVT(rumdx_nh_state* nh_dev, float dt, unsigned thermostat_on_mask, float omega2, unsigned dof);
+  // The thermostat's update is left due; without store_forces the step leaves
+  // energies and virials out.  Returns the number of kinetic-energy partials.
+  unsigned CalcFIntegrateNVT(const rumdx_nh_state* nh_dev, float dt, unsigned thermostat_on_mask, bool store_forces);
   // Average duration (ms) of the fused step kernel alone over `reps`
   // launches, bracketed by HIP events like TimeForceKernel.  The launches
   // advance copies of the velocities, images and low position parts, write
@@ -754,7 +758,17 @@ class IntegratorNVT : public Integrator {
   void SetTemperatureChangePerTimeStep(double dT);
   // The step with the forces of `pp` computed in the same kernel
   // (PairPotential::CalcFIntegrateNVT): CalcF and Integrate of Simulation.Run.
-  void IntegrateFused(PairPotential& pp);
+  void IntegrateFused(PairPotential& pp, bool store_forces);
+  // While recording a block of steps over sorted lists, a step's thermostat
+  // update is left to the next step's list update (NeighborList takes it with
+  // TakeDue) or, at the end, to Defer(false): one launch less per step.
+  void Defer(bool on);
+  bool TakeDue(rumdx_nh_update* out);
+  void FinishDue();
+  void DropDue() {  // a recording failed: nothing ran
+    defer_ = false;
+    due_partials_ = 0;
+  }
   // nsteps steps as a chain of one-kernel steps (PairPotential::ChainStep).
   void IntegrateChain(PairPotential& pp, unsigned nsteps);
 
@@ -763,6 +777,10 @@ class IntegratorNVT : public Integrator {
   void PullState();
   // omega^2 = 4 pi^2 / tau^2 formed in double, passed as float (src/IntegratorNVT.cu:88)
   float Omega2() const;
+  // Notes the update of a step just launched, done at once unless deferred.
+  void NoteDue(unsigned npartials);
+  bool defer_ = false;
+  unsigned due_partials_ = 0;  // 0: none due
   unsigned thermostat_on_ = 0;
   float relaxation_time_ = 0.2f;
   rumdx_nh_state host_state_{0.0, 0.0, 0.0, 0.0};
@@ -915,7 +933,7 @@ class Sample {
   };
   void PrepareRun();
   PairPotential* ChainPotential();
-  void StepOnce(bool zero_momentum);
+  void StepOnce(bool zero_momentum, bool store_forces = true);
   Block CaptureBlock(unsigned nsteps, bool reset_first);
   unsigned pb_ = 0, tp_ = 0;
   unsigned user_dofs_ = 0;

@@ -268,12 +268,12 @@ void Sample::PrepareRun() {
   if (FusedStepPotential() != nullptr || ChainPotential() != nullptr) pd_.EnsureNextPositions();
 }
 
-void Sample::StepOnce(bool zero_momentum) {
+void Sample::StepOnce(bool zero_momentum, bool store_forces) {
   if (zero_momentum) itg_->SetMomentumToZero();
   PairPotential* pp = FusedStepPotential();
   if (pp != nullptr && pd_.HasNextPositions()) {
     BumpSlotEpoch();
-    static_cast<IntegratorNVT*>(itg_)->IntegrateFused(*pp);
+    static_cast<IntegratorNVT*>(itg_)->IntegrateFused(*pp, store_forces);
     return;
   }
   CalcF(false);
@@ -314,12 +314,17 @@ Sample::Block Sample::CaptureBlock(unsigned nsteps, bool reset_first) {
       if (reset_first) itg_->SetMomentumToZero();
       static_cast<IntegratorNVT*>(itg_)->IntegrateChain(*chain, nsteps);
     } else {
-      for (unsigned k = 0; k < nsteps; ++k) StepOnce(k == 0 && reset_first);
+      // the forces of the inner steps are replaced before anything reads them
+      auto* itg = nl != nullptr && nl->IsSorted() ? dynamic_cast<IntegratorNVT*>(itg_) : nullptr;
+      if (itg) itg->Defer(true);
+      for (unsigned k = 0; k < nsteps; ++k) StepOnce(k == 0 && reset_first, k + 1 == nsteps);
+      if (itg) itg->Defer(false);
     }
     // fused steps alternate the two position arrays: the graph ends in the
     // one it starts from (a copy after an odd number of them)
     pd_.MovePositionsTo(home, stream_);
   } catch (...) {
+    if (auto* itg = dynamic_cast<IntegratorNVT*>(itg_)) itg->DropDue();
     (void)hipStreamEndCapture(stream_, &g);
     if (g) (void)hipGraphDestroy(g);
     if (pd_.d_r.get() != home) pd_.SwapPositions();  // nothing ran
