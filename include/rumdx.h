@@ -281,6 +281,9 @@ int rumdx_nblist_build_sorted(rumdx_particles* p, rumdx_nblist* nb, const float 
  * carry no launch for it.  Call it before reading those flags.  Returns
  * RUMDX_OK without a launch when the list has no sorted build arrays. */
 int rumdx_nblist_build_stats(const rumdx_particles* p, rumdx_nblist* nb, void* stream);
+/* The same, then the RUMDX_NB_FLAGS flags copied to out (device memory, or
+ * pinned host memory to be read after the stream's next synchronisation). */
+int rumdx_nblist_read_flags(const rumdx_particles* p, rumdx_nblist* nb, uint32_t* out, void* stream);
 
 /* The same result as rumdx_nblist_build_sorted -- particle order, cells and
  * lists bit for bit -- for particles that a previous sorted build of this list
@@ -518,6 +521,18 @@ int rumdx_kinetic_energy(const rumdx_particles* p, const rumdx_nh_state* nh_dev,
  * bitwise reproducible. */
 int rumdx_reduce_f4(const float* arr4_dev, uint32_t n, uint32_t comp_mask, double* out_dev,
                     void* workspace_dev, void* stream);
+
+/* The kinetic part of Sample::GetStress (src/Sample.cu:393-444): out_dev[0..5] =
+ * sum_i 2 m v_a v_b for (xx, yy, zz, yz, xz, xy), float products added in FP64
+ * in a fixed order.  Six doubles. */
+int rumdx_kinetic_stress(const rumdx_particles* p, double* out_dev, void* workspace_dev, void* stream);
+
+/* Particles first .. first + count - 1 of a float4 array in original order:
+ * the first ncomp (1 to 4) components of each, packed, to out (device memory or
+ * pinned host memory).  slot_of_dev: rumdx_slot_index's table, or NULL when the
+ * slots are in original order. */
+int rumdx_read_original(const float* arr4_dev, const uint32_t* slot_of_dev, uint32_t first, uint32_t count,
+                        uint32_t ncomp, float* out, void* stream);
 
 /* rumdx_reduce_f4 without a caller workspace, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,

@@ -47,7 +47,7 @@ __device__ __forceinline__ double3 displacement_f64(float4 a, float4 b, const Bo
 __global__ __launch_bounds__(kBlock) void k_slot_index(const uint32_t* __restrict__ idx,
                                                        uint32_t* __restrict__ slot_of, uint32_t n) {
   const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-  if (s < n) slot_of[idx[s]] = s;
+  if (s < n && idx[s] < n) slot_of[idx[s]] = s;  // a permutation of 0 .. n-1
 }
 
 struct BondSums {

@@ -91,12 +91,13 @@ __global__ __launch_bounds__(kBlock) void k_nvt(NvtArgs a, Box bx) {
   }
 }
 
-// Fixed-order sums of `ncomp`-strided block partials into out[c] * scale.
+// Fixed-order sums of `ncomp`-strided block partials into out[c] * scale, c below
+// nout.
 __global__ __launch_bounds__(kBlock) void k_finish_sums(const double* __restrict__ partials, uint32_t np,
                                                         uint32_t ncomp, uint32_t mask, double scale,
-                                                        double* __restrict__ out) {
+                                                        double* __restrict__ out, uint32_t nout) {
   __shared__ double s_red[kBlock / 64];
-  for (uint32_t c = 0; c < ncomp; ++c) {
+  for (uint32_t c = 0; c < nout; ++c) {
     double s = 0.0;
     if ((mask >> c) & 1u) s = sum_partials(partials + c, np, ncomp, s_red);
     if (threadIdx.x == 0) out[c] = s * scale;
@@ -186,10 +187,78 @@ void launch_nvt(const NvtArgs& a, const Box& bx, hipStream_t st) {
   hipLaunchKernelGGL((k_nvt<THERMO, HILO, SKIN>), dim3(blocks_for(a.n)), dim3(kBlock), 0, st, a, bx);
 }
 
+// ---------------------------------------------------------------- kinetic stress
+// Sample::GetStress's kinetic sums (src/Sample.cu:420-437): components xx, yy,
+// zz, yz (SET 0) or xz, xy (SET 1) as block partials, 4 per block.
+template <int SET>
+__global__ __launch_bounds__(kBlock) void k_kinetic_stress(const float4* __restrict__ v, double* partials, uint32_t n) {
+#pragma clang fp contract(off)
+  __shared__ double s_red[kBlock / 64];
+  const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
+  const uint32_t i = b * kBlock + threadIdx.x;
+  float c[4] = {0.f, 0.f, 0.f, 0.f};
+  if (i < n) {
+    const float4 x = v[i];
+    const float m2 = 2.f / x.w;
+    if (SET == 0) {
+      c[0] = m2 * x.x * x.x;
+      c[1] = m2 * x.y * x.y;
+      c[2] = m2 * x.z * x.z;
+      c[3] = m2 * x.y * x.z;
+    } else {
+      c[0] = m2 * x.x * x.z;
+      c[1] = m2 * x.x * x.y;
+    }
+  }
+  for (int k = 0; k < (SET == 0 ? 4 : 2); ++k) {
+    const double s = block_sum(static_cast<double>(c[k]), s_red);
+    if (threadIdx.x == 0) partials[static_cast<size_t>(b) * 4 + k] = s;
+  }
+}
+
+// ---------------------------------------------------------------- original order
+// One packed component per thread, so the writes (to pinned host memory as a
+// rule) are contiguous; the reads gather within the float4 array.
+__global__ __launch_bounds__(kBlock) void k_read_original(const float* __restrict__ a,
+                                                          const uint32_t* __restrict__ slot_of, uint32_t first,
+                                                          uint32_t count, uint32_t nc, float* __restrict__ out) {
+  const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+  if (t >= count * nc) return;
+  const uint32_t i = first + t / nc;
+  out[t] = a[4ull * (slot_of != nullptr ? slot_of[i] : i) + t % nc];
+}
+
 }  // namespace
 }  // namespace rumdx
 
 using namespace rumdx;
+
+extern "C" int rumdx_kinetic_stress(const rumdx_particles* p, double* out_dev, void* workspace_dev, void* stream) {
+  if (p == nullptr || p->v_dev == nullptr || out_dev == nullptr || workspace_dev == nullptr)
+    return fail(RUMDX_E_INVALID, "rumdx_kinetic_stress: null argument");
+  if (p->n == 0) return fail(RUMDX_E_INVALID, "rumdx_kinetic_stress: sample has no particles");
+  const hipStream_t st = as_stream(stream);
+  const uint32_t nb = blocks_for(p->n);
+  const float4* v = reinterpret_cast<const float4*>(p->v_dev);
+  double* part = Workspace::partials(workspace_dev);
+  hipLaunchKernelGGL(k_kinetic_stress<0>, dim3(nb), dim3(kBlock), 0, st, v, part, p->n);
+  hipLaunchKernelGGL(k_finish_sums, dim3(1), dim3(kBlock), 0, st, part, nb, 4u, 15u, 1.0, out_dev, 4u);
+  hipLaunchKernelGGL(k_kinetic_stress<1>, dim3(nb), dim3(kBlock), 0, st, v, part, p->n);
+  hipLaunchKernelGGL(k_finish_sums, dim3(1), dim3(kBlock), 0, st, part, nb, 4u, 3u, 1.0, out_dev + 4, 2u);
+  return check_launch("rumdx_kinetic_stress");
+}
+
+extern "C" int rumdx_read_original(const float* arr4_dev, const uint32_t* slot_of_dev, uint32_t first, uint32_t count,
+                                   uint32_t ncomp, float* out, void* stream) {
+  if (arr4_dev == nullptr || out == nullptr || ncomp < 1 || ncomp > 4)
+    return fail(RUMDX_E_INVALID, "rumdx_read_original: invalid argument");
+  if (count == 0) return RUMDX_OK;
+  if (static_cast<uint64_t>(count) * ncomp >= (1ull << 32))
+    return fail(RUMDX_E_INVALID, "rumdx_read_original: too many particles at once");
+  hipLaunchKernelGGL(k_read_original, dim3(blocks_for(count * ncomp)), dim3(kBlock), 0, as_stream(stream), arr4_dev,
+                     slot_of_dev, first, count, ncomp, out);
+  return check_launch("rumdx_read_original");
+}
 
 extern "C" int rumdx_version(void) { return RUMDX_VERSION; }
 
@@ -291,7 +360,7 @@ extern "C" int rumdx_zero_momentum(rumdx_particles* p, void* workspace_dev, void
   hipLaunchKernelGGL(k_momentum_sum, dim3(nb), dim3(kBlock), 0, st, reinterpret_cast<const float4*>(p->v_dev),
                      Workspace::partials(workspace_dev), p->n);
   hipLaunchKernelGGL(k_finish_sums, dim3(1), dim3(kBlock), 0, st, Workspace::partials(workspace_dev), nb, 4u, 15u, 1.0,
-                     tot);
+                     tot, 4u);
   hipLaunchKernelGGL(k_momentum_apply, dim3(nb), dim3(kBlock), 0, st, reinterpret_cast<float4*>(p->v_dev), tot, p->n);
   return check_launch("rumdx_zero_momentum");
 }
@@ -308,7 +377,7 @@ extern "C" int rumdx_kinetic_energy(const rumdx_particles* p, const rumdx_nh_sta
                      reinterpret_cast<const float4*>(p->v_dev), reinterpret_cast<const float4*>(p->f_dev), nh_dev, dt,
                      thermostat_on_mask, Workspace::partials(workspace_dev), p->n);
   hipLaunchKernelGGL(k_finish_sums, dim3(1), dim3(kBlock), 0, as_stream(stream), Workspace::partials(workspace_dev), nb,
-                     1u, 1u, 0.5, out_dev);
+                     1u, 1u, 0.5, out_dev, 1u);
   return check_launch("rumdx_kinetic_energy");
 }
 
@@ -369,7 +438,7 @@ extern "C" int rumdx_reduce_f4_static(const float* arr4_dev, uint32_t n, uint32_
   hipLaunchKernelGGL(k_reduce_f4, dim3(nb), dim3(kBlock), 0, as_stream(stream), reinterpret_cast<const float4*>(arr4_dev),
                      comp_mask & 15u, partials, n);
   hipLaunchKernelGGL(k_finish_sums, dim3(1), dim3(kBlock), 0, as_stream(stream), partials, nb, 4u, comp_mask & 15u,
-                     1.0, out_dev);
+                     1.0, out_dev, 4u);
   return check_launch(entry);
 }
 
@@ -382,6 +451,6 @@ extern "C" int rumdx_reduce_f4(const float* arr4_dev, uint32_t n, uint32_t comp_
   hipLaunchKernelGGL(k_reduce_f4, dim3(nb), dim3(kBlock), 0, as_stream(stream), reinterpret_cast<const float4*>(arr4_dev),
                      comp_mask & 15u, Workspace::partials(workspace_dev), n);
   hipLaunchKernelGGL(k_finish_sums, dim3(1), dim3(kBlock), 0, as_stream(stream), Workspace::partials(workspace_dev), nb,
-                     4u, comp_mask & 15u, 1.0, out_dev);
+                     4u, comp_mask & 15u, 1.0, out_dev, 4u);
   return check_launch("rumdx_reduce_f4");
 }

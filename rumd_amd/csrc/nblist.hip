@@ -690,12 +690,17 @@ __global__ __launch_bounds__(kBlock) void k_tile_resort(uint32_t* __restrict__ f
 // The statistics of the last sorted build from its per-tile records: longest
 // list (kept as the maximum with the old value), largest halo and largest
 // tile.  One workgroup, launched on request between steps rather than after
-// every build, so captured steps carry no launch for it.
+// every build, so captured steps carry no launch for it.  With out the flags go
+// there too (without tile records nothing else is done).
 __global__ __launch_bounds__(kBlock) void k_build_stats(uint32_t* __restrict__ flags,
                                                         const uint4* __restrict__ tile_info,
-                                                        const uint32_t* __restrict__ tile_max, uint32_t ntiles) {
-  if (flags[RUMDX_FLAG_STATS] == 0u) return;
+                                                        const uint32_t* __restrict__ tile_max, uint32_t ntiles,
+                                                        uint32_t* __restrict__ out) {
   __shared__ uint32_t s_max[kBlock / 64];
+  if (tile_info == nullptr || flags[RUMDX_FLAG_STATS] == 0u) {
+    if (out != nullptr && threadIdx.x < RUMDX_NB_FLAGS) out[threadIdx.x] = flags[threadIdx.x];
+    return;
+  }
   uint32_t ml = 0, mh = 0, mt = 0;
   for (uint32_t t = threadIdx.x; t < ntiles; t += kBlock) {
     const uint4 info = tile_info[t];
@@ -711,6 +716,8 @@ __global__ __launch_bounds__(kBlock) void k_build_stats(uint32_t* __restrict__ f
     flags[RUMDX_FLAG_MAXHALO] = mh;
     flags[RUMDX_FLAG_MAXTILE] = mt;
     flags[RUMDX_FLAG_STATS] = 0u;
+    if (out != nullptr)
+      for (uint32_t k = 0; k < RUMDX_NB_FLAGS; ++k) out[k] = flags[k];
   }
 }
 
@@ -1613,17 +1620,33 @@ extern "C" int rumdx_nblist_rebuild_sorted_due(rumdx_particles* p, rumdx_nblist*
   return check_launch("rumdx_nblist_rebuild_sorted");
 }
 
-extern "C" int rumdx_nblist_build_stats(const rumdx_particles* p, rumdx_nblist* nb, void* stream) {
+namespace rumdx {
+namespace {
+
+int build_stats(const char* entry, const rumdx_particles* p, rumdx_nblist* nb, uint32_t* out, void* stream) {
   if (p == nullptr || nb == nullptr || nb->flags_dev == nullptr)
-    return fail(RUMDX_E_INVALID, "rumdx_nblist_build_stats: null argument");
-  if (nb->nbl16_dev == nullptr || nb->tile_info_dev == nullptr || nb->sort_scratch_dev == nullptr || nb->ntiles == 0)
-    return RUMDX_OK;  // no sorted build: the N2 build keeps the flags itself
+    return fail(RUMDX_E_INVALID, std::string(entry) + ": null argument");
+  const bool sorted =
+      nb->nbl16_dev != nullptr && nb->tile_info_dev != nullptr && nb->sort_scratch_dev != nullptr && nb->ntiles != 0;
+  if (!sorted && out == nullptr) return RUMDX_OK;  // the N2 build keeps the flags itself
   const uint32_t ncells =
       static_cast<uint32_t>(nb->nc[0]) * static_cast<uint32_t>(nb->nc[1]) * static_cast<uint32_t>(nb->nc[2]);
-  const SortScratch s = carve(nb->sort_scratch_dev, p->nvp, ncells);
   hipLaunchKernelGGL(k_build_stats, dim3(1), dim3(kBlock), 0, as_stream(stream), nb->flags_dev,
-                     reinterpret_cast<const uint4*>(nb->tile_info_dev), s.tile_max, nb->ntiles);
-  return check_launch("rumdx_nblist_build_stats");
+                     sorted ? reinterpret_cast<const uint4*>(nb->tile_info_dev) : nullptr,
+                     sorted ? carve(nb->sort_scratch_dev, p->nvp, ncells).tile_max : nullptr, nb->ntiles, out);
+  return check_launch(entry);
+}
+
+}  // namespace
+}  // namespace rumdx
+
+extern "C" int rumdx_nblist_build_stats(const rumdx_particles* p, rumdx_nblist* nb, void* stream) {
+  return build_stats("rumdx_nblist_build_stats", p, nb, nullptr, stream);
+}
+
+extern "C" int rumdx_nblist_read_flags(const rumdx_particles* p, rumdx_nblist* nb, uint32_t* out, void* stream) {
+  if (out == nullptr) return fail(RUMDX_E_INVALID, "rumdx_nblist_read_flags: null argument");
+  return build_stats("rumdx_nblist_read_flags", p, nb, out, stream);
 }
 
 extern "C" int rumdx_tile_shape(const int32_t nc[3]) {

@@ -1,6 +1,8 @@
 // Errors, device memory, the Device singleton and simulation boxes.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstring>
 #include <sstream>
 
 #include "rumd_host.h"
@@ -64,6 +66,76 @@ template class DeviceArray<uint16_t>;
 template class DeviceArray<char>;
 template class DeviceArray<rumdx_nh_state>;
 template class DeviceArray<rumdx_replica>;
+
+// ------------------------------------------------------------------ pinned host memory
+template <class T>
+void PinnedArray<T>::resize(size_t n) {
+  if (n == n_) return;
+  release();
+  if (n == 0) return;
+  void* p = nullptr;
+  hip_check(hipHostMalloc(&p, n * sizeof(T), hipHostMallocDefault), "PinnedArray", "resize");
+  std::memset(p, 0, n * sizeof(T));
+  ptr_ = static_cast<T*>(p);
+  n_ = n;
+}
+
+template <class T>
+void PinnedArray<T>::release() {
+  if (ptr_) (void)hipHostFree(ptr_);
+  ptr_ = nullptr;
+  n_ = 0;
+}
+
+template class PinnedArray<float>;
+template class PinnedArray<double>;
+template class PinnedArray<uint32_t>;
+
+OriginalOrderReader::~OriginalOrderReader() {
+  for (hipEvent_t e : done_)
+    if (e) (void)hipEventDestroy(e);
+}
+
+void OriginalOrderReader::Read(const float* arr4, const uint32_t* unsorted_index, unsigned n, unsigned ncomp,
+                               float* out, hipStream_t st) {
+  if (n == 0) return;
+  const uint32_t* slot_of = nullptr;
+  if (unsorted_index != nullptr) {
+    if (slot_of_.size() < n) slot_of_.resize(n);
+    rumdx_particles p{};
+    p.unsorted_index_dev = const_cast<uint32_t*>(unsorted_index);
+    p.n = p.nvp = n;
+    rumdx_check(rumdx_slot_index(&p, slot_of_.get(), st), "ParticleData", "Get");
+    slot_of = slot_of_.get();
+  }
+  const unsigned per = static_cast<unsigned>(kChunk / ncomp);  // particles per chunk
+  const size_t half = std::min<size_t>(static_cast<size_t>(n) * ncomp, kChunk);
+  const size_t need = n > per ? 2 * half : half;
+  if (stage_.size() < need) stage_.resize(need);
+  if (n <= per) {
+    rumdx_check(rumdx_read_original(arr4, slot_of, 0, n, ncomp, stage_.get(), st), "ParticleData", "Get");
+    hip_check(hipStreamSynchronize(st), "ParticleData", "Get");
+    std::memcpy(out, stage_.get(), static_cast<size_t>(n) * ncomp * sizeof(float));
+    return;
+  }
+  for (hipEvent_t& e : done_)
+    if (e == nullptr) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "ParticleData", "Get");
+  const unsigned chunks = (n + per - 1) / per;
+  for (unsigned c = 0; c <= chunks; ++c) {
+    if (c < chunks) {
+      const unsigned first = c * per, count = std::min(per, n - first);
+      rumdx_check(rumdx_read_original(arr4, slot_of, first, count, ncomp, stage_.get() + (c % 2) * half, st),
+                  "ParticleData", "Get");
+      hip_check(hipEventRecord(done_[c % 2], st), "ParticleData", "Get");
+    }
+    if (c > 0) {
+      const unsigned first = (c - 1) * per, count = std::min(per, n - first);
+      hip_check(hipEventSynchronize(done_[(c - 1) % 2]), "ParticleData", "Get");
+      std::memcpy(out + static_cast<size_t>(first) * ncomp, stage_.get() + ((c - 1) % 2) * half,
+                  static_cast<size_t>(count) * ncomp * sizeof(float));
+    }
+  }
+}
 
 // ------------------------------------------------------------------ Device
 Device& Device::GetDevice() {

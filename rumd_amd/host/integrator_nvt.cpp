@@ -158,11 +158,8 @@ double IntegratorNVT::GetKineticEnergy(bool) {
   rumdx_check(rumdx_kinetic_energy(S->GetParticleData().Descriptor(), d_state_.get(), timeStep, thermostat_on_,
                                    S->ScalarOut(), S->Workspace(), S->GetStream()),
               "IntegratorNVT", "GetKineticEnergy");
-  double ke = 0.0;
-  hip_check(hipMemcpyAsync(&ke, S->ScalarOut(), sizeof(double), hipMemcpyDeviceToHost, S->GetStream()),
-            "IntegratorNVT", "GetKineticEnergy");
   hip_check(hipStreamSynchronize(S->GetStream()), "IntegratorNVT", "GetKineticEnergy");
-  return ke;
+  return S->ScalarOut()[0];
 }
 
 void IntegratorNVT::SetTimeStep(float dt) {

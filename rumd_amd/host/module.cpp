@@ -19,12 +19,8 @@ py::array_t<float> get_xyz(Sample& s, const char* what) {
   const unsigned n = s.GetNumberOfParticles();
   if (!n) throw RUMD_Error("Sample", "Get", "Sample has no particles");
   s.Synchronize();
-  std::vector<float> a(4ull * n);
-  s.GetParticleData().Get(what, a.data(), s.GetStream());
   py::array_t<float> out({static_cast<py::ssize_t>(n), static_cast<py::ssize_t>(3)});
-  auto o = out.mutable_unchecked<2>();
-  for (unsigned i = 0; i < n; ++i)
-    for (int k = 0; k < 3; ++k) o(i, k) = a[4ull * i + k];
+  s.GetParticleData().Get(what, out.mutable_data(), s.GetStream(), 3);
   return out;
 }
 

@@ -31,10 +31,8 @@ double sum_energy(Sample* s, const float* f, const char* cls) {
   const hipStream_t st = s->GetStream();
   rumdx_check(rumdx_reduce_f4(f, s->GetNumberOfParticles(), 8u, s->ScalarOut(), s->Workspace(), st), cls,
               "GetPotentialEnergy");
-  double out[4];
-  hip_check(hipMemcpyAsync(out, s->ScalarOut(), sizeof(out), hipMemcpyDeviceToHost, st), cls, "GetPotentialEnergy");
   hip_check(hipStreamSynchronize(st), cls, "GetPotentialEnergy");
-  return out[3];
+  return s->ScalarOut()[3];
 }
 
 }  // namespace

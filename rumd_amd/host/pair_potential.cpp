@@ -325,6 +325,8 @@ void NeighborList::Allocate() {
   }
   allocated_nvp_ = nvp;
   allocated_ = true;
+  flags_changed_ = true;
+  flags_queued_ = false;
   fused_check_pending_ = false;
   InvalidateSortOrder();
   rumdx_check(rumdx_nblist_request_rebuild(&desc_, st), "NeighborList", "Allocate");
@@ -346,7 +348,9 @@ void NeighborList::UpdateNBlist(bool forces_follow) {
   const hipStream_t st = sample_->GetStream();
   if (!fused_check_pending_) rumdx_check(rumdx_nblist_check(p, &desc_, box, st), "NeighborList", "UpdateNBlist");
   fused_check_pending_ = false;
+  flags_changed_ = true;
   if (method == SORT) {
+    sample_->GetParticleData().NoteSorted();
     // skin-triggered rebuilds re-sort tile by tile; the first build, and any
     // after the host changed positions or arrays, sorts from scratch
     const bool resort = UseTileResort() && !force_full_sort_;
@@ -398,15 +402,27 @@ void NeighborList::Settle() {
   }
 }
 
+void NeighborList::QueueFlagsRead() {
+  if (!allocated_ || !flags_changed_ || flags_queued_) return;
+  flags_host_.resize(RUMDX_NB_FLAGS);
+  rumdx_check(rumdx_nblist_read_flags(sample_->GetParticleData().Descriptor(), &desc_, flags_host_.get(),
+                                      sample_->GetStream()),
+              "NeighborList", "UpdateNBlist");
+  flags_queued_ = true;
+}
+
 void NeighborList::ReadFlags(uint32_t* f) {
-  if (desc_.nbl16_dev != nullptr)
-    rumdx_check(rumdx_nblist_build_stats(sample_->GetParticleData().Descriptor(), &desc_, sample_->GetStream()),
-                "NeighborList", "UpdateNBlist");
-  flags_.download(f, RUMDX_NB_FLAGS, sample_->GetStream());
+  if (!flags_queued_) {
+    flags_changed_ = true;
+    QueueFlagsRead();
+    hip_check(hipStreamSynchronize(sample_->GetStream()), "NeighborList", "UpdateNBlist");
+  }
+  flags_queued_ = false;
+  std::memcpy(f, flags_host_.get(), RUMDX_NB_FLAGS * sizeof(uint32_t));
 }
 
 bool NeighborList::HandleOverflow() {
-  if (!allocated_) return false;
+  if (!allocated_ || !flags_changed_) return false;
   uint32_t f[RUMDX_NB_FLAGS];
   ReadFlags(f);
   if (f[RUMDX_FLAG_ERROR]) {
@@ -442,7 +458,10 @@ bool NeighborList::HandleOverflow() {
       if (!f[RUMDX_FLAG_OVERFLOW]) return true;
     }
   }
-  if (!f[RUMDX_FLAG_OVERFLOW]) return false;
+  if (!f[RUMDX_FLAG_OVERFLOW]) {
+    flags_changed_ = false;
+    return false;
+  }
   const unsigned n = sample_->GetNumberOfParticles();
   // the build counts past capacity, so MAXLEN is the true longest list
   unsigned grown = std::min(std::max(max_nbrs_ + max_nbrs_ / 2, f[RUMDX_FLAG_MAXLEN] + f[RUMDX_FLAG_MAXLEN] / 4 + 8), n);
@@ -658,6 +677,7 @@ void PairPotential::ChainStep(rumdx_nh_state* nh_dev, float dt, unsigned thermos
   rumdx_nblist* nb = neighborList.GetResolvedMethod() == NeighborList::NONE ? nullptr : neighborList.Descriptor();
   const float* box = sample->GetSimulationBox()->GetBox8();
   const hipStream_t st = sample->GetStream();
+  neighborList.NoteFlagsChanged();
   if (step == 0 && nb != nullptr)
     rumdx_check(rumdx_nblist_check(pd.Descriptor(), nb, box, st), GetID_String().c_str(), "ChainStep");
   rumdx_check(rumdx_pair_lj_small_step(pd.Descriptor(), nb, d_params_.get(), table_types_, box, cutoff_method_,
@@ -707,11 +727,8 @@ double PairPotential::GetPotentialEnergy() {
   LaunchForce(&p, true, false, st, "GetPotentialEnergy");
   rumdx_check(rumdx_reduce_f4(pe_f_.get(), p.n, 8u, sample->ScalarOut(), sample->Workspace(), st),
               GetID_String().c_str(), "GetPotentialEnergy");
-  double out[4];
-  hip_check(hipMemcpyAsync(out, sample->ScalarOut(), sizeof(out), hipMemcpyDeviceToHost, st), "PairPotential",
-            "GetPotentialEnergy");
   hip_check(hipStreamSynchronize(st), "PairPotential", "GetPotentialEnergy");
-  return out[3];
+  return sample->ScalarOut()[3];
 }
 
 float PairPotential::TimeForceKernel(unsigned reps) {

@@ -25,6 +25,7 @@ void ParticleData::SetNumberOfParticles(unsigned n, unsigned pb, bool mixed_posi
   std::vector<uint32_t> id(nvp_);
   std::iota(id.begin(), id.end(), 0u);
   d_unsorted_index.upload(id.data(), nvp_, nullptr);
+  sorted_ = false;
   types_.assign(n_, 0);
   if (masses_.empty()) masses_.assign(1, 1.f);
   // v.w = 1/m must be valid before the first step
@@ -89,15 +90,14 @@ std::vector<uint32_t> ParticleData::UnsortedIndex(hipStream_t st) {
 }
 
 std::vector<float> ParticleData::GatherToSlots(const float* orig4, hipStream_t st) {
-  const std::vector<uint32_t> idx = UnsortedIndex(st);
   std::vector<float> slot(4ull * nvp_, 0.f);
+  if (!sorted_) {
+    std::memcpy(slot.data(), orig4, 4ull * n_ * sizeof(float));
+    return slot;
+  }
+  const std::vector<uint32_t> idx = UnsortedIndex(st);
   for (unsigned s = 0; s < n_; ++s) std::memcpy(&slot[4ull * s], orig4 + 4ull * idx[s], 4 * sizeof(float));
   return slot;
-}
-
-void ParticleData::Scatter(const std::vector<float>& slot4, float* out4, hipStream_t st) {
-  const std::vector<uint32_t> idx = UnsortedIndex(st);
-  for (unsigned s = 0; s < n_; ++s) std::memcpy(out4 + 4ull * idx[s], &slot4[4ull * s], 4 * sizeof(float));
 }
 
 void ParticleData::SetPositions(const float* xyz, hipStream_t st) {
@@ -185,7 +185,7 @@ void ParticleData::SetForces(const float* f4, hipStream_t st) {
   d_f.upload(slot.data(), slot.size(), st);
 }
 
-void ParticleData::Get(const char* what, float* out4, hipStream_t st) {
+void ParticleData::Get(const char* what, float* out, hipStream_t st, unsigned ncomp) {
   const DeviceArray<float>* a = nullptr;
   const std::string w(what);
   if (w == "r") a = &d_r;
@@ -196,9 +196,7 @@ void ParticleData::Get(const char* what, float* out4, hipStream_t st) {
   else if (w == "sts") a = &d_sts;
   else if (w == "rlo") a = mixed_ ? &d_rlo : nullptr;
   if (a == nullptr) throw RUMD_Error("ParticleData", "Get", "unknown array " + w);
-  std::vector<float> slot(4ull * nvp_);
-  a->download(slot.data(), slot.size(), st);
-  Scatter(slot, out4, st);
+  reader_.Read(a->get(), sorted_ ? d_unsorted_index.get() : nullptr, n_, ncomp, out, st);
 }
 
 void ParticleData::GetTypes(int32_t* out, hipStream_t) { std::copy(types_.begin(), types_.end(), out); }
@@ -218,6 +216,7 @@ void ParticleData::ResetSorting(hipStream_t st) {
   std::vector<uint32_t> id(nvp_);
   std::iota(id.begin(), id.end(), 0u);
   d_unsorted_index.upload(id.data(), nvp_, st);
+  sorted_ = false;
   auto put = [&](DeviceArray<float>& d, std::vector<float>& h) {
     h.resize(4ull * nvp_, 0.f);
     d.upload(h.data(), h.size(), st);

@@ -207,6 +207,7 @@ void ReplicaBatch::RestoreState() {
   copy_device(idx_, save_idx_, stream_);
   copy_device(nh_, save_nh_, stream_);
   copy_device(flags_, save_flags_, stream_);
+  flags_changed_ = true;
   rumdx_check(rumdx_batch_request_rebuild(&desc_, stream_), "ReplicaBatch", "RestoreState");
   hip_check(hipStreamSynchronize(stream_), "ReplicaBatch", "RestoreState");
 }
@@ -251,6 +252,7 @@ rumdx_replica ReplicaBatch::HostReplica(unsigned r) const {
 // (the state Relayout read back, or the configurations AddReplica was given).
 // Thermostat states restart at Ps = 0.
 void ReplicaBatch::Allocate() {
+  flags_changed_ = true;
   if (reps_.empty()) throw RUMD_Error("ReplicaBatch", "Allocate", "no replicas");
   if (table_.empty()) throw RUMD_Error("ReplicaBatch", "Allocate", "no potential set");
   const unsigned nrep = static_cast<unsigned>(reps_.size());
@@ -415,6 +417,7 @@ void ReplicaBatch::Allocate() {
 }
 
 void ReplicaBatch::CalcF() {
+  flags_changed_ = true;
   if (!allocated_) Allocate();
   rumdx_check(rumdx_batch_update_lists(&desc_, stream_), "ReplicaBatch", "CalcF");
   rumdx_check(rumdx_batch_forces(&desc_, params_.get(), cutoff_method_, stream_), "ReplicaBatch", "CalcF");
@@ -433,6 +436,7 @@ void ReplicaBatch::Step() {
 }
 
 float ReplicaBatch::TimeForceKernel(unsigned reps) {
+  flags_changed_ = true;
   if (!allocated_) Allocate();
   if (reps == 0) reps = 1;
   rumdx_check(rumdx_batch_update_lists(&desc_, stream_), "ReplicaBatch", "TimeForceKernel");
@@ -473,6 +477,7 @@ void ReplicaBatch::InvalidateGraphs() {
 }
 
 void ReplicaBatch::RunSteps(unsigned nsteps, unsigned block) {
+  flags_changed_ = true;
   if (!allocated_) Allocate();
   if (block == 0) block = 1;
   unsigned done = 0;
@@ -509,7 +514,7 @@ void ReplicaBatch::RunSteps(unsigned nsteps, unsigned block) {
 // force kernel rescans the stencil for an overflowed list) and rebuilds all.
 void ReplicaBatch::Synchronize() {
   hip_check(hipStreamSynchronize(stream_), "ReplicaBatch", "Synchronize");
-  if (!allocated_) return;
+  if (!allocated_ || !flags_changed_) return;
   std::vector<uint32_t> fl(static_cast<size_t>(RUMDX_BATCH_FLAGS) * reps_.size());
   flags_.download(fl.data(), fl.size(), stream_);
   uint32_t longest = 0;
@@ -518,7 +523,10 @@ void ReplicaBatch::Synchronize() {
     overflow = overflow || fl[RUMDX_BATCH_FLAGS * r + 1] != 0u;
     longest = std::max(longest, fl[RUMDX_BATCH_FLAGS * r + 3]);
   }
-  if (!overflow) return;
+  if (!overflow) {
+    flags_changed_ = false;
+    return;
+  }
   unsigned max_n = 0;
   for (const Spec& s : reps_) max_n = std::max(max_n, static_cast<unsigned>(s.types.size()));
   max_nbrs_ = std::min(std::max(max_nbrs_ + max_nbrs_ / 2, longest + longest / 4 + 8), max_n);
@@ -551,15 +559,8 @@ std::vector<float> ReplicaBatch::Slots(const DeviceArray<float>& a, unsigned rep
   if (replica >= reps_.size()) throw RUMD_Error("ReplicaBatch", "Get", "replica index out of range");
   Synchronize();
   const unsigned n = GetNumberOfParticles(replica);
-  std::vector<float> all(4ull * n);
-  hip_check(hipMemcpyAsync(all.data(), a.get() + 4ull * slot0_[replica], all.size() * sizeof(float),
-                           hipMemcpyDeviceToHost, stream_),
-            "ReplicaBatch", "Get");
-  hip_check(hipStreamSynchronize(stream_), "ReplicaBatch", "Get");
-  const std::vector<uint32_t> id = SlotIds(replica);
   std::vector<float> out(static_cast<size_t>(comps) * n);
-  for (unsigned s = 0; s < n; ++s)
-    for (unsigned c = 0; c < comps; ++c) out[static_cast<size_t>(comps) * id[s] + c] = all[4ull * s + c];
+  reader_.Read(a.get() + 4ull * slot0_[replica], idx_.get() + slot0_[replica], n, comps, out.data(), stream_);
   return out;
 }
 

@@ -115,6 +115,8 @@ class ReplicaBatch {
   float skin_ = 0.3f, max_cutoff_ = 0.f, dt_ = 0.0025f;
   unsigned user_max_nbrs_ = 0, max_nbrs_ = 0, lanes_per_particle_ = 1;
   bool saved_ = false;
+  bool flags_changed_ = true;  // work that may change the flags was launched since they were read
+  OriginalOrderReader reader_;
   bool allocated_ = false;
   bool staged_forces_ = true;
   bool workgroup_sort_ = true;

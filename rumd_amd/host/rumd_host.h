@@ -73,6 +73,44 @@ class DeviceArray {
   size_t n_ = 0;
 };
 
+// Owned pinned host memory that kernels write directly: results a host read
+// waits for arrive with the stream's synchronisation, without a copy of their
+// own.
+template <class T>
+class PinnedArray {
+ public:
+  PinnedArray() = default;
+  ~PinnedArray() { release(); }
+  PinnedArray(const PinnedArray&) = delete;
+  PinnedArray& operator=(const PinnedArray&) = delete;
+  void resize(size_t n);
+  void release();
+  T* get() const { return ptr_; }
+  size_t size() const { return n_; }
+
+ private:
+  T* ptr_ = nullptr;
+  size_t n_ = 0;
+};
+
+// Reads device float4 arrays into host memory in original particle order: a
+// kernel gathers and packs the wanted components into pinned memory, at most
+// two chunks of kChunk floats (4 MiB in all), the next one filling while the
+// host copies the last.
+class OriginalOrderReader {
+ public:
+  ~OriginalOrderReader();
+  // unsorted_index: the slots' original ids (n of them), or null when the
+  // slots are in original order.
+  void Read(const float* arr4, const uint32_t* unsorted_index, unsigned n, unsigned ncomp, float* out, hipStream_t st);
+
+ private:
+  static constexpr size_t kChunk = 1u << 19;
+  PinnedArray<float> stage_;
+  DeviceArray<uint32_t> slot_of_;
+  hipEvent_t done_[2] = {nullptr, nullptr};
+};
+
 // ------------------------------------------------------------------ Device
 // Device singleton (src/Device.cu:143-222): name, memory, sync, timing.
 class Device {
@@ -183,6 +221,11 @@ class NeighborList {
   // forces_follow the caller initialises forces and virials next, so a rebuild
   // need not move them.
   void UpdateNBlist(bool forces_follow = false);
+  // Work that may change the flags has been launched since they were read.
+  void NoteFlagsChanged() { flags_changed_ = true; }
+  // Queues the read of the flags for the next HandleOverflow (before the
+  // stream is synchronised); nothing when they cannot have changed.
+  void QueueFlagsRead();
   // Allocates buffers now (before a graph capture, which may not allocate).
   void EnsureAllocated();
   // Called after an integrator step that ran this list's skin check fused.
@@ -195,7 +238,8 @@ class NeighborList {
   void InvalidateSortOrder();
   // Every sorted rebuild sorts from scratch while set (for timing the two paths).
   void SetForceFullSort(bool on) { force_full_sort_ = on; }
-  // Reads the flags; grows the list after an overflow.  Synchronises.
+  // Acts on the flags (grows the list after an overflow).  Synchronises unless
+  // they were queued or cannot have changed since the last call.
   bool HandleOverflow();
   // Asks the next UpdateNBlist to rebuild (device flag, on the sample's stream).
   void RequestRebuild();
@@ -226,8 +270,11 @@ class NeighborList {
   rumdx_nblist* Descriptor() { return &desc_; }
 
  private:
-  // Downloads the flags after gathering the last sorted build's statistics.
+  // The flags after gathering the last sorted build's statistics.  Synchronises.
   void ReadFlags(uint32_t* f);
+  bool flags_changed_ = true;  // since the last HandleOverflow
+  bool flags_queued_ = false;  // flags_host_ holds them at the next synchronisation
+  PinnedArray<uint32_t> flags_host_;
   void Allocate();
   void Settle();
   void Prune();
@@ -810,7 +857,10 @@ class ParticleData {
   void SetVelocities(const float* xyz, hipStream_t st);
   void SetImages(const float* xyz, hipStream_t st);
   void SetForces(const float* f4, hipStream_t st);
-  void Get(const char* what, float* out4, hipStream_t st);  // "r","v","f","w","im","sts": n x 4, original order
+  // "r", "v", "f", "w", "im", "sts" or "rlo": n x ncomp, original order
+  void Get(const char* what, float* out, hipStream_t st, unsigned ncomp = 4);
+  // The slots may be in another order than the particles' from now on.
+  void NoteSorted() { sorted_ = true; }
   void GetTypes(int32_t* out, hipStream_t st);
   void ResetSorting(hipStream_t st);
   rumdx_particles* Descriptor() { return &desc_; }
@@ -831,10 +881,11 @@ class ParticleData {
 
  private:
   void UpdateMassesOnDevice(hipStream_t st);
-  void Scatter(const std::vector<float>& slot4, float* out4, hipStream_t st);
   std::vector<float> GatherToSlots(const float* orig4, hipStream_t st);
   unsigned n_ = 0, nvp_ = 0;
   bool mixed_ = false;
+  bool sorted_ = false;  // false: slot order is the original order
+  OriginalOrderReader reader_;
   std::vector<float> masses_;
   std::vector<int32_t> types_;  // original order
   rumdx_particles desc_{};
@@ -945,7 +996,7 @@ class Sample {
   ParticleData pd_;
   hipStream_t stream_ = nullptr;
   DeviceArray<char> workspace_;
-  DeviceArray<double> scalars_;
+  PinnedArray<double> scalars_;  // results of the FP64 sums, read after a synchronisation
   // captured step blocks: key = (block size, momentum reset at first step)
   std::map<std::pair<unsigned, bool>, Block> graphs_;
   bool fused_steps_ = true;

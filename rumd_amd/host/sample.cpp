@@ -12,7 +12,7 @@ constexpr unsigned kPbThreshold = 10000;  // src/Sample.cu:36-39
 Sample::Sample(unsigned pb, unsigned tp) : pb_(pb), tp_(tp) {
   Device::GetDevice().Init();
   hip_check(hipStreamCreate(&stream_), "Sample", "Sample");
-  scalars_.resize(8);
+  scalars_.resize(16);
 }
 
 Sample::~Sample() {
@@ -148,6 +148,9 @@ void Sample::CalcF(bool calc_stresses) {
 }
 
 void Sample::Synchronize() {
+  // the lists' flags come back with this synchronisation
+  for (Potential* p : potentials_)
+    if (auto* pp = dynamic_cast<PairPotential*>(p)) pp->GetNeighborList().QueueFlagsRead();
   hip_check(hipStreamSynchronize(stream_), "Sample", "Synchronize");
   for (Potential* p : potentials_)
     if (auto* pp = dynamic_cast<PairPotential*>(p))
@@ -160,9 +163,8 @@ double Sample::GetPotentialEnergy() {
   Synchronize();
   rumdx_check(rumdx_reduce_f4(pd_.d_f.get(), GetNumberOfParticles(), 8u, scalars_.get(), workspace_.get(), stream_),
               "Sample", "GetPotentialEnergy");
-  double out[4];
-  scalars_.download(out, 4, stream_);
-  double pe = out[3];
+  hip_check(hipStreamSynchronize(stream_), "Sample", "GetPotentialEnergy");
+  double pe = scalars_.get()[3];
   for (Potential* p : potentials_)
     if (!p->EnergyIncludedInParticleSum()) pe += p->GetPotentialEnergy();
   return pe;
@@ -172,9 +174,8 @@ double Sample::GetVirial() {
   Synchronize();
   rumdx_check(rumdx_reduce_f4(pd_.d_w.get(), GetNumberOfParticles(), 8u, scalars_.get(), workspace_.get(), stream_),
               "Sample", "GetVirial");
-  double out[4];
-  scalars_.download(out, 4, stream_);
-  double w = out[3] / 6.0;
+  hip_check(hipStreamSynchronize(stream_), "Sample", "GetVirial");
+  double w = scalars_.get()[3] / 6.0;
   for (Potential* p : potentials_)
     if (!p->EnergyIncludedInParticleSum()) w += p->GetVirial();
   return w;
@@ -184,27 +185,15 @@ double Sample::GetVirial() {
 std::vector<double> Sample::GetStress() {
   Synchronize();
   const unsigned n = GetNumberOfParticles();
-  double s[6] = {0, 0, 0, 0, 0, 0};
-  double out[4];
-  rumdx_check(rumdx_reduce_f4(pd_.d_sts.get(), n, 15u, scalars_.get(), workspace_.get(), stream_), "Sample", "GetStress");
-  scalars_.download(out, 4, stream_);
-  for (int k = 0; k < 4; ++k) s[k] = out[k];
-  rumdx_check(rumdx_reduce_f4(pd_.d_w.get(), n, 6u, scalars_.get(), workspace_.get(), stream_), "Sample", "GetStress");
-  scalars_.download(out, 4, stream_);
-  s[4] = out[1];
-  s[5] = out[2];
-  std::vector<float> v(4ull * n);
-  pd_.Get("v", v.data(), stream_);
-  for (unsigned i = 0; i < n; ++i) {
-    const float m2 = 2.f / v[4ull * i + 3];
-    const float vx = v[4ull * i], vy = v[4ull * i + 1], vz = v[4ull * i + 2];
-    s[0] -= m2 * vx * vx;
-    s[1] -= m2 * vy * vy;
-    s[2] -= m2 * vz * vz;
-    s[3] -= m2 * vy * vz;
-    s[4] -= m2 * vx * vz;
-    s[5] -= m2 * vx * vy;
-  }
+  double* out = scalars_.get();
+  // configurational sums: sts, then w.y and w.z; kinetic sums (all six)
+  rumdx_check(rumdx_reduce_f4(pd_.d_sts.get(), n, 15u, out, workspace_.get(), stream_), "Sample", "GetStress");
+  rumdx_check(rumdx_reduce_f4(pd_.d_w.get(), n, 6u, out + 4, workspace_.get(), stream_), "Sample", "GetStress");
+  rumdx_check(rumdx_kinetic_stress(pd_.Descriptor(), out + 8, workspace_.get(), stream_), "Sample", "GetStress");
+  hip_check(hipStreamSynchronize(stream_), "Sample", "GetStress");
+  const double conf[6] = {out[0], out[1], out[2], out[3], out[5], out[6]};
+  double s[6];
+  for (int k = 0; k < 6; ++k) s[k] = conf[k] - out[8 + k];
   const double V = box_->GetVolume();
   std::vector<double> r(6);
   for (int k = 0; k < 6; ++k) r[k] = 0.5 * s[k] / V;
@@ -368,6 +357,8 @@ void Sample::RunSteps(unsigned long first_step, unsigned nsteps, unsigned block,
     if (NeighborList* nl = FusedCheckList()) nl->ResetFusedCheck();
     pd_.MovePositionsTo(it->second.r_home, stream_);
     hip_check(hipGraphLaunch(it->second.exec, stream_), "Sample", "RunSteps");
+    for (Potential* p : potentials_)
+      if (auto* pp = dynamic_cast<PairPotential*>(p)) pp->GetNeighborList().NoteFlagsChanged();
     if (NeighborList* nl = FusedCheckList()) nl->NoteFusedCheck();
   }
   Synchronize();
