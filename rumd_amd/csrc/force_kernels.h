@@ -173,15 +173,23 @@ __device__ __forceinline__ void combine_lanes(Acc& a, uint32_t lg) {
 }
 
 // The pairs of particle i's N2 list (u32 slots, column-major) that fall to
-// lane `part` of the 2^lgp sharing it: entries part, part + 2^lgp, ...  An
+// lane `part` of the 2^lgp sharing it: entries part, part + 2^lgp, ..., four at
+// a time with their reads in flight together.  A list of at most kShortList
+// entries is one such round of four lanes already, and takes no more.  An
 // overflowed list takes all pairs, shared alike.
+constexpr uint32_t kShortList = 32, kShortLg = 2;
+
 template <bool STR, class PP>
 __device__ __forceinline__ void list_forces(const PP& pp, uint32_t i, uint32_t part, uint32_t lgp, double xi, double yi,
                                             double zi, const float4* __restrict__ r, const uint32_t* nbl, uint32_t nn,
                                             uint32_t n, uint32_t nvp, uint32_t max_nbrs, const float4* prow,
                                             const Box& bx, const Exclusions& ex, Acc& a) {
-  const uint32_t step = 1u << lgp;
   if (nn < max_nbrs) {
+    if (nn <= kShortList && lgp > kShortLg) {
+      if (part >= (1u << kShortLg)) return;
+      lgp = kShortLg;
+    }
+    const uint32_t step = 1u << lgp;
     const size_t stride = static_cast<size_t>(nvp) << lgp;
     const uint32_t* col = nbl + static_cast<size_t>(part) * nvp + i;
     uint32_t k = part;
@@ -194,14 +202,17 @@ __device__ __forceinline__ void list_forces(const PP& pp, uint32_t i, uint32_t p
       pair_term<STR>(pp, xi, yi, zi, r2, prow, bx, a);
       pair_term<STR>(pp, xi, yi, zi, r3, prow, bx, a);
     }
-    for (; k < nn; k += step) {
-      const uint32_t j = *col;
-      col += stride;
-      pair_term<STR>(pp, xi, yi, zi, r[j], prow, bx, a);
+    if (k < nn) {  // up to three more, past the list standing in for the first
+      const bool two = k + step < nn, three = k + 2 * step < nn;
+      const uint32_t j0 = col[0], j1 = col[two ? stride : 0], j2 = col[three ? 2 * stride : 0];
+      const float4 r0 = r[j0], r1 = r[j1], r2 = r[j2];
+      pair_term<STR>(pp, xi, yi, zi, r0, prow, bx, a);
+      if (two) pair_term<STR>(pp, xi, yi, zi, r1, prow, bx, a);
+      if (three) pair_term<STR>(pp, xi, yi, zi, r2, prow, bx, a);
     }
   } else {
     const ExclusionRange er = ex.of(i);
-    for (uint32_t j = part; j < n; j += step)
+    for (uint32_t j = part; j < n; j += 1u << lgp)
       if (j != i && !ex.excludes(er, j)) pair_term<STR>(pp, xi, yi, zi, r[j], prow, bx, a);
   }
 }
