@@ -638,6 +638,11 @@ typedef struct rumdx_batch {
  * counterpart in the reference. */
 int rumdx_batch_forces_nvt(rumdx_batch* b, const float* params_dev, int cutoff_method, float dt,
                            void* workspace_dev, void* stream);
+/* The same step without potential energies and virials (f.w and w are left
+ * unspecified): for a step that another one follows before anything reads
+ * them.  Positions, velocities and thermostats come out as the same bits. */
+int rumdx_batch_forces_nvt_inner(rumdx_batch* b, const float* params_dev, int cutoff_method, float dt,
+                                 void* workspace_dev, void* stream);
 /* Bytes of device workspace rumdx_batch_nvt_step / rumdx_batch_energies need. */
 size_t rumdx_batch_workspace_bytes(uint32_t nslots);
 /* Marks every replica's list stale. */

@@ -575,56 +575,65 @@ __global__ __launch_bounds__(kBlock) void k_b_build(BatchArgs a, const uint32_t*
 }
 
 // ------------------------------------------------------------------ forces
-// FP32 pair arithmetic with the minimum-image displacement taken exactly on
-// the fixed-point positions (to_fixed above) and rounded once to FP32.
+// Pair terms on the fixed-point positions (to_fixed above).  The wrapping
+// difference of two coordinates is the minimum image, exactly, in units of
+// L 2^-32, and exact in FP64 too.  The squared distance is summed there and
+// rounded to FP32 once, in simulation units; the term of the force over the
+// displacement is FP32 arithmetic, and a particle's force is summed over the
+// integer displacements in FP64 and scaled once by L 2^-32 (an FP32 number).
+// FP64 instructions issue at FP32's rate here and the kernels are bound by VALU
+// issue, so what counts is their number: scaling and rounding each displacement
+// first takes nine conversions and products per pair, this six fewer.
 struct Acc {
-  float fx = 0.f, fy = 0.f, fz = 0.f, u = 0.f, vir = 0.f;
+  double fx = 0.0, fy = 0.0, fz = 0.0;
+  float u = 0.f, vir = 0.f;
 };
 
-// One axis of the displacement: the wrapping difference of the fixed-point
-// coordinates (the minimum image, exactly) scaled by L 2^-32 in FP64 (exact:
-// a 32-bit integer times a float over a power of two) and rounded once to FP32,
-// so the displacement is the correctly rounded one.
-__device__ __forceinline__ float fixed_delta(int32_t a, int32_t b, double unit) {
-  return static_cast<float>(
-      static_cast<double>(static_cast<int32_t>(static_cast<uint32_t>(a) - static_cast<uint32_t>(b))) * unit);
+// One pair.  Without `live` it adds nothing (a list's padding).  1/r^2 is
+// refined by one Newton step: the r^-14 term multiplies its error by seven.
+// Median error against FP64 over the sum of |f_ij|, 56 replicas of 261 to
+// 6,000 particles: 1.96e-7 (2.43e-7 with rounded displacements and an unrefined
+// reciprocal).
+__device__ __forceinline__ double fixed_diff(int32_t a, int32_t b) {
+  return static_cast<double>(static_cast<int32_t>(static_cast<uint32_t>(a) - static_cast<uint32_t>(b)));
 }
-
-template <int CUT>
-__device__ __forceinline__ void pair_b(int4 fi, int4 fj, double unit, const float4* prow, Acc& a) {
-  const float dx = fixed_delta(fi.x, fj.x, unit);
-  const float dy = fixed_delta(fi.y, fj.y, unit);
-  const float dz = fixed_delta(fi.z, fj.z, unit);
-  const float d2 = dx * dx + dy * dy + dz * dz;
+template <int CUT, bool ENERGY>
+__device__ __forceinline__ void pair_b(int4 fi, int4 fj, double unit2, const float4* prow, bool live, Acc& a) {
+  const double dx = fixed_diff(fi.x, fj.x), dy = fixed_diff(fi.y, fj.y), dz = fixed_diff(fi.z, fj.z);
+  const float d2 = static_cast<float>((dx * dx + dy * dy + dz * dz) * unit2);
   const float4 pa = prow[2 * fj.w];
-  const float4 pb = prow[2 * fj.w + 1];
-  // 1/r^2 from its own reciprocal (1 ulp) rather than the square of 1/r
-  // (2.5 ulp): the r^-14 force term multiplies that error by seven.  The
-  // batch kernel waits on gathers more than on VALU, so the second
-  // transcendental costs little here.
-  float rinv = 0.f;
-  const float inv2 = __builtin_amdgcn_rcpf(d2);
-  if (CUT == RUMDX_CUTOFF_SF) rinv = __builtin_amdgcn_rsqf(d2);
-  const float inv6 = inv2 * inv2 * inv2;
-  float s = (inv6 * inv2) * fmaf(pb.x, inv6, pb.y);
-  float u;
-  if (CUT == RUMDX_CUTOFF_SP) {
-    u = fmaf(inv6, fmaf(pa.y, inv6, pa.z), pb.z);
-  } else if (CUT == RUMDX_CUTOFF_SF) {
-    u = fmaf(inv6, fmaf(pa.y, inv6, pa.z), pb.w);
-    s = fmaf(-pa.w, rinv, s);
-    u = fmaf(pa.w, d2 * rinv, u);
+  float rinv = 0.f, inv2;
+  if (CUT == RUMDX_CUTOFF_SF) {
+    rinv = __builtin_amdgcn_rsqf(d2);
+    inv2 = rinv * rinv;
+    inv2 = fmaf(inv2, fmaf(-d2, inv2, 1.f), inv2);
   } else {
-    u = inv6 * fmaf(pa.y, inv6, pa.z);
+    inv2 = __builtin_amdgcn_rcpf(d2);
+    inv2 = d2 > 0.f ? fmaf(inv2, fmaf(-d2, inv2, 1.f), inv2) : inv2;  // coincident particles stay infinite
   }
-  const bool in = d2 < pa.x;
+  const float inv6 = inv2 * inv2 * inv2;
+  float s = (inv6 * inv2) * fmaf(pa.y, inv6, pa.z);
+  if (CUT == RUMDX_CUTOFF_SF) s = fmaf(-pa.w, rinv, s);
+  const bool in = live && d2 < pa.x;
   s = in ? s : 0.f;
-  u = in ? u : 0.f;
-  a.fx += dx * s;
-  a.fy += dy * s;
-  a.fz += dz * s;
-  a.u += u;
-  a.vir += d2 * s;
+  const double sd = s;
+  a.fx += dx * sd;
+  a.fy += dy * sd;
+  a.fz += dz * sd;
+  if (ENERGY) {
+    const float4 pb = prow[2 * fj.w + 1];
+    float u;
+    if (CUT == RUMDX_CUTOFF_SP) {
+      u = fmaf(inv6, fmaf(pb.x, inv6, pb.y), pb.z);
+    } else if (CUT == RUMDX_CUTOFF_SF) {
+      u = fmaf(inv6, fmaf(pb.x, inv6, pb.y), pb.w);
+      u = fmaf(pa.w, d2 * rinv, u);
+    } else {
+      u = inv6 * fmaf(pb.x, inv6, pb.y);
+    }
+    a.u += in ? u : 0.f;
+    a.vir += d2 * s;
+  }
 }
 
 struct CellArrays {
@@ -633,17 +642,21 @@ struct CellArrays {
   const uint32_t* cell_n;
 };
 
-// The LDS table of the LJ pair term: per type pair {rc^2, A12, A6, s(rc) rc}
-// and {12 A12, 6 A6, -u(rc), -(u(rc) + s(rc) rc^2)}.
+// The LDS table of the LJ pair term: per type pair {rc^2, 12 A12, 6 A6,
+// s(rc) rc}, all that a force needs, and {A12, A6, -u(rc), -(u(rc) + s(rc)
+// rc^2)}.
 __device__ __forceinline__ void load_lj_table(float4* s_tab, const float* __restrict__ params, uint32_t nt) {
   for (uint32_t k = threadIdx.x; k < nt * nt; k += blockDim.x) {
     const float* q = params + static_cast<size_t>(k) * RUMDX_NUM_PARAM;
     const float rc = q[0], a12 = q[1], a6 = q[2];
     const float src = q[RUMDX_NUM_PARAM - 2], ucut = q[RUMDX_NUM_PARAM - 1];
-    s_tab[2 * k] = make_float4(rc * rc, a12, a6, src);
-    s_tab[2 * k + 1] = make_float4(12.f * a12, 6.f * a6, -ucut, -fmaf(src, rc, ucut));
+    s_tab[2 * k] = make_float4(rc * rc, 12.f * a12, 6.f * a6, src);
+    s_tab[2 * k + 1] = make_float4(a12, a6, -ucut, -fmaf(src, rc, ucut));
   }
 }
+
+// A replica's fixed-point unit, L 2^-32 (exact: a power of two times L).
+__device__ __forceinline__ float fixed_unit(const rumdx_replica& rp) { return rp.L * 2.3283064365386963e-10f; }
 
 // Neighbour positions read from the batch's fixed-point array.
 struct GlobalFixed {
@@ -651,23 +664,31 @@ struct GlobalFixed {
   __device__ __forceinline__ int4 operator()(uint32_t j) const { return fixed[j]; }
 };
 
-// Neighbour positions read from a replica staged in LDS (slot j at s[j - slot0]).
+// Neighbour positions read from a replica staged in LDS: slot j at byte 16 j +
+// base of the workgroup's LDS (base may wrap), one address instruction.
 struct StagedFixed {
-  const int4* s;
-  uint32_t slot0;
-  __device__ __forceinline__ int4 operator()(uint32_t j) const { return s[j - slot0]; }
+  using LdsInt4 = __attribute__((address_space(3))) const int4;
+  uint32_t base;
+  __device__ __forceinline__ StagedFixed(const int4* s, uint32_t slot0)
+      : base(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((LdsInt4*)s)) - 16u * slot0) {}
+  __device__ __forceinline__ int4 operator()(uint32_t j) const {
+    LdsInt4* p = reinterpret_cast<LdsInt4*>(static_cast<uintptr_t>(16u * j + base));
+    return make_int4(p->x, p->y, p->z, p->w);
+  }
 };
 
 // One lane's share of slot i's pair terms: entries part, part + 2^lgp, ... of
-// its list, four loads in flight, positions through `pos`.  An overflowed
-// list rescans the build-time stencil (from global memory) in its first lane.
-template <int CUT, class Pos>
+// its list in order through `pos`, eight at a time and the last up to seven by
+// fours.  Entries past the list's end stand for slot i itself and add nothing,
+// so the end of a list waits for memory once or twice, not once per entry.  An
+// overflowed list rescans the build-time stencil in its first lane.
+template <int CUT, bool ENERGY, class Pos>
 __device__ __forceinline__ void slot_terms(const BatchArgs& a, const rumdx_replica& rp, uint32_t i, int4 fi,
                                            uint32_t part, uint32_t lgp, const uint32_t* __restrict__ nbl,
                                            const uint32_t* __restrict__ num_nbrs, uint32_t max_nbrs,
                                            const CellArrays& cells, const float4* prow, const Pos& pos, Acc& acc) {
   const uint32_t step = 1u << lgp;
-  const double unit = static_cast<double>(rp.L) * 2.3283064365386963e-10;  // L 2^-32, exact
+  const double unit2 = static_cast<double>(fixed_unit(rp)) * static_cast<double>(fixed_unit(rp));  // exact
   const uint32_t nn = num_nbrs[i];
   if (nn >= max_nbrs) {
     if (part == 0) {
@@ -684,46 +705,69 @@ __device__ __forceinline__ void slot_terms(const BatchArgs& a, const rumdx_repli
                                                                 nc * ((cy + dy + nc) % nc + nc * ((cz + dz + nc) % nc)));
             const uint32_t b0 = cells.cell_start[c], m = cells.cell_n[c];
             for (uint32_t j = b0; j < b0 + m; ++j)
-              if (j != i) pair_b<CUT>(fi, a.fixed[j], unit, prow, acc);
+              if (j != i) pair_b<CUT, ENERGY>(fi, pos(j), unit2, prow, true, acc);
           }
     }
     return;
   }
-  // eight list entries (and their positions) in flight per pass: the list
-  // reads come from HBM, and fewer waves than that would leave their latency
-  // exposed at one staged workgroup per CU
   const size_t stride = static_cast<size_t>(a.nslots) << lgp;
   const uint32_t* col = nbl + static_cast<size_t>(part) * a.nslots + i;
   uint32_t k = part;
-  for (; k + 7 * step < nn; k += 8 * step) {
-    uint32_t j[8];
+  uint32_t j[8];
+  if (k + 7 * step < nn) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) j[u] = col[u * stride];
-    col += 8 * stride;
+  }
+  for (; k + 7 * step < nn; k += 8 * step) {
     int4 fj[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) fj[u] = pos(j[u]);
+    col += 8 * stride;
+    if (k + 15 * step < nn) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) pair_b<CUT>(fi, fj[u], unit, prow, acc);
+      for (int u = 0; u < 8; ++u) j[u] = col[u * stride];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) pair_b<CUT, ENERGY>(fi, fj[u], unit2, prow, true, acc);
   }
-  for (; k < nn; k += step, col += stride) pair_b<CUT>(fi, pos(*col), unit, prow, acc);
+  for (; k < nn; k += 4 * step) {
+    uint32_t j[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) j[u] = k + u * step < nn ? col[u * stride] : i;
+    col += 4 * stride;
+    int4 fj[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) fj[u] = pos(j[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) pair_b<CUT, ENERGY>(fi, fj[u], unit2, prow, k + u * step < nn, acc);
+  }
 }
 
-// Sums the 2^lgp lanes of each slot (a fixed butterfly); every lane of the
-// wave takes part.
-__device__ __forceinline__ void combine_slot_lanes(Acc& acc, uint32_t lgp) {
+// A slot's sums over its 2^lgp lanes (a fixed butterfly), the forces scaled to
+// simulation units; every lane of the wave takes part.
+struct SlotSum {
+  float fx, fy, fz, u, vir;
+};
+template <bool ENERGY>
+__device__ __forceinline__ SlotSum combine_slot_lanes(const Acc& acc, uint32_t lgp, float unit) {
+  SlotSum t{static_cast<float>(acc.fx * unit), static_cast<float>(acc.fy * unit), static_cast<float>(acc.fz * unit),
+            acc.u, acc.vir};
   for (uint32_t o = 1; o < (1u << lgp); o <<= 1) {
-    acc.fx += __shfl_xor(acc.fx, o, 64);
-    acc.fy += __shfl_xor(acc.fy, o, 64);
-    acc.fz += __shfl_xor(acc.fz, o, 64);
-    acc.u += __shfl_xor(acc.u, o, 64);
-    acc.vir += __shfl_xor(acc.vir, o, 64);
+    t.fx += __shfl_xor(t.fx, o, 64);
+    t.fy += __shfl_xor(t.fy, o, 64);
+    t.fz += __shfl_xor(t.fz, o, 64);
+    if (ENERGY) {
+      t.u += __shfl_xor(t.u, o, 64);
+      t.vir += __shfl_xor(t.vir, o, 64);
+    }
   }
+  return t;
 }
 
-__device__ __forceinline__ void store_slot(const BatchArgs& a, uint32_t i, const Acc& acc) {
-  a.f[i] = make_float4(acc.fx, acc.fy, acc.fz, 0.5f * acc.u);
-  a.w[i] = make_float4(0.f, 0.f, 0.f, acc.vir);
+template <bool ENERGY>
+__device__ __forceinline__ void store_slot(const BatchArgs& a, uint32_t i, const SlotSum& t) {
+  a.f[i] = make_float4(t.fx, t.fy, t.fz, 0.5f * t.u);
+  if (ENERGY) a.w[i] = make_float4(0.f, 0.f, 0.f, t.vir);
 }
 
 // One particle's list over 2^lgp lanes (lane part takes entries part,
@@ -736,21 +780,21 @@ __global__ __launch_bounds__(kBlock) void k_b_force(BatchArgs a, const uint32_t*
                                                     CellArrays cells, const float* __restrict__ params,
                                                     uint32_t nt, uint32_t lgp) {
   extern __shared__ float4 s_tab[];
-  load_lj_table(s_tab, params, nt);
-  __syncthreads();
   const uint32_t step = 1u << lgp;
   const uint32_t i = (blockIdx.x * kBlock + threadIdx.x) >> lgp, part = threadIdx.x & (step - 1u);
-  const uint32_t rep = a.block_rep[i / kBlock];
+  const uint32_t rep = a.block_rep[((blockIdx.x * kBlock) >> lgp) / kBlock];  // the workgroup's one replica
   const rumdx_replica rp = a.rep[rep];
+  load_lj_table(s_tab, params, nt);
+  __syncthreads();
   const bool live = i - rp.slot0 < rp.n;
   Acc acc;
   if (live) {
     const int4 fi = a.fixed[i];
-    slot_terms<CUT>(a, rp, i, fi, part, lgp, nbl, num_nbrs, max_nbrs, cells, s_tab + 2 * fi.w * nt,
-                    GlobalFixed{a.fixed}, acc);
+    slot_terms<CUT, true>(a, rp, i, fi, part, lgp, nbl, num_nbrs, max_nbrs, cells, s_tab + 2 * fi.w * nt,
+                          GlobalFixed{a.fixed}, acc);
   }
-  combine_slot_lanes(acc, lgp);
-  if (live && part == 0) store_slot(a, i, acc);
+  const SlotSum t = combine_slot_lanes<true>(acc, lgp, fixed_unit(rp));
+  if (live && part == 0) store_slot<true>(a, i, t);
 }
 
 // The same pair terms with the replica staged: a workgroup takes one work
@@ -759,85 +803,133 @@ __global__ __launch_bounds__(kBlock) void k_b_force(BatchArgs a, const uint32_t*
 // time, reading every neighbour from LDS.  Lane mapping and summation order
 // are those of k_b_force, so the forces are the same bits.
 //
-// With FUSE every work item is a whole replica, and the workgroup then also
-// takes the replica's NVT step (k_b_nvt's per-particle update and its
-// per-256-slot kinetic-energy partials, in the same order): nothing else
-// reads this replica's positions during the launch, so they are updated in
-// place.
+// With kStepStore or kStepInner every work item is a whole replica, and the
+// workgroup also takes the replica's NVT step: k_b_nvt's update of every slot
+// and k_b_nvt_finish's thermostat, the kinetic energy added in the same order
+// (wave sums, 256-slot blocks, then the blocks).  Nothing else reads this
+// replica during the launch and its pair terms read the staged copy, so with
+// one lane per particle a slot is advanced in place as soon as its force is
+// summed and the update's memory traffic overlaps other waves' pair terms;
+// with more lanes the forces go through memory first.  kStepInner leaves
+// forces, energies and virials out, for a step whose forces the next one
+// replaces before anything can read them.
+// VALU issue bounds the pair terms (76 % of cycles measured).  512 replicas of
+// 261 to 8,186 particles (2.15 million), shifted forces: 291 us a step for
+// kStepInner and 315 for kStepStore, the thermostats included; 355 before, as
+// two launches with rounded displacements, energies always computed and the
+// update after all of a replica's pair terms.
 constexpr uint32_t kStagedBlock = 1024;
 static_assert(kStagedBlock <= kMaxWorkgroup, "staged force workgroup");
 static_assert(kStagedBlock % kBlock == 0, "whole integrator blocks per pass");
 
+// A replica's thermostat after a step of summed m v^2 `tot`:
+// Ps += dt omega^2 min(KE2 / (dof T) - 1, 10) in FP64.
+__device__ __forceinline__ void nh_advance_replica(rumdx_nh_state& s, const rumdx_replica& rp, double tot, float dt) {
+  s.ke2_sum = tot;
+  if (rp.omega2 > 0.f) {
+    double dev = tot / (static_cast<double>(rp.dof) * s.target_T) - 1.0;
+    if (dev > 10.0) dev = 10.0;  // runaway clamp (src/IntegratorNVT.cu:432-434)
+    s.ps += static_cast<double>(dt) * static_cast<double>(rp.omega2) * dev;
+    s.target_T += s.dT_per_step;
+  }
+}
+
 struct BatchNvt {
-  const rumdx_nh_state* nh;
+  rumdx_nh_state* nh;
   const float4* last_r;
-  double* partials;  // one per 256-slot block, as k_b_nvt writes them
   float dt;
   float skin2_over_4;
 };
 
-template <int CUT, bool FUSE = false>
+constexpr int kForcesOnly = 0, kStepStore = 1, kStepInner = 2;
+
+template <int CUT, int FUSE>
 __global__ __launch_bounds__(kStagedBlock) void k_b_force_staged(BatchArgs a, const uint32_t* __restrict__ nbl,
                                                                  const uint32_t* __restrict__ num_nbrs,
                                                                  uint32_t max_nbrs, CellArrays cells,
                                                                  const float* __restrict__ params, uint32_t nt,
                                                                  uint32_t lgp, const uint4* __restrict__ work,
                                                                  BatchNvt nv) {
+  constexpr bool ENERGY = FUSE != kStepInner;
   extern __shared__ float4 s_dyn[];
   float4* s_tab = s_dyn;
   int4* s_fix = reinterpret_cast<int4*>(s_dyn + 2 * nt * nt);
-  load_lj_table(s_tab, params, nt);
   const uint4 wk = work[blockIdx.x];
   const rumdx_replica rp = a.rep[wk.x];
+  load_lj_table(s_tab, params, nt);
   for (uint32_t k = threadIdx.x; k < rp.n; k += kStagedBlock) s_fix[k] = a.fixed[rp.slot0 + k];
   __syncthreads();
-  const StagedFixed pos{s_fix, rp.slot0};
+  const StagedFixed pos(s_fix, rp.slot0);
   const uint32_t step = 1u << lgp, part = threadIdx.x & (step - 1u);
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const Box bx = rep_box(rp);
+  const float ps = FUSE != kForcesOnly && rp.omega2 > 0.f ? static_cast<float>(nv.nh[wk.x].ps) : 0.f;
+  const float unit = fixed_unit(rp);
+  // one slot's leapfrog step; every lane of the wave takes part, and lane
+  // `pass` keeps the wave's m v^2
+  double wave_ke = 0.0;
+  const auto advance = [&](uint32_t i, bool live, float4 r, float4 v, float4 last, float4 f, uint32_t pass) {
+    float ke2 = 0.f;
+    if (live) {
+      float4 lo = make_float4(0.f, 0.f, 0.f, 0.f);
+      float3 shift;
+      ke2 = nvt_particle<false>(r, v, f, shift, lo, ps, nv.dt, bx);
+      a.r[i] = r;
+      a.fixed[i] = to_fixed(r, fixed_scale(rp));
+      a.v[i] = v;
+      add_image_shift(a.im, i, shift);
+      if (min_image_d2_f32(r, last, bx) > nv.skin2_over_4) a.flags[kRepFlags * wk.x + kRebuild] = 1u;
+    }
+    const double sum = wave_sum(static_cast<double>(ke2));
+    if (lane == pass) wave_ke = sum;
+  };
+  const bool at_once = FUSE != kForcesOnly && lgp == 0;
   for (uint32_t base = wk.y; base < wk.z; base += kStagedBlock >> lgp) {
     const uint32_t i = base + (threadIdx.x >> lgp);
     const bool live = i < wk.z;
+    float4 r, v, last;
+    if (at_once && live) {
+      r = a.r[i];
+      v = a.v[i];
+      last = nv.last_r[i];
+    }
     Acc acc;
     if (live) {
       const int4 fi = pos(i);
-      slot_terms<CUT>(a, rp, i, fi, part, lgp, nbl, num_nbrs, max_nbrs, cells, s_tab + 2 * fi.w * nt, pos, acc);
+      slot_terms<CUT, ENERGY>(a, rp, i, fi, part, lgp, nbl, num_nbrs, max_nbrs, cells, s_tab + 2 * fi.w * nt, pos,
+                              acc);
     }
-    combine_slot_lanes(acc, lgp);
-    if (live && part == 0) store_slot(a, i, acc);
+    const SlotSum t = combine_slot_lanes<ENERGY>(acc, lgp, unit);
+    if (live && part == 0 && (ENERGY || !at_once)) store_slot<ENERGY>(a, i, t);
+    if (at_once)
+      advance(i, live, r, v, last, make_float4(t.fx, t.fy, t.fz, 0.f), (base - wk.y) / kStagedBlock);
   }
-  if (FUSE) {
-    // the replica's forces are stored; its slots in 256-slot blocks, each
-    // block's m v^2 summed as k_b_nvt's block_sum does (its four waves' sums
-    // in order)
+  if (FUSE != kForcesOnly) {
+    __syncthreads();  // the staging is no longer read, and the forces are stored
+    if (!at_once) {
+      for (uint32_t base = wk.y; base < wk.z; base += kStagedBlock) {
+        const uint32_t i = base + threadIdx.x;
+        const bool live = i < wk.z;
+        float4 r, v, last, f;
+        if (live) {
+          r = a.r[i];
+          v = a.v[i];
+          last = nv.last_r[i];
+          f = a.f[i];
+        }
+        advance(i, live, r, v, last, f, (base - wk.y) / kStagedBlock);
+      }
+    }
+    double* s_w = reinterpret_cast<double*>(s_dyn);
+    const uint32_t passes = (rp.n + kStagedBlock - 1) / kStagedBlock;  // at most 10: the staging fits LDS
+    if (lane < passes) s_w[lane * (kStagedBlock / 64) + wave] = wave_ke;
     __syncthreads();
-    double* s_w = reinterpret_cast<double*>(s_dyn);  // the staging is no longer read
-    const Box bx = rep_box(rp);
-    const float ps = rp.omega2 > 0.f ? static_cast<float>(nv.nh[wk.x].ps) : 0.f;
-    const uint32_t nb = (rp.n + kBlock - 1) / kBlock;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    for (uint32_t b0 = 0; b0 < nb; b0 += kStagedBlock / kBlock) {
-      const uint32_t i = rp.slot0 + b0 * kBlock + threadIdx.x;
-      float ke2 = 0.f;
-      if (i - rp.slot0 < rp.n) {
-        float4 r = a.r[i], v = a.v[i];
-        float4 lo = make_float4(0.f, 0.f, 0.f, 0.f);
-        float3 shift;
-        ke2 = nvt_particle<false>(r, v, a.f[i], shift, lo, ps, nv.dt, bx);
-        a.r[i] = r;
-        a.fixed[i] = to_fixed(r, fixed_scale(rp));
-        a.v[i] = v;
-        add_image_shift(a.im, i, shift);
-        if (min_image_d2_f32(r, nv.last_r[i], bx) > nv.skin2_over_4) a.flags[kRepFlags * wk.x + kRebuild] = 1u;
-      }
-      const double wsum = wave_sum(static_cast<double>(ke2));
-      if (lane == 0) s_w[wave] = wsum;
-      __syncthreads();
-      const uint32_t q = threadIdx.x;  // block b0 + q, q < 4
-      if (q < kStagedBlock / kBlock && b0 + q < nb) {
-        double sum = 0.0;
-        for (uint32_t k = 0; k < kBlock / 64; ++k) sum += s_w[q * (kBlock / 64) + k];
-        nv.partials[rp.slot0 / kBlock + b0 + q] = sum;
-      }
-      __syncthreads();
+    if (wave == 0) {
+      double sum = 0.0;  // slots 256 lane, ...: at most 40 blocks
+      if (lane < (rp.n + kBlock - 1) / kBlock)
+        for (uint32_t k = 0; k < kBlock / 64; ++k) sum += s_w[lane * (kBlock / 64) + k];
+      const double tot = wave_sum(sum);
+      if (lane == 0) nh_advance_replica(nv.nh[wk.x], rp, tot, nv.dt);
     }
   }
 }
@@ -870,8 +962,7 @@ __global__ __launch_bounds__(kBlock) void k_b_nvt(BatchArgs a, const rumdx_nh_st
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
-// One workgroup per replica: its block partials in order, then
-// Ps += dt omega^2 min(KE2 / (dof T) - 1, 10) in FP64.
+// One workgroup per replica: its block partials in order, then the thermostat.
 __global__ __launch_bounds__(kBlock) void k_b_nvt_finish(const rumdx_replica* __restrict__ reps,
                                                          const double* __restrict__ partials,
                                                          rumdx_nh_state* __restrict__ nh, float dt) {
@@ -879,16 +970,7 @@ __global__ __launch_bounds__(kBlock) void k_b_nvt_finish(const rumdx_replica* __
   const rumdx_replica rp = reps[blockIdx.x];
   const uint32_t b0 = rp.slot0 / kBlock, nb = (rp.n + kBlock - 1) / kBlock;
   const double tot = sum_partials(partials + b0, nb, 1, s_red);
-  if (threadIdx.x == 0) {
-    rumdx_nh_state& s = nh[blockIdx.x];
-    s.ke2_sum = tot;
-    if (rp.omega2 > 0.f) {
-      double dev = tot / (static_cast<double>(rp.dof) * s.target_T) - 1.0;
-      if (dev > 10.0) dev = 10.0;  // runaway clamp (src/IntegratorNVT.cu:432-434)
-      s.ps += static_cast<double>(dt) * static_cast<double>(rp.omega2) * dev;
-      s.target_T += s.dT_per_step;
-    }
-  }
+  if (threadIdx.x == 0) nh_advance_replica(nh[blockIdx.x], rp, tot, dt);
 }
 
 // ------------------------------------------------------------------ energies
@@ -1029,9 +1111,9 @@ int check_batch_forces(const rumdx_batch* b, const float* params_dev, const char
   return RUMDX_OK;
 }
 
-// The replica-staged force kernel over the batch's work list (with FUSE, the
-// NVT update too).
-template <bool FUSE>
+// The replica-staged force kernel over the batch's work list (with kStepStore
+// or kStepInner, the NVT update too).
+template <int FUSE>
 int launch_staged(const rumdx_batch* b, const float* params_dev, int cutoff_method, const BatchNvt& nv,
                   hipStream_t st, const char* entry) {
   const uint32_t lpp = b->lanes_per_particle;
@@ -1039,7 +1121,10 @@ int launch_staged(const rumdx_batch* b, const float* params_dev, int cutoff_meth
   const BatchArgs a = args_of(b);
   const CellArrays cells{b->slot_cell_dev, b->cell_start_dev, b->cell_n_dev};
   size_t lds_staged = sizeof(float4) * 2 * b->ntypes * b->ntypes + sizeof(int4) * b->max_rep_n;
-  if (FUSE) lds_staged = std::max(lds_staged, sizeof(double) * (kStagedBlock / 64));  // the update's wave sums
+  // the update's wave sums replace the staging
+  if (FUSE != kForcesOnly)
+    lds_staged = std::max(lds_staged, sizeof(double) * ((b->max_rep_n + kStagedBlock - 1) / kStagedBlock) *
+                                          (kStagedBlock / 64));
   const auto* work = reinterpret_cast<const uint4*>(b->force_work_dev);
   const auto launch = [&](auto kernel) -> int {
     // above 64 KiB a workgroup's dynamic LDS must be opted into
@@ -1074,7 +1159,7 @@ extern "C" int rumdx_batch_forces(rumdx_batch* b, const float* params_dev, int c
   const size_t lds = sizeof(float4) * 2 * b->ntypes * b->ntypes;
   const CellArrays cells{b->slot_cell_dev, b->cell_start_dev, b->cell_n_dev};
   if (b->force_work_dev != nullptr)
-    return launch_staged<false>(b, params_dev, cutoff_method, BatchNvt{}, st, "rumdx_batch_forces");
+    return launch_staged<kForcesOnly>(b, params_dev, cutoff_method, BatchNvt{}, st, "rumdx_batch_forces");
   switch (cutoff_method) {
     case RUMDX_CUTOFF_NS:
       hipLaunchKernelGGL(k_b_force<RUMDX_CUTOFF_NS>, dim3(nblk), dim3(kBlock), lds, st, a, b->nbl_dev, b->num_nbrs_dev,
@@ -1107,22 +1192,35 @@ extern "C" int rumdx_batch_nvt_step(rumdx_batch* b, float dt, void* workspace_de
   return check_launch("rumdx_batch_nvt_step");
 }
 
+namespace rumdx {
+namespace {
+
+template <int FUSE>
+int batch_step(rumdx_batch* b, const float* params_dev, int cutoff_method, float dt, void* workspace_dev, void* stream,
+               const char* entry) {
+  int rc = check_batch_forces(b, params_dev, entry);
+  if (rc != RUMDX_OK) return rc;
+  const std::string e(entry);
+  if (b->force_work_dev == nullptr || b->force_work_whole == 0)
+    return fail(RUMDX_E_INVALID, e + ": needs a staged work list of whole replicas");
+  if (workspace_dev == nullptr || b->nh_dev == nullptr || b->last_r_dev == nullptr)
+    return fail(RUMDX_E_INVALID, e + ": null workspace, thermostat state or last_r");
+  const BatchNvt nv{b->nh_dev, reinterpret_cast<const float4*>(b->last_r_dev), dt, 0.25f * b->skin * b->skin};
+  return launch_staged<FUSE>(b, params_dev, cutoff_method, nv, as_stream(stream), entry);
+}
+
+}  // namespace
+}  // namespace rumdx
+
 extern "C" int rumdx_batch_forces_nvt(rumdx_batch* b, const float* params_dev, int cutoff_method, float dt,
                                       void* workspace_dev, void* stream) {
-  int rc = check_batch_forces(b, params_dev, "rumdx_batch_forces_nvt");
-  if (rc != RUMDX_OK) return rc;
-  if (b->force_work_dev == nullptr || b->force_work_whole == 0)
-    return fail(RUMDX_E_INVALID, "rumdx_batch_forces_nvt: needs a staged work list of whole replicas");
-  if (workspace_dev == nullptr || b->nh_dev == nullptr || b->last_r_dev == nullptr)
-    return fail(RUMDX_E_INVALID, "rumdx_batch_forces_nvt: null workspace, thermostat state or last_r");
-  const hipStream_t st = as_stream(stream);
-  double* partials = static_cast<double*>(workspace_dev);
-  const BatchNvt nv{b->nh_dev, reinterpret_cast<const float4*>(b->last_r_dev), partials, dt,
-                    0.25f * b->skin * b->skin};
-  rc = launch_staged<true>(b, params_dev, cutoff_method, nv, st, "rumdx_batch_forces_nvt");
-  if (rc != RUMDX_OK) return rc;
-  hipLaunchKernelGGL(k_b_nvt_finish, dim3(b->nrep), dim3(kBlock), 0, st, b->rep_dev, partials, b->nh_dev, dt);
-  return check_launch("rumdx_batch_forces_nvt");
+  return batch_step<kStepStore>(b, params_dev, cutoff_method, dt, workspace_dev, stream, "rumdx_batch_forces_nvt");
+}
+
+extern "C" int rumdx_batch_forces_nvt_inner(rumdx_batch* b, const float* params_dev, int cutoff_method, float dt,
+                                            void* workspace_dev, void* stream) {
+  return batch_step<kStepInner>(b, params_dev, cutoff_method, dt, workspace_dev, stream,
+                                "rumdx_batch_forces_nvt_inner");
 }
 
 extern "C" int rumdx_batch_energies(rumdx_batch* b, float dt, double* out_dev, void* workspace_dev, void* stream) {

@@ -423,12 +423,13 @@ void ReplicaBatch::CalcF() {
   rumdx_check(rumdx_batch_forces(&desc_, params_.get(), cutoff_method_, stream_), "ReplicaBatch", "CalcF");
 }
 
-void ReplicaBatch::Step() {
+void ReplicaBatch::Step(bool inner) {
   if (!allocated_) Allocate();
   if (UsesFusedSteps()) {
     rumdx_check(rumdx_batch_update_lists(&desc_, stream_), "ReplicaBatch", "RunSteps");
-    rumdx_check(rumdx_batch_forces_nvt(&desc_, params_.get(), cutoff_method_, dt_, workspace_.get(), stream_),
-                "ReplicaBatch", "RunSteps");
+    const auto step = inner ? rumdx_batch_forces_nvt_inner : rumdx_batch_forces_nvt;
+    rumdx_check(step(&desc_, params_.get(), cutoff_method_, dt_, workspace_.get(), stream_), "ReplicaBatch",
+                "RunSteps");
     return;
   }
   CalcF();
@@ -492,7 +493,8 @@ void ReplicaBatch::RunSteps(unsigned nsteps, unsigned block) {
       hipGraph_t g = nullptr;
       hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "ReplicaBatch", "RunSteps");
       try {
-        for (unsigned k = 0; k < block; ++k) Step();
+        // only the block's last step leaves energies and virials behind
+        for (unsigned k = 0; k < block; ++k) Step(k + 1 < block);
       } catch (...) {
         (void)hipStreamEndCapture(stream_, &g);
         if (g) (void)hipGraphDestroy(g);

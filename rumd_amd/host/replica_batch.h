@@ -99,7 +99,7 @@ class ReplicaBatch {
   };
   void Allocate();
   void Relayout();
-  void Step();
+  void Step(bool inner = false);
   void InvalidateGraphs();
   rumdx_replica HostReplica(unsigned r) const;
   std::vector<float> Slots(const DeviceArray<float>& a, unsigned replica, unsigned comps);

@@ -10,6 +10,7 @@ import pytest
 import oracle
 from capi import GpuSystem, check, gpu_available, lib
 from helpers import FORCE_TOL_GUARDED, force_errors, ka_table, load_golden, unsort
+from test_gpu_batch import make_batch
 from test_gpu_potentials import PE_ATOL, _forms, _table
 from rumd_amd import conf_io, configs, rumd
 
@@ -235,3 +236,29 @@ def test_sorted_lists_and_steps_at_each_tile_shape(n):
         d -= box * np.rint(d / box)
         near = np.flatnonzero((d * d).sum(axis=1) < (2.5 * 0.8) ** 2)
         assert set(near) - {i} <= set(ids[off[i]:off[i + 1]].tolist())
+
+
+@pytest.mark.parametrize("tp", [1, 2])
+def test_batch_steps_at_the_edges_of_the_passes(tp):
+    """Batched steps in one launch (a captured block: its inner steps without
+    energies) against separate calls: the same bits at the edges of the 256-slot
+    blocks and 1024-slot passes, with complete lists and with lists of which
+    all but a few overflow (partners then come from the cells)."""
+    sizes = [256, 257, 1024, 1025, 2049]
+    systems = [configs.ka_random_lattice(n, density=1.2, temperature=0.9, seed=300 + n) for n in sizes]
+    for cap in (None, 40):
+        out = []
+        for fused in (False, True):
+            b = make_batch(systems, [0.8, 1.5, 0.6, 1.0, 0.9], max_nbrs=cap)
+            b.SetThermostat(2, 0.6, 0.0)  # NVE
+            b.SetLanesPerParticle(tp)
+            b.SetFusedSteps(fused)
+            print(f"[case] batch passes fused={fused} lanes={tp} cap={cap}", flush=True)
+            b.RunSteps(10, 10)
+            out.append([(b.GetPositions(r), b.GetVelocities(r), b.GetForcesAndEnergies(r)) for r in range(len(sizes))]
+                       + [b.GetThermostatStates(), b.GetEnergies()])
+        for r in range(len(sizes)):
+            for k in range(3):
+                np.testing.assert_array_equal(out[0][r][k], out[1][r][k], err_msg=f"replica {r} array {k}")
+        np.testing.assert_array_equal(np.asarray(out[0][-2]), np.asarray(out[1][-2]))
+        np.testing.assert_array_equal(np.asarray(out[0][-1]), np.asarray(out[1][-1]))
