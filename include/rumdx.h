@@ -477,9 +477,37 @@ int rumdx_nvt_finish(const rumdx_nh_update* due, void* stream);
 /* rumdx_nblist_rebuild_sorted with a thermostat update that is due (due may be
  * NULL) done by one more workgroup of its first kernel, in every call; with
  * carry_forces 0 a rebuild leaves f and w behind (the next force call
- * initialises them). */
+ * initialises them).  With slot_of_dev (may be NULL) a rebuild also keeps the
+ * slot index of rumdx_slot_index up to date. */
 int rumdx_nblist_rebuild_sorted_due(rumdx_particles* p, rumdx_nblist* nb, const float box[8], int carry_forces,
-                                    const rumdx_nh_update* due, void* stream);
+                                    const rumdx_nh_update* due, uint32_t* slot_of_dev, void* stream);
+/* A step's bonded terms (at most RUMDX_MAX_BONDED_TERMS, added to the pair
+ * force in f in their order) and its NVT update in one kernel: the entry points
+ * of the term kinds followed by rumdx_nvt_step_due, bit for bit, except that
+ * the new positions go to r_out_dev (not p->r_dev; the caller swaps the two
+ * afterwards).  nb: the list whose skin the step checks, or NULL.  With
+ * store_forces 0 the summed forces, energies and virials are not written back.
+ * start, list, type (bonds only) and params are those of the term's own entry
+ * point.  No counterpart in the reference. */
+#define RUMDX_MAX_BONDED_TERMS 4
+#define RUMDX_TERM_BOND_HARMONIC 0
+#define RUMDX_TERM_BOND_FENE 1
+#define RUMDX_TERM_ANGLE_COSSQ 2
+#define RUMDX_TERM_ANGLE_SQ 3
+#define RUMDX_TERM_DIHEDRAL_RYCKAERT 4
+#define RUMDX_TERM_DIHEDRAL_PERIODIC 5
+typedef struct rumdx_bonded_term {
+  int kind;
+  uint32_t ntypes;
+  const uint32_t* start_dev;
+  const uint32_t* list_dev;
+  const uint32_t* type_dev;
+  const float* params_dev;
+} rumdx_bonded_term;
+int rumdx_bonded_nvt_due(const rumdx_particles* p, const rumdx_bonded_term* terms, uint32_t nterms,
+                         const uint32_t* slot_of_dev, const rumdx_nblist* nb, const float box[8], float* r_out_dev,
+                         const rumdx_nh_state* nh_dev, float dt, uint32_t thermostat_on_mask, int store_forces,
+                         void* workspace_dev, void* stream);
 
 /* Steps of a small sample (n <= RUMDX_SMALL_STEP_MAX) whose only force term is
  * a 12-6 pair potential over a list of the N2 method, or over all pairs (nb ==

@@ -440,6 +440,8 @@ struct HomeArrays {
   uint32_t* slot_cell;
   uint16_t* lane_order;
   uint32_t* cell_start;  // the build copies its cells' starts here from start_next
+  uint32_t* slot_of;     // slot index of the n particles kept up to date when non-null
+  uint32_t n;
 };
 
 // ------------------------------------------------------------------ incremental re-sort
@@ -1118,7 +1120,9 @@ __global__ __launch_bounds__(kBuildBlock) void k_build_tiles(uint32_t* __restric
     }
     o.im[i] = s.t_im[i];
     if (o.rlo != nullptr) o.rlo[i] = s.t_rlo[i];
-    o.idx[i] = s.t_idx[i];
+    const uint32_t id = s.t_idx[i];
+    o.idx[i] = id;
+    if (o.slot_of != nullptr && id < o.n) o.slot_of[id] = i;
   }
   // Lane order of the force kernel: the tile's particles by descending list
   // length, ties by slot (a rank count over unique keys; deterministic).
@@ -1529,7 +1533,7 @@ int check_sorted_args(const char* entry, const rumdx_particles* p, const rumdx_n
 // end of both sorted builds (the particles are staged in sorted order in s,
 // their cell starts in s.start_next).
 void launch_tile_build(rumdx_particles* p, rumdx_nblist* nb, const Box& bx, const SortScratch& s, hipStream_t st,
-                       bool carry) {
+                       bool carry, uint32_t* slot_of) {
   const TileGeom tg{nb->nc[0],           nb->nc[1],
                     nb->nc[2],           nb->cell_rank_dev,
                     s.start_next,        nb->tile_first_rank_dev,
@@ -1541,7 +1545,8 @@ void launch_tile_build(rumdx_particles* p, rumdx_nblist* nb, const Box& bx, cons
                         reinterpret_cast<float4*>(p->w_dev),
                         reinterpret_cast<float4*>(p->im_dev), reinterpret_cast<float4*>(p->rlo_dev),
                         p->unsorted_index_dev, reinterpret_cast<float4*>(nb->last_r_dev), nb->slot_cell_dev,
-                        nb->lane_order_dev, nb->cell_start_dev};
+                        nb->lane_order_dev, nb->cell_start_dev, slot_of,
+                        p->n};
   hipLaunchKernelGGL(k_build_tiles, dim3(nb->ntiles), dim3(kBuildBlock), sizeof(float4) * (nb->halo_cap + 1u), st,
                      nb->flags_dev, s, tg, nb->cut_skin2_dev, nb->ntypes, bx, home, nb->nbl16_dev, nb->num_nbrs_dev,
                      p->nvp, nb->max_nbrs);
@@ -1585,16 +1590,17 @@ extern "C" int rumdx_nblist_build_sorted(rumdx_particles* p, rumdx_nblist* nb, c
                      reinterpret_cast<const float4*>(p->f_dev), reinterpret_cast<const float4*>(p->w_dev),
                      reinterpret_cast<const float4*>(p->im_dev), reinterpret_cast<const float4*>(p->rlo_dev),
                      p->unsorted_index_dev, s, p->n);
-  launch_tile_build(p, nb, bx, s, st, true);
+  launch_tile_build(p, nb, bx, s, st, true, nullptr);
   return check_launch("rumdx_nblist_build_sorted");
 }
 
 extern "C" int rumdx_nblist_rebuild_sorted(rumdx_particles* p, rumdx_nblist* nb, const float box[8], void* stream) {
-  return rumdx_nblist_rebuild_sorted_due(p, nb, box, 1, nullptr, stream);
+  return rumdx_nblist_rebuild_sorted_due(p, nb, box, 1, nullptr, nullptr, stream);
 }
 
 extern "C" int rumdx_nblist_rebuild_sorted_due(rumdx_particles* p, rumdx_nblist* nb, const float box[8],
-                                               int carry_forces, const rumdx_nh_update* due, void* stream) {
+                                               int carry_forces, const rumdx_nh_update* due, uint32_t* slot_of_dev,
+                                               void* stream) {
   int rc = check_sorted_args("rumdx_nblist_rebuild_sorted", p, nb, box);
   if (rc != RUMDX_OK) return rc;
   if (due != nullptr && (due->nh_dev == nullptr || due->workspace_dev == nullptr || due->dof == 0))
@@ -1616,7 +1622,7 @@ extern "C" int rumdx_nblist_rebuild_sorted_due(rumdx_particles* p, rumdx_nblist*
   const NvtFinish fin = due != nullptr ? finish_args(*due) : NvtFinish{};
   hipLaunchKernelGGL(k_tile_resort, dim3(nb->ntiles + (due != nullptr ? 1u : 0u)), dim3(kBlock), 0, st, nb->flags_dev,
                      s, tg, bx, old, p->n, fin);
-  launch_tile_build(p, nb, bx, s, st, carry);
+  launch_tile_build(p, nb, bx, s, st, carry, slot_of_dev);
   return check_launch("rumdx_nblist_rebuild_sorted");
 }
 

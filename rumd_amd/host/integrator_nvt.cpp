@@ -83,6 +83,20 @@ void IntegratorNVT::IntegrateFused(PairPotential& pp, bool store_forces) {
   NoteDue(np);
 }
 
+void IntegratorNVT::IntegrateBonded(const rumdx_bonded_term* terms, uint32_t nterms, const uint32_t* slot_of,
+                                    bool store_forces) {
+  FinishDue();
+  NeighborList* nl = S->FusedCheckList();
+  ParticleData& pd = S->GetParticleData();
+  rumdx_check(rumdx_bonded_nvt_due(pd.Descriptor(), terms, nterms, slot_of, nl ? nl->Descriptor() : nullptr,
+                                   S->GetSimulationBox()->GetBox8(), pd.NextPositions(), d_state_.get(), timeStep,
+                                   thermostat_on_, store_forces ? 1 : 0, S->Workspace(), S->GetStream()),
+              "IntegratorNVT", "Integrate");
+  pd.SwapPositions();
+  if (nl) nl->NoteFusedCheck();
+  NoteDue(rumdx_nvt_partials(S->GetNumberOfParticles()));
+}
+
 void IntegratorNVT::NoteDue(unsigned npartials) {
   if (!thermostat_on_) return;
   due_partials_ = npartials;

@@ -191,6 +191,10 @@ void MoleculeData::UploadAngles() {
   sample_->InvalidateGraphs();
 }
 
+uint32_t* MoleculeData::SlotIndexArray() {
+  return slot_of_.size() == sample_->GetNumberOfParticles() ? slot_of_.get() : nullptr;
+}
+
 const uint32_t* MoleculeData::SlotIndex() {
   const unsigned n = sample_->GetNumberOfParticles();
   // allocated with the lists, never here: this runs inside captured graphs
@@ -238,17 +242,30 @@ void BondHarmonic::SetExclusions(PairPotential* non_bond_pot) {
   if (!pairs.empty()) non_bond_pot->GetNeighborList().AddExclusions(pairs);
 }
 
-void BondHarmonic::Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method) {
+MoleculeData* BondHarmonic::Topology(const char* method) {
   if (!sample) throw RUMD_Error(GetID_String(), method, "no sample");
   MoleculeData* m = sample->GetMoleculeData();
   if (m == nullptr) throw RUMD_Error(GetID_String(), method, "no molecule data: read a topology first");
   if (params_.empty()) throw RUMD_Error(GetID_String(), method, "no bond parameters set");
+  return m;
+}
+
+void BondHarmonic::Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method) {
+  MoleculeData* m = Topology(method);
   const uint32_t* slot_of = m->SlotIndex();
   const auto entry = fene_ ? rumdx_bond_fene : rumdx_bond_harmonic;
   rumdx_check(entry(p, slot_of, m->BondStart(), m->BondOther(), m->BondType(), d_params_.get(),
                     static_cast<uint32_t>(params_.size() / 2), sample->GetSimulationBox()->GetBox8(),
                     initialize ? 1 : 0, calc_stresses ? 1 : 0, sample->GetStream()),
               GetID_String().c_str(), method);
+}
+
+bool BondHarmonic::BondedTerm(rumdx_bonded_term* t) {
+  MoleculeData* m = Topology("CalcF");
+  *t = rumdx_bonded_term{fene_ ? RUMDX_TERM_BOND_FENE : RUMDX_TERM_BOND_HARMONIC,
+                         static_cast<uint32_t>(params_.size() / 2),
+                         m->BondStart(), m->BondOther(), m->BondType(), d_params_.get()};
+  return true;
 }
 
 void BondHarmonic::CalcF(bool initialize, bool calc_stresses) {
@@ -289,19 +306,32 @@ void AngleCosSq::SetExclusions(PairPotential* non_bond_pot) {
   if (!pairs.empty()) non_bond_pot->GetNeighborList().AddExclusions(pairs);
 }
 
-void AngleCosSq::Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method) {
+MoleculeData* AngleCosSq::Topology(const char* method) {
   if (!sample) throw RUMD_Error(GetID_String(), method, "no sample");
   MoleculeData* m = sample->GetMoleculeData();
   if (m == nullptr) throw RUMD_Error(GetID_String(), method, "no molecule data: read a topology first");
   if (params_.empty()) throw RUMD_Error(GetID_String(), method, "no angle parameters set");
   if (m->GetNumberOfAngleTypes() > params_.size() / 2)
     throw RUMD_Error(GetID_String(), method, "an angle type of the topology has no parameters");
+  return m;
+}
+
+void AngleCosSq::Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method) {
+  MoleculeData* m = Topology(method);
   const uint32_t* slot_of = m->SlotIndex();
   auto* entry = squared_ ? rumdx_angle_sq : rumdx_angle_cossq;
   rumdx_check(entry(p, slot_of, m->AngleStart(), m->AngleAtoms(), d_params_.get(),
                     static_cast<uint32_t>(params_.size() / 2), sample->GetSimulationBox()->GetBox8(),
                     initialize ? 1 : 0, calc_stresses ? 1 : 0, sample->GetStream()),
               GetID_String().c_str(), method);
+}
+
+bool AngleCosSq::BondedTerm(rumdx_bonded_term* t) {
+  MoleculeData* m = Topology("CalcF");
+  *t = rumdx_bonded_term{squared_ ? RUMDX_TERM_ANGLE_SQ : RUMDX_TERM_ANGLE_COSSQ,
+                         static_cast<uint32_t>(params_.size() / 2),
+                         m->AngleStart(), m->AngleAtoms(), nullptr, d_params_.get()};
+  return true;
 }
 
 void AngleCosSq::CalcF(bool initialize, bool calc_stresses) {
@@ -346,19 +376,32 @@ void DihedralRyckaert::SetExclusions(PairPotential* non_bond_pot) {
   if (!pairs.empty()) non_bond_pot->GetNeighborList().AddExclusions(pairs);
 }
 
-void DihedralRyckaert::Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method) {
+MoleculeData* DihedralRyckaert::Topology(const char* method) {
   if (!sample) throw RUMD_Error(GetID_String(), method, "no sample");
   MoleculeData* m = sample->GetMoleculeData();
   if (m == nullptr) throw RUMD_Error(GetID_String(), method, "no molecule data: read a topology first");
   if (params_.empty()) throw RUMD_Error(GetID_String(), method, "no dihedral parameters set");
   if (m->GetNumberOfDihedralTypes() > params_.size() / 6)
     throw RUMD_Error(GetID_String(), method, "a dihedral type of the topology has no parameters");
+  return m;
+}
+
+void DihedralRyckaert::Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method) {
+  MoleculeData* m = Topology(method);
   const uint32_t* slot_of = m->SlotIndex();
   auto* entry = periodic_ ? rumdx_dihedral_periodic : rumdx_dihedral_ryckaert;
   rumdx_check(entry(p, slot_of, m->DihedralStart(), m->DihedralAtoms(), d_params_.get(),
                     static_cast<uint32_t>(params_.size() / 6), sample->GetSimulationBox()->GetBox8(),
                     initialize ? 1 : 0, calc_stresses ? 1 : 0, sample->GetStream()),
               GetID_String().c_str(), method);
+}
+
+bool DihedralRyckaert::BondedTerm(rumdx_bonded_term* t) {
+  MoleculeData* m = Topology("CalcF");
+  *t = rumdx_bonded_term{periodic_ ? RUMDX_TERM_DIHEDRAL_PERIODIC : RUMDX_TERM_DIHEDRAL_RYCKAERT,
+                         static_cast<uint32_t>(params_.size() / 6),
+                         m->DihedralStart(), m->DihedralAtoms(), nullptr, d_params_.get()};
+  return true;
 }
 
 void DihedralRyckaert::CalcF(bool initialize, bool calc_stresses) {

@@ -358,7 +358,9 @@ void NeighborList::UpdateNBlist(bool forces_follow) {
     auto* itg = dynamic_cast<IntegratorNVT*>(sample_->GetIntegrator());
     if (itg != nullptr && !resort) itg->FinishDue();
     const bool take = itg != nullptr && itg->TakeDue(&due);
-    const int rc = resort ? rumdx_nblist_rebuild_sorted_due(p, &desc_, box, forces_follow ? 0 : 1, take ? &due : nullptr, st)
+    MoleculeData* m = sample_->GetMoleculeData();
+    const int rc = resort ? rumdx_nblist_rebuild_sorted_due(p, &desc_, box, forces_follow ? 0 : 1, take ? &due : nullptr,
+                                                            m ? m->SlotIndexArray() : nullptr, st)
                           : rumdx_nblist_build_sorted(p, &desc_, box, st);
     rumdx_check(rc, "NeighborList", "UpdateNBlist");
     sort_valid_ = true;

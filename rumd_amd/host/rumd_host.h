@@ -172,6 +172,9 @@ class Potential {
   virtual double GetVirial() { return 0.0; }
   // Bonds, angles: potentials whose terms come from the sample's topology.
   virtual bool IsMolecularPotential() const { return false; }
+  // The potential as a term of a step's one bonded kernel
+  // (rumdx_bonded_nvt_due), or false if it cannot be one.
+  virtual bool BondedTerm(rumdx_bonded_term*) { return false; }
   void SetVerbose(bool vb) { verbose = vb; }
   void SetID_String(const std::string& s) { ID_String = s; }
   std::string GetID_String() const { return ID_String; }
@@ -233,6 +236,8 @@ class NeighborList {
   void ResetFusedCheck() { fused_check_pending_ = false; }
   bool FusedCheckPending() const { return fused_check_pending_; }
   // True when the next sorted rebuild must be a full one (rumdx_nblist_build_sorted).
+  // Whether the next update leaves a slot index current that was so before.
+  bool KeepsSlotIndex() const { return GetResolvedMethod() != SORT || (UseTileResort() && !force_full_sort_); }
   bool NeedsFullSort() const { return GetResolvedMethod() == SORT && !UseTileResort(); }
   bool UseTileResort() const { return sort_valid_ && last_max_tile_ <= RUMDX_RESORT_TILE_MAX / 2; }
   void InvalidateSortOrder();
@@ -620,6 +625,8 @@ class MoleculeData {
   const std::vector<uint32_t>& GetAngles() const { return angles_; }
   // Refreshes slot_of from the particles' unsorted index (on the sample's stream).
   const uint32_t* SlotIndex();
+  // The slot index's array without a refresh (null unless it fits the sample).
+  uint32_t* SlotIndexArray();
   const uint32_t* BondStart() const { return bond_start_.get(); }
   const uint32_t* BondOther() const { return bond_other_.get(); }
   const uint32_t* BondType() const { return bond_type_.get(); }
@@ -651,6 +658,7 @@ class BondHarmonic : public Potential {
   void Initialize() override {}
   double GetPotentialEnergy() override;
   bool IsMolecularPotential() const override { return true; }
+  bool BondedTerm(rumdx_bonded_term* t) override;
   std::vector<float> GetParams() const { return params_; }
   // Bond types whose pairs the non-bonded potentials skip.
   std::vector<unsigned> GetExcludedTypes() const;
@@ -659,6 +667,8 @@ class BondHarmonic : public Potential {
   void SetExclusions(PairPotential* non_bond_pot);
 
  private:
+  // The topology, once the potential can act on it.
+  MoleculeData* Topology(const char* method);
   void Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method);
 
  protected:
@@ -690,6 +700,7 @@ class DihedralRyckaert : public Potential {
   void Initialize() override {}
   double GetPotentialEnergy() override;
   bool IsMolecularPotential() const override { return true; }
+  bool BondedTerm(rumdx_bonded_term* t) override;
   // DihedralPotential::SetExclude / SetExclusions: the end atoms (a, d) leave
   // the pair potential's list (on by default).
   void SetExclude(bool exclude) { exclude_dihedral_ = exclude; }
@@ -700,6 +711,8 @@ class DihedralRyckaert : public Potential {
   bool periodic_ = false;  // PeriodicDihedral
 
  private:
+  // The topology, once the potential can act on it.
+  MoleculeData* Topology(const char* method);
   void Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method);
   std::vector<float> params_;  // c_0..c_5 per type
   bool exclude_dihedral_ = true;
@@ -731,6 +744,7 @@ class AngleCosSq : public Potential {
   void Initialize() override {}
   double GetPotentialEnergy() override;
   bool IsMolecularPotential() const override { return true; }
+  bool BondedTerm(rumdx_bonded_term* t) override;
   std::vector<float> GetParams() const { return params_; }
   // AnglePotential::SetExclude / SetExclusions (src/AnglePotential.cu:63-66):
   // the end atoms (a, c) of every angle leave the pair potential's list
@@ -742,6 +756,8 @@ class AngleCosSq : public Potential {
   bool squared_ = false;  // AngleSq: u = k/2 (theta - theta0)^2
 
  private:
+  // The topology, once the potential can act on it.
+  MoleculeData* Topology(const char* method);
   void Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method);
   std::vector<float> params_;  // (theta0, k) per angle type
   bool exclude_angle_ = true;
@@ -806,6 +822,8 @@ class IntegratorNVT : public Integrator {
   // The step with the forces of `pp` computed in the same kernel
   // (PairPotential::CalcFIntegrateNVT): CalcF and Integrate of Simulation.Run.
   void IntegrateFused(PairPotential& pp, bool store_forces);
+  // The bonded terms and the step in one kernel, after the pair forces.
+  void IntegrateBonded(const rumdx_bonded_term* terms, uint32_t nterms, const uint32_t* slot_of, bool store_forces);
   // While recording a block of steps over sorted lists, a step's thermostat
   // update is left to the next step's list update (NeighborList takes it with
   // TakeDue) or, at the end, to Defer(false): one launch less per step.
@@ -984,7 +1002,11 @@ class Sample {
   };
   void PrepareRun();
   PairPotential* ChainPotential();
-  void StepOnce(bool zero_momentum, bool store_forces = true);
+  // The bonded potentials' terms when the steps take rumdx_bonded_nvt_due (a
+  // pair potential and one to four of them), else 0.
+  uint32_t BondedTerms(rumdx_bonded_term* terms);
+  // slots_known: the slot index was current before this step.
+  void StepOnce(bool zero_momentum, bool store_forces = true, bool slots_known = false);
   Block CaptureBlock(unsigned nsteps, bool reset_first);
   unsigned pb_ = 0, tp_ = 0;
   unsigned user_dofs_ = 0;

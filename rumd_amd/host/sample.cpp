@@ -254,15 +254,40 @@ void Sample::PrepareRun() {
       // re-sort of skin-triggered rebuilds (the build settles its capacities)
       if (nl.NeedsFullSort()) nl.UpdateNBlist();
     }
-  if (FusedStepPotential() != nullptr || ChainPotential() != nullptr) pd_.EnsureNextPositions();
+  rumdx_bonded_term terms[RUMDX_MAX_BONDED_TERMS];
+  if (FusedStepPotential() != nullptr || ChainPotential() != nullptr || BondedTerms(terms) != 0)
+    pd_.EnsureNextPositions();
 }
 
-void Sample::StepOnce(bool zero_momentum, bool store_forces) {
+uint32_t Sample::BondedTerms(rumdx_bonded_term* terms) {
+  if (!fused_steps_ || potentials_.size() < 2 || potentials_.size() > 1 + RUMDX_MAX_BONDED_TERMS ||
+      molecules_ == nullptr || molecules_->SlotIndexArray() == nullptr ||
+      dynamic_cast<IntegratorNVT*>(itg_) == nullptr || dynamic_cast<PairPotential*>(potentials_.front()) == nullptr)
+    return 0;
+  uint32_t n = 0;
+  for (size_t k = 1; k < potentials_.size(); ++k)
+    if (!potentials_[k]->BondedTerm(&terms[n++])) return 0;
+  return n;
+}
+
+void Sample::StepOnce(bool zero_momentum, bool store_forces, bool slots_known) {
   if (zero_momentum) itg_->SetMomentumToZero();
   PairPotential* pp = FusedStepPotential();
   if (pp != nullptr && pd_.HasNextPositions()) {
     BumpSlotEpoch();
     static_cast<IntegratorNVT*>(itg_)->IntegrateFused(*pp, store_forces);
+    return;
+  }
+  rumdx_bonded_term terms[RUMDX_MAX_BONDED_TERMS];
+  const uint32_t nterms = pd_.HasNextPositions() ? BondedTerms(terms) : 0u;
+  if (nterms != 0) {
+    if (!box_) throw RUMD_Error("Sample", "CalcF", "No simulation box has been set");
+    BumpSlotEpoch();
+    const bool known =
+        slots_known && static_cast<PairPotential*>(potentials_.front())->GetNeighborList().KeepsSlotIndex();
+    potentials_.front()->CalcF(true, false);
+    const uint32_t* slot_of = known ? molecules_->SlotIndexArray() : molecules_->SlotIndex();
+    static_cast<IntegratorNVT*>(itg_)->IntegrateBonded(terms, nterms, slot_of, store_forces);
     return;
   }
   CalcF(false);
@@ -306,7 +331,7 @@ Sample::Block Sample::CaptureBlock(unsigned nsteps, bool reset_first) {
       // the forces of the inner steps are replaced before anything reads them
       auto* itg = nl != nullptr && nl->IsSorted() ? dynamic_cast<IntegratorNVT*>(itg_) : nullptr;
       if (itg) itg->Defer(true);
-      for (unsigned k = 0; k < nsteps; ++k) StepOnce(k == 0 && reset_first, k + 1 == nsteps);
+      for (unsigned k = 0; k < nsteps; ++k) StepOnce(k == 0 && reset_first, k + 1 == nsteps, k > 0);
       if (itg) itg->Defer(false);
     }
     // fused steps alternate the two position arrays: the graph ends in the
@@ -374,6 +399,7 @@ MoleculeData* Sample::GetMoleculeData() { return molecules_.get(); }
 
 MoleculeData* Sample::CreateMoleculeData() {
   if (!GetNumberOfParticles()) throw RUMD_Error("Sample", "ReadMoleculeData", "Sample has no particles");
+  InvalidateGraphs();
   molecules_ = std::make_unique<MoleculeData>(this);
   return molecules_.get();
 }

@@ -262,3 +262,77 @@ def test_batch_steps_at_the_edges_of_the_passes(tp):
                 np.testing.assert_array_equal(out[0][r][k], out[1][r][k], err_msg=f"replica {r} array {k}")
         np.testing.assert_array_equal(np.asarray(out[0][-2]), np.asarray(out[1][-2]))
         np.testing.assert_array_equal(np.asarray(out[0][-1]), np.asarray(out[1][-1]))
+
+
+def _melt(golden_dir, chains, copies, method, kinds):
+    """`chains` five-bead chains of the pentamer melt, the box repeated `copies`
+    times per axis, with the potentials named in `kinds`."""
+    c = load_golden(golden_dir / "pentamer200_rho0.85_T0.5.xyz.gz")
+    box = np.asarray(c.box, np.float64)
+    shifts = np.array([[x, y, z] for x in range(copies) for y in range(copies) for z in range(copies)])
+    mid = (copies - 1) / 2.0
+    pos = np.concatenate([c.positions[:5 * chains] + (sh - mid) * box for sh in shifts])
+    total = copies ** 3 * chains
+    n, big = 5 * total, box * copies
+    pos -= big * np.rint(pos / big)
+    rng = np.random.default_rng(5)
+    s = rumd.Sample(0, 0)
+    s.SetVerbose(False)
+    s.SetConfiguration(conf_io.Configuration(
+        n=n, box=big, types=np.zeros(n, np.int32), positions=pos, masses=np.ones(1),
+        velocities=rng.normal(size=(n, 3)), images=np.zeros((n, 3))))
+    pot = rumd.Pot_LJ_12_6(cutoff_method=rumd.ShiftedPotential)
+    pot.SetVerbose(False)
+    pot.SetParams(0, 0, Sigma=1.0, Epsilon=1.0, Rcut=2.5)
+    pot.SetNbListSkin(0.3)
+    pot.SetNB_Method(method)
+    s.SetPotential(pot)
+    md = s.CreateMoleculeData()
+    first = 5 * np.arange(total)
+    md.SetBonds([int(x) for f in first for k in range(4) for x in (f + k, f + k + 1, k % 2)])
+    md.SetAngles([int(x) for f in first for k in range(3) for x in (f + k, f + k + 1, f + k + 2, 0)])
+    md.SetDihedrals([int(x) for f in first[::2] for k in range(2) for x in (f + k, f + k + 1, f + k + 2, f + k + 3, 0)])
+    for kind in kinds:
+        p = getattr(rumd, kind)()
+        p.SetVerbose(False)
+        if kind == "BondHarmonic":
+            p.SetParams(bond_type=0, bond_length=1.0, stiffness=100.0, exclude=False)
+        elif kind == "BondFENE":
+            p.SetParams(1, 2.5, 30.0, False)
+        elif kind.startswith("Angle"):
+            p.SetParams(angle_type=0, theta0=2.0, ktheta=20.0)
+        else:
+            p.SetParams(dihedral_type=0, coeffs=[1.0, -0.5, 0.3, 0.2, 0.1, -0.2][:4 if kind.startswith("P") else 6])
+        s.AddPotential(p)
+    itg = rumd.IntegratorNVT(timeStep=0.002, targetTemperature=1.0, thermostatRelaxationTime=0.2)
+    s.SetIntegrator(itg)
+    return s, itg, (pot, md)
+
+
+# one to four terms, every kind; remainders of the 256-slot workgroups; both
+# groupings of the kinetic energy
+@pytest.mark.parametrize("chains,copies,method,kinds", [
+    (51, 1, "none", ("BondHarmonic",)), (52, 1, "n2", ("BondFENE", "AngleSq")),
+    (200, 1, "n2", ("BondHarmonic", "AngleCosSq", "DihedralRyckaert")),
+    (200, 2, "sort", ("BondHarmonic", "BondFENE", "AngleSq", "PeriodicDihedral")),
+    (199, 3, "sort", ("BondHarmonic", "AngleCosSq"))])
+def test_bonded_steps_equal_the_separate_calls(golden_dir, chains, copies, method, kinds):
+    print(f"[case] bonded steps {5 * chains * copies ** 3} {method} {kinds}", flush=True)
+    a, itg_a, keep_a = _melt(golden_dir, chains, copies, method, kinds)
+    b, itg_b, keep_b = _melt(golden_dir, chains, copies, method, kinds)
+    i = 0
+    for steps, block in ((7, 7), (1, 5), (24, 8)):
+        a.RunSteps(i, steps, block, 20)
+        for k in range(i, i + steps):
+            if k % 20 == 0:
+                itg_b.SetMomentumToZero()
+            b.CalcF()
+            itg_b.Integrate()
+        i += steps
+        b.Synchronize()
+        for get in ("GetPositions", "GetVelocities", "GetImages", "GetForcesAndEnergies", "GetVirials"):
+            np.testing.assert_array_equal(getattr(a, get)(), getattr(b, get)(), err_msg=f"{get} after {i} steps")
+        assert itg_a.GetThermostatState() == itg_b.GetThermostatState()
+        assert itg_a.GetKineticEnergy() == itg_b.GetKineticEnergy()
+    if method != "none":
+        assert keep_a[0].GetNumberOfNbListBuilds() == keep_b[0].GetNumberOfNbListBuilds() > 1
