@@ -230,15 +230,21 @@ __device__ __forceinline__ void list_f64(const PosD& pi, uint32_t i, uint32_t nn
 
 // Tile lists of the sorted method: `split` workgroups per tile, the halo as
 // double positions in LDS by one gather over the slot list the build recorded,
-// a particle's list spread over as many of the 512 lanes as fit.  Bound by VALU
+// a particle's list spread over as many of its lanes as fit.  Bound by VALU
 // issue (45 operations a pair, 57 where the image is needed) with the LDS reads
-// close behind (64 bytes a pair).  At KA N = 32,768 (216 tiles) 56.5 -> 20.6 us
-// against one lane per particle walking 2-byte entries; 24.4 us with 32-byte
-// records in LDS.
+// close behind (64 bytes a pair).  At KA N = 32,768 56.5 -> 20.6 us in 216 tiles
+// against one lane per particle walking 2-byte entries (19.3 in the 726 smaller
+// tiles a sample of this size has); 24.4 us with 32-byte records in LDS.
 constexpr uint32_t kBlockF64 = 512;
+// Tiles of up to 128 particles on average fill fewer lanes (eight to a particle
+// at most), and the smaller workgroup lets one more share a CU.  384 against 512
+// lanes: 14.0 / 16.0 us at 18 particles a tile (n = 9,000), 19.3 / 22.4 at 45
+// (32,768), 28.2 / 28.3 at 87 (60,000), but 36.4 / 30.9 at 215 (110,000).
+constexpr uint32_t kBlockF64Small = 384;
+constexpr uint32_t kSmallTileF64 = 128;
 
-template <int CUT, bool STR, bool INIT>
-__global__ __launch_bounds__(kBlockF64) void k_lj_tiles_f64(
+template <int CUT, bool STR, bool INIT, uint32_t BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_lj_tiles_f64(
     const float4* __restrict__ r, const float4* __restrict__ rlo, float4* __restrict__ f, float4* __restrict__ w,
     float4* __restrict__ sts, const uint16_t* __restrict__ nbl16, const uint32_t* __restrict__ num_nbrs,
     const uint16_t* __restrict__ lane_order, const float* __restrict__ params, uint32_t nt, Box bx,
@@ -259,19 +265,19 @@ __global__ __launch_bounds__(kBlockF64) void k_lj_tiles_f64(
   if (staged) {
     const uint32_t* hs = halo_slots + static_cast<size_t>(t) * halo_cap;
     // slots of four particles, then their positions: each set in flight together
-    for (uint32_t q0 = threadIdx.x; q0 < info.x; q0 += 4u * kBlockF64) {
+    for (uint32_t q0 = threadIdx.x; q0 < info.x; q0 += 4u * BLOCK) {
       uint32_t slot[4];
       PosD p[4];
 #pragma unroll
       for (uint32_t u = 0; u < 4u; ++u) {
-        const uint32_t q = q0 + u * kBlockF64;
+        const uint32_t q = q0 + u * BLOCK;
         slot[u] = hs[q < info.x ? q : q0];
       }
 #pragma unroll
       for (uint32_t u = 0; u < 4u; ++u) p[u] = pos_d(r, rlo, slot[u]);
 #pragma unroll
       for (uint32_t u = 0; u < 4u; ++u)
-        if (q0 + u * kBlockF64 < info.x) s_pd.put(q0 + u * kBlockF64, shifted_f64(p[u], shifts, bx));
+        if (q0 + u * BLOCK < info.x) s_pd.put(q0 + u * BLOCK, shifted_f64(p[u], shifts, bx));
     }
   }
   __syncthreads();
@@ -280,9 +286,9 @@ __global__ __launch_bounds__(kBlockF64) void k_lj_tiles_f64(
   const uint32_t all = info.w - info.z;
   const uint32_t np = all > share ? (all - share + split - 1u) / split : 0u;
   uint32_t lg = 0;
-  while (lg < 3u && (np << (lg + 1u)) <= kBlockF64) ++lg;
+  while (lg < 3u && (np << (lg + 1u)) <= BLOCK) ++lg;
   const uint32_t part = threadIdx.x & ((1u << lg) - 1u), step = 1u << lg;
-  for (uint32_t c0 = 0; c0 < np; c0 += kBlockF64 >> lg) {
+  for (uint32_t c0 = 0; c0 < np; c0 += BLOCK >> lg) {
     const uint32_t k = c0 + (threadIdx.x >> lg);
     const bool live = k < np;
     AccD a;
@@ -381,12 +387,18 @@ int launch_f64(const rumdx_particles* p, const rumdx_nblist* nb, const float* pa
     // A small sample has fewer tiles than the chip holds workgroups: several
     // workgroups then share a tile, each staging its halo.  One / two / four:
     // 27 / 18 / 13 us at 64 tiles (n = 9,000), 23 / 16 / 16 at 125 (20,000),
-    // 32 / 30 / 40 at 343 (60,000), 31 / 36 / 51 at 512 (110,000).
+    // 32 / 30 / 40 at 343 (60,000), 31 / 36 / 51 at 512 (110,000), in 4^3 tiles.
     const uint32_t split = nb->ntiles >= 384u ? 1u : nb->ntiles >= 96u ? 2u : 4u;
-    hipLaunchKernelGGL((k_lj_tiles_f64<CUT, STR, INIT>), dim3(nb->ntiles * split), dim3(kBlockF64),
-                       tiles_f64_lds(cap, nt), st, r, rlo, f, w, sts, nb->nbl16_dev, nb->num_nbrs_dev,
-                       nb->lane_order_dev, params, nt, bx, reinterpret_cast<const uint4*>(nb->tile_info_dev),
-                       nb->tile_halo_dev, nb->halo_cap, cap, fb, p->nvp, nb->max_nbrs, split);
+    const auto launch = [&](auto kernel, uint32_t block) {
+      hipLaunchKernelGGL(kernel, dim3(nb->ntiles * split), dim3(block), tiles_f64_lds(cap, nt), st, r, rlo, f, w, sts,
+                         nb->nbl16_dev, nb->num_nbrs_dev, nb->lane_order_dev, params, nt, bx,
+                         reinterpret_cast<const uint4*>(nb->tile_info_dev), nb->tile_halo_dev, nb->halo_cap, cap, fb,
+                         p->nvp, nb->max_nbrs, split);
+    };
+    if (p->n <= static_cast<uint64_t>(kSmallTileF64) * nb->ntiles)
+      launch(k_lj_tiles_f64<CUT, STR, INIT, kBlockF64Small>, kBlockF64Small);
+    else
+      launch(k_lj_tiles_f64<CUT, STR, INIT, kBlockF64>, kBlockF64);
   } else {
     // a wave per particle over all pairs; 16 lanes over a list (some 90
     // entries), so that a sample of a thousand particles fills the CUs

@@ -336,3 +336,17 @@ def test_bonded_steps_equal_the_separate_calls(golden_dir, chains, copies, metho
         assert itg_a.GetKineticEnergy() == itg_b.GetKineticEnergy()
     if method != "none":
         assert keep_a[0].GetNumberOfNbListBuilds() == keep_b[0].GetNumberOfNbListBuilds() > 1
+
+
+# the FP64 tile kernel's two workgroup sizes (small tiles and 4x4x4 cells)
+@pytest.mark.parametrize("n", [9001, 33001, 130001])
+def test_fp64_forces_at_each_workgroup_size(n):
+    print(f"[case] fp64 tile shapes n={n}", flush=True)
+    a, pot, _ = _stepping_sample(n, "sort", True, False)
+    pot.SetFP64Forces(True)
+    a.CalcF()
+    pos4 = configs.pack_pos4(a.GetPositions(), a.GetTypes())
+    box = np.array([a.GetSimulationBox().GetLength(k) for k in range(3)])
+    f_ref, _ = oracle.forces_cells(pos4, box, 2, ka_table(), SF)
+    # the output's rounding (2^-24) and the float parameters the oracle shares
+    assert force_errors(a.GetForces(), f_ref[:, :3])["guarded_max"] <= 2e-7
