@@ -79,7 +79,7 @@ extern "C" {
 #define RUMDX_FLAG_DONE 4      /* internal completion counter, zero between calls */
 #define RUMDX_FLAG_MAXHALO 5   /* largest tile halo (particles) of the last sorted build, after rumdx_nblist_build_stats */
 #define RUMDX_FLAG_ERROR 6     /* nonzero: the last sorted build is unusable, RUMDX_BUILD_ERR_* bits */
-#define RUMDX_FLAG_EXCL_PENDING 7 /* internal: set by a completed build, cleared once its lists' exclusions are applied */
+#define RUMDX_FLAG_EXCL_PENDING 7 /* unused, zero (a build applies its lists' exclusions itself) */
 #define RUMDX_FLAG_MAXTILE 8   /* most particles in one cell tile, last sorted build, after rumdx_nblist_build_stats */
 #define RUMDX_FLAG_PRUNE 9     /* != 0: the next rumdx_nblist_prune rebuilds the inner lists */
 #define RUMDX_FLAG_STATS 10    /* internal: set by a completed sorted build, cleared by rumdx_nblist_build_stats */

@@ -120,7 +120,6 @@ __device__ __forceinline__ bool rebuild_pending(const uint32_t* flags) {
 __device__ __forceinline__ void complete_build(uint32_t* flags) {
   flags[RUMDX_FLAG_REBUILD] = 0u;
   flags[RUMDX_FLAG_BUILDS] += 1u;
-  flags[RUMDX_FLAG_EXCL_PENDING] = 1u;
   flags[RUMDX_FLAG_PRUNE] = 1u;
 }
 
@@ -1019,6 +1018,55 @@ __device__ __forceinline__ uint32_t build_particle_lane(uint32_t i, float4 ri, i
   return cnt;
 }
 
+// Exclusions on slot i's list in a tile of the sorted method
+// (apply_exclusion_list, src/NeighborList.cu:1323-1432): it loses the entries of
+// the particles its owner must not interact with, in place and in order, eight
+// entries' slots and ids read together.  Entries are decoded through the tile's
+// halo slot list hs (npart long), so tiles whose halo was not staged (their
+// force kernel rescans cells and skips exclusions there) and overflowed lists
+// are left alone.
+__device__ __forceinline__ void apply_exclusions(uint32_t i, const Exclusions& ex, uint32_t npart, bool bytes,
+                                                 const uint32_t* hs, uint16_t* nbl16, uint32_t* num_nbrs,
+                                                 uint32_t nvp, uint32_t max_nbrs) {
+  const ExclusionRange er = ex.of(i);
+  if (er.e0 == er.e1) return;
+  const uint32_t nn = num_nbrs[i];
+  if (nn >= max_nbrs) return;
+  u32x4* grp = reinterpret_cast<u32x4*>(nbl16);
+  u32x4 w = {0u, 0u, 0u, 0u};
+  uint32_t kept = 0;
+  for (uint32_t g = 0; g * 8u < nn; ++g) {
+    const u32x4 q = grp[static_cast<size_t>(g) * nvp + i];
+    const uint32_t m = nn - g * 8u < 8u ? nn - g * 8u : 8u;
+    uint32_t id[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t h = decode_entry(group_entry(q, e), bytes);
+      id[e] = static_cast<uint32_t>(e) < m && h < npart ? hs[h] : i;  // its own slot: never excluded
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) id[e] = ex.idx[id[e]];
+    uint32_t drop = 0;  // entries to leave out
+    for (uint32_t x = er.e0; x < er.e1; ++x) {
+      const uint32_t o = ex.ids[x];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) drop |= id[e] == o ? 1u << e : 0u;
+    }
+    if (drop == 0u && kept == g * 8u) {  // nothing left out so far: the group stands
+      kept += m;
+      continue;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (static_cast<uint32_t>(e) < m && !(drop & (1u << e)))
+        group_append(w, kept++, group_entry(q, e), grp, nvp, i);
+  }
+  if (kept < nn) {
+    if (kept & 7u) grp[static_cast<size_t>(kept >> 3) * nvp + i] = w;
+    num_nbrs[i] = kept;
+  }
+}
+
 // Workgroup of the tile build: one tile's halo positions are staged in LDS
 // once and shared by all its waves, so a larger workgroup has more waves in
 // flight per byte of LDS (the candidate loop is bound by LDS latency).
@@ -1040,7 +1088,7 @@ __global__ __launch_bounds__(kBuildBlock) void k_build_tiles(uint32_t* __restric
                                                              uint32_t nt, Box bx, HomeArrays o,
                                                              uint16_t* __restrict__ nbl16,
                                                              uint32_t* __restrict__ num_nbrs, uint32_t nvp,
-                                                             uint32_t max_nbrs) {
+                                                             uint32_t max_nbrs, Exclusions ex) {
   if (!rebuild_pending(flags)) return;
   // Arrival at the start (grouped counters, kArriveGroups), once every wave of
   // the block has read the request: its round trip overlaps the halo loads, and
@@ -1153,6 +1201,13 @@ __global__ __launch_bounds__(kBuildBlock) void k_build_tiles(uint32_t* __restric
     }
     o.lane_order[h.slot0 + rk] = static_cast<uint16_t>(k);
   }
+  // The lists above are complete (block_max_u32's barriers).  A launch of its own
+  // cost 4 us at every step to find nothing to do and 36 at a rebuild (100,000
+  // particles in chains).
+  if (ex.start != nullptr && staged)
+    for (uint32_t i = h.slot0 + threadIdx.x; i < h.slot1; i += kBuildBlock)
+      apply_exclusions(i, ex, h.npart, bytes, tg.halo_slots + static_cast<size_t>(t) * tg.halo_cap, nbl16, num_nbrs,
+                       nvp, max_nbrs);
   if (threadIdx.x == 0) {
     // per-tile records (longest list here, halo and slot range in tile_info),
     // reduced by k_build_stats when the host asks; plain stores, so no block
@@ -1187,51 +1242,6 @@ __global__ __launch_bounds__(kBuildBlock) void k_build_tiles(uint32_t* __restric
   const uint32_t r0 = tg.first_rank[t], r1 = tg.first_rank[t + 1];
   for (uint32_t c = r0 + threadIdx.x; c < r1; c += kBuildBlock) o.cell_start[c] = tg.cell_start[c];
   if (t == tg.ntiles - 1 && threadIdx.x == 0) o.cell_start[r1] = tg.cell_start[r1];
-}
-
-// Exclusions on the lists of the sorted method (apply_exclusion_list,
-// src/NeighborList.cu:1323-1432), after a rebuild only: each list loses the
-// entries of the particles its owner must not interact with, in place and in
-// order.  Entries are decoded through the tile's halo slot list, so tiles whose
-// halo was not staged (their force kernel rescans cells and skips exclusions
-// there) and overflowed lists are left alone.  A completed build raises
-// flags[EXCL_PENDING]; without it every block returns at once (no atomics on
-// the many idle steps).  With it, every block counts its arrival on the
-// build's grouped counters and the last one clears the flag, so no block can
-// miss it.
-__global__ __launch_bounds__(kBlock) void k_apply_exclusions(uint32_t* __restrict__ flags,
-                                                             const uint4* __restrict__ tile_info,
-                                                             const uint32_t* __restrict__ tile_halo, uint32_t halo_cap,
-                                                             Exclusions ex, uint16_t* __restrict__ nbl16,
-                                                             uint32_t* __restrict__ num_nbrs, uint32_t nvp,
-                                                             uint32_t max_nbrs, uint32_t* __restrict__ arrive) {
-  if (__hip_atomic_load(flags + RUMDX_FLAG_EXCL_PENDING, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) return;
-  // arrival at the start, on the grouped counters (the build left them at zero)
-  const bool last = threadIdx.x == 0 && grouped_arrival_last(arrive);
-  {
-    const uint32_t t = blockIdx.x;
-    const uint4 info = tile_info[t];
-    const bool staged = (info.y >> 16) == halo_cap && info.x <= halo_cap;
-    const bool bytes = info.x <= kByteEntryHalo;
-    const uint32_t* hs = tile_halo + static_cast<size_t>(t) * halo_cap;
-    for (uint32_t i = info.z + threadIdx.x; staged && i < info.w; i += kBlock) {
-      const ExclusionRange er = ex.of(i);
-      if (er.e0 == er.e1) continue;
-      const uint32_t nn = num_nbrs[i];
-      if (nn >= max_nbrs) continue;
-      uint32_t kept = 0;
-      for (uint32_t k = 0; k < nn; ++k) {
-        const size_t at = (static_cast<size_t>(k >> 3) * nvp + i) * 8u + (k & 7u);
-        const uint16_t e = nbl16[at];
-        const uint32_t h = decode_entry(e, bytes);
-        if (h < info.x && ex.excludes(er, hs[h])) continue;
-        nbl16[(static_cast<size_t>(kept >> 3) * nvp + i) * 8u + (kept & 7u)] = e;
-        ++kept;
-      }
-      num_nbrs[i] = kept;
-    }
-  }
-  if (last) flags[RUMDX_FLAG_EXCL_PENDING] = 0u;
 }
 
 // Converts tile-format entries (halo offsets) back to slots.
@@ -1529,9 +1539,8 @@ int check_sorted_args(const char* entry, const rumdx_particles* p, const rumdx_n
   return RUMDX_OK;
 }
 
-// The tile build, its finishing kernel and the exclusion pass: the common
-// end of both sorted builds (the particles are staged in sorted order in s,
-// their cell starts in s.start_next).
+// The tile build: the common end of both sorted builds (the particles are
+// staged in sorted order in s, their cell starts in s.start_next).
 void launch_tile_build(rumdx_particles* p, rumdx_nblist* nb, const Box& bx, const SortScratch& s, hipStream_t st,
                        bool carry, uint32_t* slot_of) {
   const TileGeom tg{nb->nc[0],           nb->nc[1],
@@ -1549,12 +1558,7 @@ void launch_tile_build(rumdx_particles* p, rumdx_nblist* nb, const Box& bx, cons
                         p->n};
   hipLaunchKernelGGL(k_build_tiles, dim3(nb->ntiles), dim3(kBuildBlock), sizeof(float4) * (nb->halo_cap + 1u), st,
                      nb->flags_dev, s, tg, nb->cut_skin2_dev, nb->ntypes, bx, home, nb->nbl16_dev, nb->num_nbrs_dev,
-                     p->nvp, nb->max_nbrs);
-  if (nb->excl_start_dev != nullptr)
-    hipLaunchKernelGGL(k_apply_exclusions, dim3(nb->ntiles), dim3(kBlock), 0, st, nb->flags_dev,
-                       reinterpret_cast<const uint4*>(nb->tile_info_dev), nb->tile_halo_dev, nb->halo_cap,
-                       Exclusions{p->unsorted_index_dev, nb->excl_start_dev, nb->excl_ids_dev}, nb->nbl16_dev,
-                       nb->num_nbrs_dev, p->nvp, nb->max_nbrs, s.arrive);
+                     p->nvp, nb->max_nbrs, Exclusions{s.t_idx, nb->excl_start_dev, nb->excl_ids_dev});
 }
 
 }  // namespace

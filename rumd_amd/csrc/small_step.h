@@ -118,7 +118,6 @@ __device__ __forceinline__ void small_build(const SmallStep& a, const Box& bx, u
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     a.flags[RUMDX_FLAG_BUILDS] += 1u;
-    a.flags[RUMDX_FLAG_EXCL_PENDING] = 1u;
     a.flags[RUMDX_FLAG_PRUNE] = 1u;
   }
   __syncthreads();  // the lists are read by other lanes below
