@@ -658,17 +658,16 @@ typedef struct rumdx_batch {
   uint32_t max_rep_cells;
 } rumdx_batch;
 
-/* rumdx_batch_forces followed by rumdx_batch_nvt_step in one launch (and the
- * thermostat's finishing kernel): with a staged work list of whole replicas
- * (force_work_whole), each workgroup computes its replica's forces and then
- * advances it in place, with the same per-256-slot kinetic-energy partials as
- * rumdx_batch_nvt_step; the results are the same bits as the two calls'.  No
- * counterpart in the reference. */
+/* rumdx_batch_forces followed by rumdx_batch_nvt_step in one launch: with a
+ * staged work list of whole replicas (force_work_whole), each workgroup computes
+ * its replica's forces, advances it in place and finishes its thermostat, the
+ * kinetic energy added in rumdx_batch_nvt_step's order; the results are the
+ * same bits as the two calls'.  No counterpart in the reference. */
 int rumdx_batch_forces_nvt(rumdx_batch* b, const float* params_dev, int cutoff_method, float dt,
                            void* workspace_dev, void* stream);
-/* The same step without potential energies and virials (f.w and w are left
- * unspecified): for a step that another one follows before anything reads
- * them.  Positions, velocities and thermostats come out as the same bits. */
+/* The same step without forces, energies and virials left behind (f and w are
+ * unspecified afterwards): for a step that another one follows before anything
+ * reads them.  Positions, velocities and thermostats come out as the same bits. */
 int rumdx_batch_forces_nvt_inner(rumdx_batch* b, const float* params_dev, int cutoff_method, float dt,
                                  void* workspace_dev, void* stream);
 /* Bytes of device workspace rumdx_batch_nvt_step / rumdx_batch_energies need. */

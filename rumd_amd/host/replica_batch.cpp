@@ -116,7 +116,14 @@ void ReplicaBatch::SetStagedForces(bool on) {
 
 // Staged forces: work items of one replica each, the largest replicas first,
 // when the largest fits one workgroup's LDS: whole replicas for fused steps,
-// else slot ranges of at most 2048.
+// else slot ranges.  A workgroup walks its item 1,024 slots at a time and one
+// runs on each CU, so a step takes as many such passes as the longest chain of
+// whole replicas has; a batch of too few replicas to fill the CUs is cut into
+// ranges instead where that saves at least three passes, although the update
+// and the thermostats are then launches of their own.  us a step, whole replicas
+// / ranges, replicas of 256 to 8,192 particles: 269 / 99 for 16 of them, 316 /
+// 183 for 100, 352 / 278 for 180, 375 / 364 for 256, 404 / 410 for 320, 510 /
+// 587 for 512.  The same bits either way.
 void ReplicaBatch::BuildForceWork() {
   force_work_.release();
   desc_.force_work_dev = nullptr;
@@ -128,9 +135,19 @@ void ReplicaBatch::BuildForceWork() {
   hip_check(hipDeviceGetAttribute(&optin, hipDeviceAttributeSharedMemPerBlockOptin, dev), "ReplicaBatch", "Allocate");
   const size_t staged_lds = 16ull * max_rep_n_ + 32ull * ntypes_ * ntypes_;
   if (!staged_forces_ || staged_lds > static_cast<size_t>(optin)) return;
-  const bool whole = fused_steps_;
-  const uint32_t chunk = whole ? 0xffffffffu : 2048u;
   const unsigned nrep = static_cast<unsigned>(reps_.size());
+  int cus = 0;
+  hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "ReplicaBatch", "Allocate");
+  const uint64_t ncu = static_cast<uint64_t>(std::max(cus, 1));
+  uint64_t passes = 0, longest = 0;
+  for (unsigned r = 0; r < nrep; ++r) {
+    const uint64_t p = (reps_[r].types.size() + 1023u) / 1024u;
+    passes += p;
+    longest = std::max(longest, p);
+  }
+  const uint64_t shared = (passes + ncu - 1) / ncu;  // passes per CU with the work spread evenly
+  const bool whole = fused_steps_ && (fused_asked_ || longest < shared + 3u);
+  const uint32_t chunk = whole ? 0xffffffffu : shared <= 2u ? 1024u : 2048u;
   std::vector<uint32_t> order(nrep);
   std::iota(order.begin(), order.end(), 0u);
   std::stable_sort(order.begin(), order.end(),
@@ -150,6 +167,7 @@ void ReplicaBatch::BuildForceWork() {
 
 void ReplicaBatch::SetFusedSteps(bool on) {
   fused_steps_ = on;
+  fused_asked_ = true;
   if (!allocated_) return;
   BuildForceWork();
   InvalidateGraphs();

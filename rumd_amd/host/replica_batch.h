@@ -45,8 +45,9 @@ class ReplicaBatch {
   bool GetWorkgroupSort() const { return workgroup_sort_; }
   bool UsesWorkgroupSort() const { return desc_.max_rep_cells != 0; }
   // Steps with the forces and the NVT update in one launch
-  // (rumdx_batch_forces_nvt; on by default with staged forces, whose work
-  // items are then whole replicas).  The same bits either way.
+  // (rumdx_batch_forces_nvt; by default with staged forces where the batch has
+  // replicas enough for work items of whole replicas, always once asked for).
+  // The same bits either way.
   void SetFusedSteps(bool on);
   bool GetFusedSteps() const { return fused_steps_; }
   bool UsesFusedSteps() const { return desc_.force_work_dev != nullptr && desc_.force_work_whole != 0; }
@@ -120,7 +121,7 @@ class ReplicaBatch {
   bool allocated_ = false;
   bool staged_forces_ = true;
   bool workgroup_sort_ = true;
-  bool fused_steps_ = true;
+  bool fused_steps_ = true, fused_asked_ = false;
   void BuildForceWork();
   uint32_t max_rep_n_ = 0, max_rep_cells_ = 0;
   hipStream_t stream_ = nullptr;

@@ -350,3 +350,21 @@ def test_fp64_forces_at_each_workgroup_size(n):
     f_ref, _ = oracle.forces_cells(pos4, box, 2, ka_table(), SF)
     # the output's rounding (2^-24) and the float parameters the oracle shares
     assert force_errors(a.GetForces(), f_ref[:, :3])["guarded_max"] <= 2e-7
+
+
+def test_small_batches_are_cut_into_slot_ranges():
+    """A batch of few large replicas takes slot ranges by default and whole
+    replicas when asked, with the same bits."""
+    systems = [configs.ka_random_lattice(n, density=1.2, temperature=0.9, seed=400 + n) for n in (4100, 3000)]
+    out = []
+    for fused in (False, True):
+        b = make_batch(systems, [0.8, 1.5])
+        if fused:
+            b.SetFusedSteps(True)
+        print(f"[case] small batch fused={fused}", flush=True)
+        b.RunSteps(12, 10)
+        assert b.UsesFusedSteps() == fused and b.GetFusedSteps()
+        out.append([(b.GetPositions(r), b.GetVelocities(r), b.GetForcesAndEnergies(r)) for r in range(2)])
+    for r in range(2):
+        for k in range(3):
+            np.testing.assert_array_equal(out[0][r][k], out[1][r][k], err_msg=f"replica {r} array {k}")
