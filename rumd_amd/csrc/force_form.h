@@ -7,8 +7,9 @@
 // skeleton is the shared kernels of force_kernels.h.  The kernels of a run's
 // steps (no stresses, initialising) are compiled per form, so the eight pairs of
 // a list group overlap; with the form as an argument every pair ended at a
-// branch over the forms (43.7 us at Buckingham N = 30,011, now 23.2 us with
-// the reciprocal and root of pot_forms.h; 63.9 -> 30.3 us at N = 150,000).  The
+// branch over the forms (43.7 us at Buckingham N = 30,011, then 23.2 us with
+// the reciprocal and root of pot_forms.h, 18.3 in smaller tiles; 63.9 -> 30.3 at
+// N = 150,000).  The
 // other variants take the form as an argument (FORM = 0), one set for all.
 //
 // Per type pair the LDS table holds three float4: {rc^2, p1, p2, p3},
