@@ -455,8 +455,8 @@ int rumdx_pair_lj_nvt(const rumdx_particles* p, const rumdx_nblist* nb, const fl
 /* Steps whose thermostat update is left to a later call: rumdx_nvt_step and
  * rumdx_pair_lj_nvt without UpdateThermostatState, the kinetic-energy partials
  * staying in the workspace (rumdx_nvt_partials(n), or nb->ntiles of them).  The
- * caller passes the update on to rumdx_nblist_rebuild_sorted_due or
- * rumdx_nvt_finish before anything else reads the state or uses the workspace.
+ * caller passes the update on to rumdx_nblist_rebuild_sorted_due,
+ * rumdx_nblist_build_n2_due or rumdx_nvt_finish before anything else reads the state or uses the workspace.
  * With store_forces 0 the fused step leaves energies and virials out: f holds
  * the forces, w is not written; the next step's forces replace them. */
 typedef struct rumdx_nh_update {
@@ -481,6 +481,10 @@ int rumdx_nvt_finish(const rumdx_nh_update* due, void* stream);
  * slot index of rumdx_slot_index up to date. */
 int rumdx_nblist_rebuild_sorted_due(rumdx_particles* p, rumdx_nblist* nb, const float box[8], int carry_forces,
                                     const rumdx_nh_update* due, uint32_t* slot_of_dev, void* stream);
+/* rumdx_nblist_build_n2 with a due thermostat update (may be NULL) done by one
+ * more workgroup, in every call. */
+int rumdx_nblist_build_n2_due(const rumdx_particles* p, rumdx_nblist* nb, const float box[8],
+                              const rumdx_nh_update* due, void* stream);
 /* A step's bonded terms (at most RUMDX_MAX_BONDED_TERMS, added to the pair
  * force in f in their order) and its NVT update in one kernel: the entry points
  * of the term kinds followed by rumdx_nvt_step_due, bit for bit, except that

@@ -9,8 +9,8 @@
 // a list group overlap; with the form as an argument every pair ended at a
 // branch over the forms (43.7 us at Buckingham N = 30,011, then 23.2 us with
 // the reciprocal and root of pot_forms.h, 18.3 in smaller tiles; 63.9 -> 30.3 at
-// N = 150,000).  The
-// other variants take the form as an argument (FORM = 0), one set for all.
+// N = 150,000).  The other variants take the form as an argument (FORM = 0), one
+// set for all.
 //
 // Per type pair the LDS table holds three float4: {rc^2, p1, p2, p3},
 // {p4, p5, p6, p7}, {s(rc) rc, shift, p8, p9}, with the energy shift u(rc) for

@@ -170,6 +170,22 @@ __device__ __forceinline__ void nvt_finish(const NvtFinish& u, double* s_red) {
   }
 }
 
+// The same by a workgroup of more than kBlock threads: the first kBlock add as
+// above.
+__device__ __forceinline__ void nvt_finish_wide(const NvtFinish& u, double* s_red) {
+  const uint32_t wave = threadIdx.x >> 6;
+  const double v = wave_sum(threadIdx.x < kBlock ? thread_partials(u.partials, u.np, 1) : 0.0);
+  if ((threadIdx.x & 63u) == 0 && wave < kBlock / 64) s_red[wave] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double tot = 0.0;
+    for (uint32_t k = 0; k < kBlock / 64; ++k) tot += s_red[k];
+    rumdx_nh_state st = *u.nh;
+    nh_advance(st, tot, u.dt, u.omega2, u.dof);
+    *u.nh = st;
+  }
+}
+
 // The kernel boundary makes the partials visible.
 __global__ __launch_bounds__(kBlock) void k_nvt_finish(NvtFinish u) {
   __shared__ double s_red[kBlock / 64];

@@ -160,7 +160,13 @@ __global__ __launch_bounds__(kN2Block) void k_build_n2(const float4* __restrict_
                                                        uint32_t* __restrict__ nbl, uint32_t* __restrict__ num_nbrs,
                                                        uint32_t* __restrict__ flags,
                                                        const float* __restrict__ cut_skin2, uint32_t nt, Box bx,
-                                                       uint32_t n, uint32_t nvp, uint32_t max_nbrs, Exclusions ex) {
+                                                       uint32_t n, uint32_t nvp, uint32_t max_nbrs, Exclusions ex,
+                                                       uint32_t nblocks, NvtFinish due) {
+  if (blockIdx.x == nblocks) {  // one more workgroup, launched when due.nh is set
+    __shared__ double s_red[kBlock / 64];
+    nvt_finish_wide(due, s_red);
+    return;
+  }
   if (!rebuild_pending(flags)) return;
   extern __shared__ float s_cut[];
   __shared__ float4 s_r[kN2Block];
@@ -182,7 +188,7 @@ __global__ __launch_bounds__(kN2Block) void k_build_n2(const float4* __restrict_
     __syncthreads();  // the first one: every wave of the block has read the request
     if (base == 0 && threadIdx.x == 0)
       last = __hip_atomic_fetch_add(flags + RUMDX_FLAG_DONE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-             gridDim.x - 1;
+             nblocks - 1;
     s_r[threadIdx.x] = next;
     __syncthreads();
     const uint32_t jn = base + kN2Block + threadIdx.x;
@@ -1355,6 +1361,11 @@ extern "C" int rumdx_nblist_request_rebuild(rumdx_nblist* nb, void* stream) {
 }
 
 extern "C" int rumdx_nblist_build_n2(const rumdx_particles* p, rumdx_nblist* nb, const float box[8], void* stream) {
+  return rumdx_nblist_build_n2_due(p, nb, box, nullptr, stream);
+}
+
+extern "C" int rumdx_nblist_build_n2_due(const rumdx_particles* p, rumdx_nblist* nb, const float box[8],
+                                         const rumdx_nh_update* due, void* stream) {
   int rc = check_nb(p, nb, "rumdx_nblist_build_n2");
   if (rc != RUMDX_OK) return rc;
   if (box == nullptr) return fail(RUMDX_E_INVALID, "rumdx_nblist_build_n2: null box");
@@ -1362,11 +1373,16 @@ extern "C" int rumdx_nblist_build_n2(const rumdx_particles* p, rumdx_nblist* nb,
   if (nb->excl_start_dev != nullptr && (nb->excl_ids_dev == nullptr || p->unsorted_index_dev == nullptr))
     return fail(RUMDX_E_INVALID, "rumdx_nblist_build_n2: exclusions need the exclusion ids and the unsorted index");
   if (p->n == 0) return RUMDX_OK;
+  if (due != nullptr && (due->nh_dev == nullptr || due->workspace_dev == nullptr || due->dof == 0))
+    return fail(RUMDX_E_INVALID, "rumdx_nblist_build_n2: incomplete thermostat update");
   const size_t lds = sizeof(float) * nb->ntypes * nb->ntypes;
-  hipLaunchKernelGGL(k_build_n2, dim3(blocks_for(p->n, kN2Block / 64)), dim3(kN2Block), lds, as_stream(stream),
+  const uint32_t nblocks = blocks_for(p->n, kN2Block / 64);
+  const NvtFinish fin = due != nullptr ? finish_args(*due) : NvtFinish{};
+  hipLaunchKernelGGL(k_build_n2, dim3(nblocks + (due != nullptr ? 1u : 0u)), dim3(kN2Block), lds, as_stream(stream),
                      reinterpret_cast<const float4*>(p->r_dev), reinterpret_cast<float4*>(nb->last_r_dev),
                      nb->nbl_dev, nb->num_nbrs_dev, nb->flags_dev, nb->cut_skin2_dev, nb->ntypes, make_box(box), p->n,
-                     p->nvp, nb->max_nbrs, Exclusions{p->unsorted_index_dev, nb->excl_start_dev, nb->excl_ids_dev});
+                     p->nvp, nb->max_nbrs, Exclusions{p->unsorted_index_dev, nb->excl_start_dev, nb->excl_ids_dev},
+                     nblocks, fin);
   return check_launch("rumdx_nblist_build_n2");
 }
 

@@ -205,8 +205,7 @@ __device__ __forceinline__ bool last_to_arrive(uint32_t* counter, uint32_t nbloc
 // Each thread adds its partials k, k + kBlock, ... in that order; the loads of
 // eight of them are issued together, so one workgroup does not wait for one
 // round trip per partial.
-__device__ __forceinline__ double sum_partials(const double* partials, uint32_t np, uint32_t stride,
-                                               double* lds4) {
+__device__ __forceinline__ double thread_partials(const double* partials, uint32_t np, uint32_t stride) {
   double v = 0.0;
   uint32_t k = threadIdx.x;
   for (; k + 7u * kBlock < np; k += 8u * kBlock) {
@@ -217,7 +216,12 @@ __device__ __forceinline__ double sum_partials(const double* partials, uint32_t 
     for (uint32_t u = 0; u < 8u; ++u) v += a[u];
   }
   for (; k < np; k += kBlock) v += partials[static_cast<size_t>(k) * stride];
-  return block_sum(v, lds4);
+  return v;
+}
+
+__device__ __forceinline__ double sum_partials(const double* partials, uint32_t np, uint32_t stride,
+                                               double* lds4) {
+  return block_sum(thread_partials(partials, np, stride), lds4);
 }
 
 // ------------------------------------------------------------------ workspace

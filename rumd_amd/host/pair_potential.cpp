@@ -349,13 +349,13 @@ void NeighborList::UpdateNBlist(bool forces_follow) {
   if (!fused_check_pending_) rumdx_check(rumdx_nblist_check(p, &desc_, box, st), "NeighborList", "UpdateNBlist");
   fused_check_pending_ = false;
   flags_changed_ = true;
+  rumdx_nh_update due;
+  auto* itg = dynamic_cast<IntegratorNVT*>(sample_->GetIntegrator());
   if (method == SORT) {
     sample_->GetParticleData().NoteSorted();
     // skin-triggered rebuilds re-sort tile by tile; the first build, and any
     // after the host changed positions or arrays, sorts from scratch
     const bool resort = UseTileResort() && !force_full_sort_;
-    rumdx_nh_update due;
-    auto* itg = dynamic_cast<IntegratorNVT*>(sample_->GetIntegrator());
     if (itg != nullptr && !resort) itg->FinishDue();
     const bool take = itg != nullptr && itg->TakeDue(&due);
     MoleculeData* m = sample_->GetMoleculeData();
@@ -368,8 +368,10 @@ void NeighborList::UpdateNBlist(bool forces_follow) {
     if (!resort && !force_full_sort_) Settle();
     Prune();
   }
-  else
-    rumdx_check(rumdx_nblist_build_n2(p, &desc_, box, st), "NeighborList", "UpdateNBlist");
+  else {
+    const bool take = itg != nullptr && itg->TakeDue(&due);
+    rumdx_check(rumdx_nblist_build_n2_due(p, &desc_, box, take ? &due : nullptr, st), "NeighborList", "UpdateNBlist");
+  }
 }
 
 // A full sort starts a new particle order.  Its halo and tile occupancy decide

@@ -329,7 +329,7 @@ Sample::Block Sample::CaptureBlock(unsigned nsteps, bool reset_first) {
       static_cast<IntegratorNVT*>(itg_)->IntegrateChain(*chain, nsteps);
     } else {
       // the forces of the inner steps are replaced before anything reads them
-      auto* itg = nl != nullptr && nl->IsSorted() ? dynamic_cast<IntegratorNVT*>(itg_) : nullptr;
+      auto* itg = nl != nullptr ? dynamic_cast<IntegratorNVT*>(itg_) : nullptr;
       if (itg) itg->Defer(true);
       for (unsigned k = 0; k < nsteps; ++k) StepOnce(k == 0 && reset_first, k + 1 == nsteps, k > 0);
       if (itg) itg->Defer(false);
