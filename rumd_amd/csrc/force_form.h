@@ -8,7 +8,7 @@
 // steps (no stresses, initialising) are compiled per form, so the eight pairs of
 // a list group overlap; with the form as an argument every pair ended at a
 // branch over the forms (43.7 us at Buckingham N = 30,011, then 23.2 us with
-// the reciprocal and root of pot_forms.h, 18.3 in smaller tiles; 63.9 -> 30.3 at
+// the reciprocal and root of pot_forms.h, 17.8 in smaller tiles; 63.9 -> 31.9 at
 // N = 150,000).  The other variants take the form as an argument (FORM = 0), one
 // set for all.
 //

@@ -10,6 +10,7 @@ import pytest
 import oracle
 from capi import GpuSystem, check, gpu_available, lib
 from helpers import force_errors, ka_table, unsort
+from test_gpu_potentials import PE_ATOL, _forms, _table
 from rumd_amd import configs
 
 pytestmark = pytest.mark.gpu
@@ -76,4 +77,36 @@ def test_fp64_energy_of_coincident_particles(method, cutoff):
     g.calc_f(cutoff, fp64=True)
     u = unsort(g.get("f"), g.unsorted_index())[:, 3]
     assert np.isposinf(u[[0, j]]).all()
+    assert np.isfinite(np.delete(u, [0, j])).all()
+
+
+# forms that have a value or an infinity of one sign at zero distance
+_AT_ZERO = ["smooth_2_4", "Gauss", "Buckingham", "IPL_18", "Yukawa", "Exp", "LJ_Gauss", "IPL_12", "IPL_9",
+            "IPL_18_class", "Dzugutov", "Fermi_Jagla", "Repulsive_Shoulder", "SAAP", "SF_Coulomb"]
+
+
+@pytest.mark.parametrize("stress", [False, True])  # compiled per form, and with the form as an argument
+@pytest.mark.parametrize("method", ["sorted", "n2", "none"])
+@pytest.mark.parametrize("case", [c for c in _forms() if c[0] in _AT_ZERO], ids=lambda c: c[0])
+def test_form_energy_of_coincident_particles(case, method, stress):
+    name, form, make, rows = case
+    table = _table(make, NS, rows)
+    s, pos4 = _ka(1003)
+    j = int(np.flatnonzero(s.types == s.types[0])[1])
+    pos4[j] = pos4[0]
+    # of the pair alone, at a distance where the form has reached its limit (or is beyond any float)
+    near = np.stack([pos4[0], pos4[0]])
+    near[:, :3] = 0.0
+    near[1, 0] = 1e-8
+    pair = 2.0 * oracle.forces_form_brute(near, s.box, 2, table, form, NS)[0][0, 3]
+    rest = oracle.forces_form_brute(np.delete(pos4, j, axis=0), s.box, 2, table, form, NS)[0]
+    g = _gpu(s, pos4, method, table, with_sts=stress)
+    print(f"[case] form {name} {method} stress={stress} coincident particles", flush=True)
+    g.calc_f(NS, form=form, stress=stress)
+    u = unsort(g.get("f"), g.unsorted_index())[:, 3]
+    if name in ("Gauss", "Exp"):
+        want = rest[0, 3] + 0.5 * pair
+        np.testing.assert_allclose(u[[0, j]], want, rtol=0, atol=max(PE_ATOL, 2e-6 * abs(want)))
+    else:
+        assert (u[[0, j]] == np.copysign(np.inf, pair)).all(), (u[[0, j]], pair)
     assert np.isfinite(np.delete(u, [0, j])).all()
