@@ -62,9 +62,17 @@ void IntegratorNVT::PullState() {
   if (d_state_.size()) d_state_.download(&host_state_, 1, S ? S->GetStream() : nullptr);
 }
 
-void IntegratorNVT::Integrate() {
+// What a step needs, checked before anything moves: the thermostat's update is
+// launched after the particles' and can refuse nothing any more.
+void IntegratorNVT::CheckStep() const {
   if (!S || !S->GetNumberOfParticles()) throw RUMD_Error("IntegratorNVT", "Integrate", kNoSample);
   if (!S->GetSimulationBox()) throw RUMD_Error("IntegratorNVT", "Integrate", "no simulation box");
+  if (thermostat_on_ && S->GetNumberOfDOFs() == 0)
+    throw RUMD_Error("IntegratorNVT", "Integrate", "zero degrees of freedom");
+}
+
+void IntegratorNVT::Integrate() {
+  CheckStep();
   FinishDue();
   NeighborList* nl = S->FusedCheckList();
   rumdx_check(rumdx_nvt_step_due(S->GetParticleData().Descriptor(), d_state_.get(), timeStep, thermostat_on_,
@@ -76,8 +84,7 @@ void IntegratorNVT::Integrate() {
 }
 
 void IntegratorNVT::IntegrateFused(PairPotential& pp, bool store_forces) {
-  if (!S || !S->GetNumberOfParticles()) throw RUMD_Error("IntegratorNVT", "Integrate", kNoSample);
-  if (!S->GetSimulationBox()) throw RUMD_Error("IntegratorNVT", "Integrate", "no simulation box");
+  CheckStep();
   const unsigned np = pp.CalcFIntegrateNVT(d_state_.get(), timeStep, thermostat_on_, store_forces);
   pp.GetNeighborList().NoteFusedCheck();
   NoteDue(np);
@@ -85,6 +92,7 @@ void IntegratorNVT::IntegrateFused(PairPotential& pp, bool store_forces) {
 
 void IntegratorNVT::IntegrateBonded(const rumdx_bonded_term* terms, uint32_t nterms, const uint32_t* slot_of,
                                     bool store_forces) {
+  CheckStep();
   FinishDue();
   NeighborList* nl = S->FusedCheckList();
   ParticleData& pd = S->GetParticleData();

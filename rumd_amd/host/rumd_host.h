@@ -842,6 +842,8 @@ class IntegratorNVT : public Integrator {
   void PullState();
   // omega^2 = 4 pi^2 / tau^2 formed in double, passed as float (src/IntegratorNVT.cu:88)
   float Omega2() const;
+  // Throws where a step cannot be taken.
+  void CheckStep() const;
   // Notes the update of a step just launched, done at once unless deferred.
   void NoteDue(unsigned npartials);
   bool defer_ = false;

@@ -1,0 +1,57 @@
+"""What the host classes keep between calls: after calls that are refused, when
+list flags are read, and for objects that serve more than one sample."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from capi import gpu_available
+from rumd_amd import conf_io, configs, rumd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _need_gpu():
+    if not gpu_available():
+        pytest.fail("no GPU visible: the gpu tests must run on an MI355X")
+
+
+def _sample(pos, box, velocity=0.5):
+    n = len(pos)
+    s = rumd.Sample(0, 0)
+    s.SetVerbose(False)
+    s.SetConfiguration(conf_io.Configuration(
+        n=n, box=np.full(3, float(box)), types=np.zeros(n, np.int32), positions=np.asarray(pos, np.float64),
+        masses=np.ones(1), velocities=np.full((n, 3), velocity), images=np.zeros((n, 3))))
+    return s
+
+
+def _lj(rcut, method="n2", max_nbrs=None):
+    pot = rumd.Pot_LJ_12_6(cutoff_method=rumd.ShiftedPotential)
+    pot.SetVerbose(False)
+    pot.SetParams(0, 0, Sigma=1.0, Epsilon=1.0, Rcut=rcut)
+    pot.SetNbListSkin(0.3)
+    pot.SetNB_Method(method)
+    if max_nbrs:
+        pot.SetNbMaxNumNbrs(max_nbrs)
+    return pot
+
+
+@pytest.mark.parametrize("method", ["n2", "none"])
+def test_a_step_without_degrees_of_freedom_moves_nothing(method):
+    """One particle has none (3 N - 3) for its thermostat: refused, as it was."""
+    s = _sample([[0.25, -1.0, 2.0]], 20.0)
+    pot, itg = _lj(2.5, method), rumd.IntegratorNVT(timeStep=0.005, targetTemperature=1.0,
+                                                    thermostatRelaxationTime=0.2)
+    s.SetPotential(pot)
+    s.SetIntegrator(itg)
+    r, v = s.GetPositions(), s.GetVelocities()
+    print(f"[case] no degrees of freedom {method}", flush=True)
+    s.CalcF()
+    for step in (itg.Integrate, lambda: s.RunSteps(0, 1, 1, 0), lambda: s.RunSteps(0, 4, 4, 0)):
+        with pytest.raises(RuntimeError, match="degrees of freedom"):
+            step()
+        np.testing.assert_array_equal(s.GetPositions(), r)
+        np.testing.assert_array_equal(s.GetVelocities(), v)
+        assert itg.GetThermostatState() == 0.0
