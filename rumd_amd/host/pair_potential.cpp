@@ -325,8 +325,7 @@ void NeighborList::Allocate() {
   }
   allocated_nvp_ = nvp;
   allocated_ = true;
-  flags_changed_ = true;
-  flags_queued_ = false;
+  NoteFlagsChanged();
   fused_check_pending_ = false;
   InvalidateSortOrder();
   rumdx_check(rumdx_nblist_request_rebuild(&desc_, st), "NeighborList", "Allocate");
@@ -348,7 +347,7 @@ void NeighborList::UpdateNBlist(bool forces_follow) {
   const hipStream_t st = sample_->GetStream();
   if (!fused_check_pending_) rumdx_check(rumdx_nblist_check(p, &desc_, box, st), "NeighborList", "UpdateNBlist");
   fused_check_pending_ = false;
-  flags_changed_ = true;
+  NoteFlagsChanged();
   rumdx_nh_update due;
   auto* itg = dynamic_cast<IntegratorNVT*>(sample_->GetIntegrator());
   if (method == SORT) {

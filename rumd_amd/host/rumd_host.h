@@ -224,8 +224,12 @@ class NeighborList {
   // forces_follow the caller initialises forces and virials next, so a rebuild
   // need not move them.
   void UpdateNBlist(bool forces_follow = false);
-  // Work that may change the flags has been launched since they were read.
-  void NoteFlagsChanged() { flags_changed_ = true; }
+  // Work that may change the flags has been launched since they were read (a
+  // queued read that nobody took up, as after an exception, is of before it).
+  void NoteFlagsChanged() {
+    flags_changed_ = true;
+    flags_queued_ = false;
+  }
   // Queues the read of the flags for the next HandleOverflow (before the
   // stream is synchronised); nothing when they cannot have changed.
   void QueueFlagsRead();

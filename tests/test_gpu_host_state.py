@@ -55,3 +55,36 @@ def test_a_step_without_degrees_of_freedom_moves_nothing(method):
         np.testing.assert_array_equal(s.GetPositions(), r)
         np.testing.assert_array_equal(s.GetVelocities(), v)
         assert itg.GetThermostatState() == 0.0
+
+
+def test_list_flags_are_read_anew_after_an_exception():
+    """Synchronize reads every list's flags and then acts on them; when acting
+    on the first list's throws, the second's are still to be read."""
+    n = 66000
+    k = 41  # 41^3 sites
+    box = 2.0 * k
+    site = np.arange(n)
+    pos = (np.stack([site // (k * k), site // k % k, site % k], axis=1) + 0.5) * 2.0 - 0.5 * box
+    s = _sample(pos, box, velocity=0.0)
+    # the first twenty are 0.2 apart after one step
+    together = pos[0] + 0.2 * np.stack([np.arange(20) % 3, np.arange(20) // 3 % 3, np.arange(20) // 9], axis=1)
+    vel = np.zeros((n, 3), np.float32)
+    vel[:20] = (together - pos[:20]) / 0.01
+    s.SetVelocities(vel)
+    itg = rumd.IntegratorNVE(timeStep=0.01)
+    s.SetIntegrator(itg)
+    # all pairs in reach: the list overflows, and cannot grow to 66,000 x 66,048 entries
+    a, b = _lj(1.2, max_nbrs=8), _lj(0.9 * box, max_nbrs=44000)
+    s.SetPotential(a)
+    s.AddPotential(b)  # ahead of the first
+    print("[case] flags after an exception", flush=True)
+    s.CalcF()
+    with pytest.raises(ValueError, match="2\\^32"):
+        s.Synchronize()
+    b.SetParams(0, 0, Sigma=1.0, Epsilon=1.0, Rcut=1.2)
+    b.SetNbMaxNumNbrs(64)
+    itg.Integrate()
+    s.CalcF()
+    s.Synchronize()  # the list of eight grows
+    s.CalcF()
+    assert np.diff(a.GetNeighborListCSR(s)[0])[:20].tolist() == [19] * 20
