@@ -148,9 +148,13 @@ void Sample::CalcF(bool calc_stresses) {
 }
 
 void Sample::Synchronize() {
-  // the lists' flags come back with this synchronisation
-  for (Potential* p : potentials_)
-    if (auto* pp = dynamic_cast<PairPotential*>(p)) pp->GetNeighborList().QueueFlagsRead();
+  // the lists' flags come back with this synchronisation (a potential that has
+  // since been given to another sample launches on that one's stream, which
+  // HandleOverflow waits for)
+  for (Potential* p : potentials_) {
+    auto* pp = dynamic_cast<PairPotential*>(p);
+    if (pp != nullptr && pp->GetSample() == this) pp->GetNeighborList().QueueFlagsRead();
+  }
   hip_check(hipStreamSynchronize(stream_), "Sample", "Synchronize");
   for (Potential* p : potentials_)
     if (auto* pp = dynamic_cast<PairPotential*>(p))

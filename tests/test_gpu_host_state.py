@@ -88,3 +88,24 @@ def test_list_flags_are_read_anew_after_an_exception():
     s.Synchronize()  # the list of eight grows
     s.CalcF()
     assert np.diff(a.GetNeighborListCSR(s)[0])[:20].tolist() == [19] * 20
+
+
+def test_list_flags_of_a_potential_given_to_another_sample():
+    """The first sample's Synchronize may find work of the second's in flight;
+    an overflow in that work is still acted upon."""
+    rng = np.random.default_rng(3)
+    n, box = 150001, 60.0
+    pos = rng.uniform(-0.5 * box, 0.5 * box, size=(n, 3))  # some 8 within 1.4 on average, some particles more than 16
+    first, second = _sample(pos[:1000], box), _sample(pos, box)
+    pot = _lj(1.1, max_nbrs=8)
+    first.SetPotential(pot)
+    first.CalcF()
+    first.Synchronize()
+    second.SetPotential(pot)
+    print("[case] flags of a shared potential", flush=True)
+    second.CalcF()
+    first.Synchronize()
+    second.Synchronize()
+    second.CalcF()
+    cnt = np.diff(pot.GetNeighborListCSR(second)[0])
+    assert cnt.max() == pot.GetActualMaxNumNbrs() > 16
