@@ -242,12 +242,16 @@ void BondHarmonic::SetExclusions(PairPotential* non_bond_pot) {
   if (!pairs.empty()) non_bond_pot->GetNeighborList().AddExclusions(pairs);
 }
 
+const char* BondHarmonic::Missing() const {
+  if (!sample) return "no sample";
+  if (sample->GetMoleculeData() == nullptr) return "no molecule data: read a topology first";
+  if (params_.empty()) return "no bond parameters set";
+  return nullptr;
+}
+
 MoleculeData* BondHarmonic::Topology(const char* method) {
-  if (!sample) throw RUMD_Error(GetID_String(), method, "no sample");
-  MoleculeData* m = sample->GetMoleculeData();
-  if (m == nullptr) throw RUMD_Error(GetID_String(), method, "no molecule data: read a topology first");
-  if (params_.empty()) throw RUMD_Error(GetID_String(), method, "no bond parameters set");
-  return m;
+  if (const char* what = Missing()) throw RUMD_Error(GetID_String(), method, what);
+  return sample->GetMoleculeData();
 }
 
 void BondHarmonic::Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method) {
@@ -261,7 +265,8 @@ void BondHarmonic::Launch(const rumdx_particles* p, bool initialize, bool calc_s
 }
 
 bool BondHarmonic::BondedTerm(rumdx_bonded_term* t) {
-  MoleculeData* m = Topology("CalcF");
+  if (Missing()) return false;  // CalcF says what
+  MoleculeData* m = sample->GetMoleculeData();
   *t = rumdx_bonded_term{fene_ ? RUMDX_TERM_BOND_FENE : RUMDX_TERM_BOND_HARMONIC,
                          static_cast<uint32_t>(params_.size() / 2),
                          m->BondStart(), m->BondOther(), m->BondType(), d_params_.get()};
@@ -306,14 +311,18 @@ void AngleCosSq::SetExclusions(PairPotential* non_bond_pot) {
   if (!pairs.empty()) non_bond_pot->GetNeighborList().AddExclusions(pairs);
 }
 
+const char* AngleCosSq::Missing() const {
+  if (!sample) return "no sample";
+  if (sample->GetMoleculeData() == nullptr) return "no molecule data: read a topology first";
+  if (params_.empty()) return "no angle parameters set";
+  if (sample->GetMoleculeData()->GetNumberOfAngleTypes() > params_.size() / 2)
+    return "an angle type of the topology has no parameters";
+  return nullptr;
+}
+
 MoleculeData* AngleCosSq::Topology(const char* method) {
-  if (!sample) throw RUMD_Error(GetID_String(), method, "no sample");
-  MoleculeData* m = sample->GetMoleculeData();
-  if (m == nullptr) throw RUMD_Error(GetID_String(), method, "no molecule data: read a topology first");
-  if (params_.empty()) throw RUMD_Error(GetID_String(), method, "no angle parameters set");
-  if (m->GetNumberOfAngleTypes() > params_.size() / 2)
-    throw RUMD_Error(GetID_String(), method, "an angle type of the topology has no parameters");
-  return m;
+  if (const char* what = Missing()) throw RUMD_Error(GetID_String(), method, what);
+  return sample->GetMoleculeData();
 }
 
 void AngleCosSq::Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method) {
@@ -327,7 +336,8 @@ void AngleCosSq::Launch(const rumdx_particles* p, bool initialize, bool calc_str
 }
 
 bool AngleCosSq::BondedTerm(rumdx_bonded_term* t) {
-  MoleculeData* m = Topology("CalcF");
+  if (Missing()) return false;  // CalcF says what
+  MoleculeData* m = sample->GetMoleculeData();
   *t = rumdx_bonded_term{squared_ ? RUMDX_TERM_ANGLE_SQ : RUMDX_TERM_ANGLE_COSSQ,
                          static_cast<uint32_t>(params_.size() / 2),
                          m->AngleStart(), m->AngleAtoms(), nullptr, d_params_.get()};
@@ -376,14 +386,18 @@ void DihedralRyckaert::SetExclusions(PairPotential* non_bond_pot) {
   if (!pairs.empty()) non_bond_pot->GetNeighborList().AddExclusions(pairs);
 }
 
+const char* DihedralRyckaert::Missing() const {
+  if (!sample) return "no sample";
+  if (sample->GetMoleculeData() == nullptr) return "no molecule data: read a topology first";
+  if (params_.empty()) return "no dihedral parameters set";
+  if (sample->GetMoleculeData()->GetNumberOfDihedralTypes() > params_.size() / 6)
+    return "a dihedral type of the topology has no parameters";
+  return nullptr;
+}
+
 MoleculeData* DihedralRyckaert::Topology(const char* method) {
-  if (!sample) throw RUMD_Error(GetID_String(), method, "no sample");
-  MoleculeData* m = sample->GetMoleculeData();
-  if (m == nullptr) throw RUMD_Error(GetID_String(), method, "no molecule data: read a topology first");
-  if (params_.empty()) throw RUMD_Error(GetID_String(), method, "no dihedral parameters set");
-  if (m->GetNumberOfDihedralTypes() > params_.size() / 6)
-    throw RUMD_Error(GetID_String(), method, "a dihedral type of the topology has no parameters");
-  return m;
+  if (const char* what = Missing()) throw RUMD_Error(GetID_String(), method, what);
+  return sample->GetMoleculeData();
 }
 
 void DihedralRyckaert::Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method) {
@@ -397,7 +411,8 @@ void DihedralRyckaert::Launch(const rumdx_particles* p, bool initialize, bool ca
 }
 
 bool DihedralRyckaert::BondedTerm(rumdx_bonded_term* t) {
-  MoleculeData* m = Topology("CalcF");
+  if (Missing()) return false;  // CalcF says what
+  MoleculeData* m = sample->GetMoleculeData();
   *t = rumdx_bonded_term{periodic_ ? RUMDX_TERM_DIHEDRAL_PERIODIC : RUMDX_TERM_DIHEDRAL_RYCKAERT,
                          static_cast<uint32_t>(params_.size() / 6),
                          m->DihedralStart(), m->DihedralAtoms(), nullptr, d_params_.get()};

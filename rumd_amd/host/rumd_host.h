@@ -671,6 +671,8 @@ class BondHarmonic : public Potential {
   void SetExclusions(PairPotential* non_bond_pot);
 
  private:
+  // What the potential lacks to act on the topology, or null.
+  const char* Missing() const;
   // The topology, once the potential can act on it.
   MoleculeData* Topology(const char* method);
   void Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method);
@@ -715,6 +717,8 @@ class DihedralRyckaert : public Potential {
   bool periodic_ = false;  // PeriodicDihedral
 
  private:
+  // What the potential lacks to act on the topology, or null.
+  const char* Missing() const;
   // The topology, once the potential can act on it.
   MoleculeData* Topology(const char* method);
   void Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method);
@@ -760,6 +764,8 @@ class AngleCosSq : public Potential {
   bool squared_ = false;  // AngleSq: u = k/2 (theta - theta0)^2
 
  private:
+  // What the potential lacks to act on the topology, or null.
+  const char* Missing() const;
   // The topology, once the potential can act on it.
   MoleculeData* Topology(const char* method);
   void Launch(const rumdx_particles* p, bool initialize, bool calc_stresses, const char* method);

@@ -109,3 +109,24 @@ def test_list_flags_of_a_potential_given_to_another_sample():
     second.CalcF()
     cnt = np.diff(pot.GetNeighborListCSR(second)[0])
     assert cnt.max() == pot.GetActualMaxNumNbrs() > 16
+
+
+@pytest.mark.parametrize("kind", ["BondHarmonic", "BondFENE", "AngleCosSq", "AngleSq", "DihedralRyckaert",
+                                  "PeriodicDihedral"])
+def test_no_steps_with_molecular_parameters_unset(kind):
+    """A run of no steps asks nothing of the potentials; one of a step names what is missing."""
+    s = _sample([[0.9 * i, 0.0, 0.1 * (i % 2)] for i in range(6)], 20.0)
+    pot, term, itg = _lj(2.5), getattr(rumd, kind)(), rumd.IntegratorNVE(timeStep=0.001)
+    md = s.CreateMoleculeData()
+    md.SetBonds([0, 1, 0, 1, 2, 0])
+    md.SetAngles([0, 1, 2, 0])
+    md.SetDihedrals([0, 1, 2, 3, 0])
+    s.SetPotential(pot)
+    s.AddPotential(term)
+    s.SetIntegrator(itg)
+    print(f"[case] parameters unset {kind}", flush=True)
+    s.RunSteps(0, 0, 10, 0)
+    assert s.PrepareRunSteps(0, 0, 10, 0) == 0
+    for steps in (1, 4):
+        with pytest.raises(RuntimeError, match="parameters"):
+            s.RunSteps(0, steps, steps, 0)
