@@ -156,8 +156,11 @@ typedef struct rumdx_nblist {
   uint16_t* lane_order_dev; /* sorted method: nvp, written by the build */
   uint32_t* tile_halo_dev;  /* sorted method: ntiles x halo_cap slots of each tile's halo, written by the build */
   uint32_t* tile_info_dev;  /* sorted method: ntiles x 4, written by the build */
-  uint32_t lanes_per_particle; /* 1, 2, 4 or 8 lanes share a particle's list in the force
-                                  kernels (RUMD's threads per particle, tp); 0 = 1 */
+  uint32_t lanes_per_particle; /* 1, 2, 4 or 8 lanes share a particle's list in the FP32 force
+                                  kernels (RUMD's threads per particle, tp); 0 = 1.  N2 lists
+                                  of at most RUMDX_SMALL_STEP_MAX particles take 16 whatever
+                                  this says, and a sorted list's small tiles more than it says
+                                  while their workgroup has lanes to spare */
   /* Exclusions (NeighborList::SetExclusion, src/NeighborList.cu:791-933): the
    * particles each particle does not interact with through this list, CSR
    * over original ids (p->unsorted_index_dev maps slots to them); NULL = none.

@@ -5,7 +5,12 @@ device (the scheme of Python/rumd/Autotune.py:83-448).
 Technical parameters, with their ranges:
 
     tp         [1, 2, 4, 8]  lanes sharing one particle's neighbour list in the
-                              force kernels (RUMD's threads per particle)
+                              force kernels (RUMD's threads per particle), where
+                              the kernels leave it to the user: not without a
+                              list (64 lanes) nor for N2 lists of up to 16,384
+                              particles (16 lanes); sorted lists in small tiles
+                              take more lanes than asked where their workgroup
+                              has them to spare
     waves      [4, 5, 6]     waves per SIMD the cell-tile force kernel is
                               compiled for (sorted lists; the tile mapping's
                               occupancy: more waves hide more latency, fewer
@@ -203,7 +208,14 @@ class Autotune:
             best["NB_method"] = "sort" if n > 8000 else "n2"
         methods = [self.fixed["NB_method"]] if "NB_method" in self.fixed else \
             [m for m in _METHODS if (m != "none" or n <= self.size_stop_no_nb) and (m != "n2" or n <= self.size_stop_n2)]
-        tps = [self.fixed["tp"]] if "tp" in self.fixed else list(_TP)
+
+        def tps(method):
+            """The values of tp that make a difference: the one there is, or all."""
+            if "tp" in self.fixed:
+                return [self.fixed["tp"]]
+            fixed_lanes = method == "none" or (method == "n2" and n <= rumd.SMALL_STEP_MAX)
+            return [best["tp"]] if fixed_lanes else list(_TP)
+
         self.trials = []
         nsteps = self._trial_steps(sim, best, saved)
 
@@ -216,7 +228,7 @@ class Autotune:
 
         scored = []
         for m in methods:
-            for tp in tps:
+            for tp in tps(m):
                 cand = dict(best, NB_method=m, tp=tp)
                 scored.append((trial(cand), cand))
         best = min(scored, key=lambda x: x[0])[1]
@@ -225,8 +237,8 @@ class Autotune:
             skins = sorted({round(s0 * f, 4) for f in (0.6, 0.8, 1.0, 1.25, 1.5)})
             scored = [(trial(dict(best, skin=sk)), dict(best, skin=sk)) for sk in skins]
             best = min(scored, key=lambda x: x[0])[1]
-            if "tp" not in self.fixed:
-                scored = [(trial(dict(best, tp=tp)), dict(best, tp=tp)) for tp in tps]
+            if len(tps(best["NB_method"])) > 1:
+                scored = [(trial(dict(best, tp=tp)), dict(best, tp=tp)) for tp in tps(best["NB_method"])]
                 best = min(scored, key=lambda x: x[0])[1]
         if "waves" not in self.fixed and best["NB_method"] == "sort":
             scored = [(trial(dict(best, waves=wv)), dict(best, waves=wv)) for wv in _WAVES]

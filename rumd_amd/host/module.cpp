@@ -60,6 +60,7 @@ PYBIND11_MODULE(_rumd, m) {
   });
 
   m.attr("VERSION") = "3.5";
+  m.attr("SMALL_STEP_MAX") = RUMDX_SMALL_STEP_MAX;  // largest sample whose N2 lists take 16 lanes each
   m.def("GetVersion", []() { return std::string("3.5"); });
   m.def("NumberOfPairPotentialParameters", []() { return RUMDX_NUM_PARAM; });
 

@@ -53,6 +53,7 @@ MoleculeData = _rumd.MoleculeData
 Integrator = _rumd.Integrator
 IntegratorNVT = _rumd.IntegratorNVT
 IntegratorNVE = _rumd.IntegratorNVE
+SMALL_STEP_MAX = _rumd.SMALL_STEP_MAX
 NoShift = _rumd.NoShift
 ShiftedPotential = _rumd.ShiftedPotential
 ShiftedForce = _rumd.ShiftedForce

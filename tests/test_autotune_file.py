@@ -59,3 +59,45 @@ def test_batch_entries_match_only_batches(tmp_path):
     assert not _same_user(batch, dict(batch, thermostats=[[0.5, 0.2], [1.6, 0.2]]))
     single = {"deviceName": "d", "N": 1500}
     assert not _same_user(batch, single)
+
+
+class _Timed(Autotune):
+    """Autotune over a made-up clock: the list method alone decides."""
+
+    def __init__(self, fastest, current, **kwargs):
+        super().__init__(**kwargs)
+        self.fastest, self.current = fastest, current
+
+    def GetCurrentTechnicalParameters(self, sim):
+        return {"pb": 64, "tp": self.current, "skin": 0.3, "NB_method": "default", "waves": 5}
+
+    @staticmethod
+    def _save(sim):
+        return {}
+
+    @staticmethod
+    def _restore(sim, saved):
+        pass
+
+    def _trial_steps(self, sim, params, saved):
+        return 40
+
+    def _time(self, sim, params, saved, nsteps):
+        return 1.0 if params["NB_method"] == self.fastest else 2.0
+
+
+@pytest.mark.parametrize("n,fastest,searched", [(500, "none", ["sort"]), (16384, "n2", ["sort"]),
+                                                (16385, "n2", ["n2", "sort"]), (40000, "sort", ["sort"])])
+def test_lanes_are_timed_only_where_they_make_a_difference(tmp_path, n, fastest, searched):
+    sim = type("Sim", (), {"sample": type("S", (), {"GetNumberOfParticles": lambda self: n})()})()
+    at = _Timed(fastest, 4, auto_filename=tmp_path / "autotune.json")
+    best = at.OptimizeTechnicalParameters(sim)
+    assert best["NB_method"] == fastest
+    tried = [t["params"] for t in at.trials if t["params"]["skin"] == 0.3]
+    for method in ("none", "n2", "sort"):
+        lanes = {p["tp"] for p in tried if p["NB_method"] == method}
+        if lanes:
+            assert lanes == ({1, 2, 4, 8} if method in searched else {4}), method
+    fixed = _Timed(fastest, 4, auto_filename=tmp_path / "autotune.json", tp=2)
+    assert fixed.OptimizeTechnicalParameters(sim)["tp"] == 2
+    assert {t["params"]["tp"] for t in fixed.trials} == {2}
