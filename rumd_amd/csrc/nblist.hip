@@ -154,14 +154,21 @@ __global__ void k_request_rebuild(uint32_t* flags) {
 // Arrivals are counted at the block's start, after its request read, so the
 // atomic's round trip overlaps the work; the block that starts last completes
 // the build.
+//
+// Every step launches the kernel, mostly to find nothing to do, so the grid is
+// bounded and a workgroup takes several groups of sixteen particles in turn
+// above 32,768 of them.  Idle launch / build at n = 100,000: 3.8 us / 6.09 ms,
+// and 7.3 / 5.97 without the bound (1.8 us / 15.8 ms with a thread per particle),
+// 2.4 / 6.50 with a quarter of it; 3.6 us / 0.62 ms at n = 30,000.  Above 80
+// scalar registers a CU holds one such workgroup instead of two (74 instead of
+// 57 us at n = 8,000).
 constexpr uint32_t kN2Block = 1024;
+constexpr uint32_t kN2Grid = 2048;
 
-__global__ __launch_bounds__(kN2Block) void k_build_n2(const float4* __restrict__ r, float4* __restrict__ last_r,
-                                                       uint32_t* __restrict__ nbl, uint32_t* __restrict__ num_nbrs,
-                                                       uint32_t* __restrict__ flags,
-                                                       const float* __restrict__ cut_skin2, uint32_t nt, Box bx,
-                                                       uint32_t n, uint32_t nvp, uint32_t max_nbrs, Exclusions ex,
-                                                       uint32_t nblocks, NvtFinish due) {
+__global__ __launch_bounds__(kN2Block) __attribute__((amdgpu_num_sgpr(80))) void k_build_n2(
+    const float4* __restrict__ r, float4* __restrict__ last_r, uint32_t* __restrict__ nbl,
+    uint32_t* __restrict__ num_nbrs, uint32_t* __restrict__ flags, const float* __restrict__ cut_skin2, uint32_t nt,
+    Box bx, uint32_t n, uint32_t nvp, uint32_t max_nbrs, Exclusions ex, uint32_t nblocks, NvtFinish due) {
   if (blockIdx.x == nblocks) {  // one more workgroup, launched when due.nh is set
     __shared__ double s_red[kBlock / 64];
     nvt_finish_wide(due, s_red);
@@ -173,47 +180,51 @@ __global__ __launch_bounds__(kN2Block) void k_build_n2(const float4* __restrict_
   __shared__ uint32_t s_max[kN2Block / 64];
   for (uint32_t k = threadIdx.x; k < nt * nt; k += kN2Block) s_cut[k] = cut_skin2[k];
   const uint32_t lane = threadIdx.x & 63u;
-  // this wave's particle (wave-uniform); the last workgroup's spare waves
-  // stage candidates and test none
-  const uint32_t i = __builtin_amdgcn_readfirstlane(blockIdx.x * (kN2Block / 64) + (threadIdx.x >> 6));
-  const bool live = i < n;
-  const float4 ri = r[live ? i : n - 1u];
-  const float* cut = s_cut + nt * __float_as_uint(ri.w);
-  const ExclusionRange er = ex.of(live ? i : n - 1u);
   const uint64_t below = (1ull << lane) - 1ull;
-  uint32_t cnt = 0;
-  bool last = false;
+  uint32_t most = 0;
   float4 next = r[threadIdx.x < n ? threadIdx.x : n - 1u];
-  for (uint32_t base = 0; base < n; base += kN2Block) {
-    __syncthreads();  // the first one: every wave of the block has read the request
-    if (base == 0 && threadIdx.x == 0)
-      last = __hip_atomic_fetch_add(flags + RUMDX_FLAG_DONE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-             nblocks - 1;
-    s_r[threadIdx.x] = next;
-    __syncthreads();
-    const uint32_t jn = base + kN2Block + threadIdx.x;
-    next = r[jn < n ? jn : n - 1u];
-    const uint32_t m = live ? min(n - base, kN2Block) : 0u;
-    for (uint32_t q = 0; q < m; q += 64u) {
-      const uint32_t j = base + q + lane;
-      const float4 rj = s_r[q + lane];
-      bool in = j < n && j != i && min_image_d2_f32(ri, rj, bx) < cut[__float_as_uint(rj.w)];
-      if (in) in = !ex.excludes(er, j);
-      const uint64_t hit = __builtin_amdgcn_ballot_w64(in);
-      if (in) {
-        const uint32_t k = cnt + static_cast<uint32_t>(__builtin_popcountll(hit & below));
-        if (k < max_nbrs) nbl[static_cast<size_t>(k) * nvp + i] = j;
+  __syncthreads();  // every wave of the block has read the request
+  const bool last = threadIdx.x == 0 && __hip_atomic_fetch_add(flags + RUMDX_FLAG_DONE, 1u, __ATOMIC_RELAXED,
+                                                               __HIP_MEMORY_SCOPE_AGENT) == nblocks - 1;
+  for (uint32_t first = blockIdx.x * (kN2Block / 64); first < n; first += nblocks * (kN2Block / 64)) {
+    // this wave's particle (wave-uniform); a last group's spare waves stage
+    // candidates and test none
+    const uint32_t i = __builtin_amdgcn_readfirstlane(first + (threadIdx.x >> 6));
+    const bool live = i < n;
+    const float4 ri = r[live ? i : n - 1u];
+    const float* cut = s_cut + nt * __float_as_uint(ri.w);
+    const ExclusionRange er = ex.of(live ? i : n - 1u);
+    uint32_t cnt = 0;
+    for (uint32_t base = 0; base < n; base += kN2Block) {
+      __syncthreads();
+      s_r[threadIdx.x] = next;
+      __syncthreads();
+      // the candidates after these, or the first again for the next group
+      const uint32_t jn = (base + kN2Block < n ? base + kN2Block : 0u) + threadIdx.x;
+      next = r[jn < n ? jn : n - 1u];
+      const uint32_t m = live ? min(n - base, kN2Block) : 0u;
+      for (uint32_t q = 0; q < m; q += 64u) {
+        const uint32_t j = base + q + lane;
+        const float4 rj = s_r[q + lane];
+        bool in = j < n && j != i && min_image_d2_f32(ri, rj, bx) < cut[__float_as_uint(rj.w)];
+        if (in) in = !ex.excludes(er, j);
+        const uint64_t hit = __builtin_amdgcn_ballot_w64(in);
+        if (in) {
+          const uint32_t k = cnt + static_cast<uint32_t>(__builtin_popcountll(hit & below));
+          if (k < max_nbrs) nbl[static_cast<size_t>(k) * nvp + i] = j;
+        }
+        // keeps counting past capacity: the true length sizes the regrowth
+        cnt += static_cast<uint32_t>(__builtin_popcountll(hit));
       }
-      // keeps counting past capacity: the true length sizes the regrowth
-      cnt += static_cast<uint32_t>(__builtin_popcountll(hit));
     }
+    if (live && lane == 0) {
+      last_r[i] = ri;
+      num_nbrs[i] = cnt < max_nbrs ? cnt : max_nbrs;  // == max_nbrs marks an overflowed list
+      if (cnt >= max_nbrs) flags[RUMDX_FLAG_OVERFLOW] = 1u;
+    }
+    most = max(most, cnt);
   }
-  if (live && lane == 0) {
-    last_r[i] = ri;
-    num_nbrs[i] = cnt < max_nbrs ? cnt : max_nbrs;  // == max_nbrs marks an overflowed list
-    if (cnt >= max_nbrs) flags[RUMDX_FLAG_OVERFLOW] = 1u;
-  }
-  const uint32_t longest = block_max_u32(cnt, s_max);
+  const uint32_t longest = block_max_u32(most, s_max);
   if (threadIdx.x == 0) {
     // an atomic only where the block raises the figure: rarely after the first build
     if (longest > __hip_atomic_load(flags + RUMDX_FLAG_MAXLEN, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
@@ -1376,7 +1387,7 @@ extern "C" int rumdx_nblist_build_n2_due(const rumdx_particles* p, rumdx_nblist*
   if (due != nullptr && (due->nh_dev == nullptr || due->workspace_dev == nullptr || due->dof == 0))
     return fail(RUMDX_E_INVALID, "rumdx_nblist_build_n2: incomplete thermostat update");
   const size_t lds = sizeof(float) * nb->ntypes * nb->ntypes;
-  const uint32_t nblocks = blocks_for(p->n, kN2Block / 64);
+  const uint32_t nblocks = std::min(blocks_for(p->n, kN2Block / 64), kN2Grid);
   const NvtFinish fin = due != nullptr ? finish_args(*due) : NvtFinish{};
   hipLaunchKernelGGL(k_build_n2, dim3(nblocks + (due != nullptr ? 1u : 0u)), dim3(kN2Block), lds, as_stream(stream),
                      reinterpret_cast<const float4*>(p->r_dev), reinterpret_cast<float4*>(nb->last_r_dev),

@@ -9,7 +9,7 @@ import pytest
 
 import oracle
 from capi import GpuSystem, check, gpu_available, lib
-from helpers import FORCE_TOL_GUARDED, force_errors, ka_table, load_golden, unsort
+from helpers import FORCE_TOL_GUARDED, force_errors, ka_table, load_golden, sorted_rows, unsort
 from test_gpu_batch import make_batch
 from test_gpu_potentials import PE_ATOL, _forms, _table
 from rumd_amd import conf_io, configs, rumd
@@ -55,6 +55,23 @@ def test_n2_lists_at_the_edges_of_the_wave_split(n):
     flags = g.flags_host()
     # (no rebuild pending, no overflow, two builds, the longest list, counter at zero)
     assert flags[:5].tolist() == [0, 0, 2, cnt.max(), 0]
+
+
+# more groups of sixteen particles than workgroups: some take two in turn
+@pytest.mark.parametrize("n", [32768, 32769, 32785])
+def test_n2_lists_beyond_one_group_per_workgroup(n):
+    s, pos4 = _ka(n)
+    g = _gpu(s, pos4, "n2", max_nbrs=160)
+    print(f"[case] n2 lists n={n}", flush=True)
+    for builds in (1, 2):
+        g.update_nblist()
+        cnt, nbl = g.neighbor_lists()
+        off, idx = oracle.nblist_brute_f32(pos4, configs.box8(s.box), 2, configs.cut_skin2_table(ka_table(), 0.3))
+        assert np.array_equal(cnt, np.diff(off))
+        lists = np.where(np.arange(nbl.shape[0])[:, None] < cnt, nbl[:, :n], np.uint32(0xffffffff))
+        assert np.array_equal(lists.T[:, : cnt.max()].astype(np.int64) & 0x7fffffff, sorted_rows(off, idx))
+        assert g.flags_host()[:5].tolist() == [0, 0, builds, cnt.max(), 0]
+        check(lib().rumdx_nblist_request_rebuild(C.byref(g.nb), None))
 
 
 # a wave per particle, four per workgroup, partners 512 at a time
