@@ -541,7 +541,10 @@ int launch_pair(const PP& pp, const char* entry, const rumdx_particles* p, const
   } else if (nb != nullptr) {
     // A small sample does not fill the chip: its lists are spread over 16
     // lanes, whatever lanes_per_particle asks (one pass of dependent reads
-    // instead of five: 7.7 -> 4.8 us at n = 1000).
+    // instead of five).  us with 16 lanes / 1, 4 and 8, LJ: 4.2 / 14.3, 6.1, 4.6 at
+    // n = 1,000; 5.1 / 15.0, 6.2, 4.8 at 8,000; 6.9 / 15.3, 6.4, 5.6 at 16,384; 9.2 /
+    // 15.2, 7.7, 6.6 at 24,000 (4 is a sample's default up to 10,000 particles, 1
+    // above).  The line is that of the one-kernel steps, which add in this order.
     const uint32_t lgn = p->n <= kSmallStepMax ? 4u : lgp;
     CellFallback fb{};
     fb.ex = Exclusions{p->unsorted_index_dev, nb->excl_start_dev, nb->excl_ids_dev};

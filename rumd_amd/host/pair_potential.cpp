@@ -668,10 +668,23 @@ unsigned PairPotential::CalcFIntegrateNVT(const rumdx_nh_state* nh_dev, float dt
   return neighborList.Descriptor()->ntiles;
 }
 
+// Largest sample whose steps over an N2 list run as a chain.  A rebuild inside a
+// chain tests its n^2 pairs with sixteen lanes per particle, in the build kernel
+// with sixty-four, so the more particles and the hotter they are, the more the
+// launch saved is paid back.  us a step, chain / separate launches, LJ at T = 0.45,
+// 0.8 and 2.0: 8.9/9.8, 9.6/10.1 and 11.0/10.8 at 3,000; 11.0/11.5, 12.3/12.2 and
+// 14.5/13.5 at 5,000; 13.2/12.8, 15.9/13.7 and 19.4/15.7 at 8,000.  Without a list
+// the chain is ahead throughout (76/89 at 8,000, 286/307 at 16,384).
+constexpr unsigned kChainN2Max = 5000;
+
 bool PairPotential::CanChainSteps() {
-  return sample != nullptr && GetPotentialForm() == 0 && !fp64_forces_ &&
-         neighborList.GetResolvedMethod() != NeighborList::SORT &&
-         sample->GetNumberOfParticles() <= RUMDX_SMALL_STEP_MAX;
+  if (sample == nullptr || GetPotentialForm() != 0 || fp64_forces_) return false;
+  const unsigned n = sample->GetNumberOfParticles();
+  switch (neighborList.GetResolvedMethod()) {
+    case NeighborList::SORT: return false;
+    case NeighborList::NONE: return n <= RUMDX_SMALL_STEP_MAX;
+    default: return n <= kChainN2Max;
+  }
 }
 
 void PairPotential::ChainStep(rumdx_nh_state* nh_dev, float dt, unsigned thermostat_on_mask, float omega2, unsigned dof,

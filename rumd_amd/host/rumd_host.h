@@ -371,8 +371,9 @@ class PairPotential : public Potential {
   bool GetFP64Forces() const { return fp64_forces_; }
   // True when the steps of a captured block of a small sample whose only force
   // term is this potential can run as one kernel each
-  // (rumdx_pair_lj_small_step): the 12-6 form in FP32 over an N2 list or over
-  // all pairs, at most RUMDX_SMALL_STEP_MAX particles.  ChainStep records step
+  // (rumdx_pair_lj_small_step): the 12-6 form in FP32 over all pairs, at most
+  // RUMDX_SMALL_STEP_MAX particles, or over an N2 list, fewer of them (the rule
+  // stands at CanChainSteps).  ChainStep records step
   // `step` of a block and swaps the position arrays; EndChain closes it.
   bool CanChainSteps();
   void ChainStep(rumdx_nh_state* nh_dev, float dt, unsigned thermostat_on_mask, float omega2, unsigned dof,

@@ -211,6 +211,12 @@ def test_one_kernel_steps_equal_the_separate_calls(n, method, thermo, mixed):
         assert pot_a.GetNumberOfNbListBuilds() == pot_b.GetNumberOfNbListBuilds() > 1
 
 
+# the largest N2 sample that steps in chains, and the smallest that does not
+@pytest.mark.parametrize("n", [5000, 5001])
+def test_steps_on_both_sides_of_the_chain_rule(n):
+    test_one_kernel_steps_equal_the_separate_calls(n, "n2", True, True)
+
+
 def test_one_kernel_steps_with_an_overflowed_list():
     """Lists that overflow inside a chain take all pairs, and grow afterwards."""
     a, pot_a, _ = _stepping_sample(1003, "n2", True, False)
