@@ -79,7 +79,7 @@ extern "C" {
 #define RUMDX_FLAG_DONE 4      /* internal completion counter, zero between calls */
 #define RUMDX_FLAG_MAXHALO 5   /* largest tile halo (particles) of the last sorted build, after rumdx_nblist_build_stats */
 #define RUMDX_FLAG_ERROR 6     /* nonzero: the last sorted build is unusable, RUMDX_BUILD_ERR_* bits */
-#define RUMDX_FLAG_EXCL_PENDING 7 /* unused, zero (a build applies its lists' exclusions itself) */
+/* word 7: reserved, zero */
 #define RUMDX_FLAG_MAXTILE 8   /* most particles in one cell tile, last sorted build, after rumdx_nblist_build_stats */
 #define RUMDX_FLAG_PRUNE 9     /* != 0: the next rumdx_nblist_prune rebuilds the inner lists */
 #define RUMDX_FLAG_STATS 10    /* internal: set by a completed sorted build, cleared by rumdx_nblist_build_stats */
@@ -669,7 +669,9 @@ typedef struct rumdx_batch {
  * staged work list of whole replicas (force_work_whole), each workgroup computes
  * its replica's forces, advances it in place and finishes its thermostat, the
  * kinetic energy added in rumdx_batch_nvt_step's order; the results are the
- * same bits as the two calls'.  No counterpart in the reference. */
+ * same bits as the two calls'.  workspace_dev is the two calls' (the one launch
+ * needs no scratch memory, but null is refused here too).  No counterpart in the
+ * reference. */
 int rumdx_batch_forces_nvt(rumdx_batch* b, const float* params_dev, int cutoff_method, float dt,
                            void* workspace_dev, void* stream);
 /* The same step without forces, energies and virials left behind (f and w are

@@ -200,31 +200,3 @@ void ParticleData::Get(const char* what, float* out, hipStream_t st, unsigned nc
 }
 
 void ParticleData::GetTypes(int32_t* out, hipStream_t) { std::copy(types_.begin(), types_.end(), out); }
-
-void ParticleData::ResetSorting(hipStream_t st) {
-  // bring every array back to original order, then identity index
-  std::vector<float> r(4ull * n_), v(4ull * n_), f(4ull * n_), w(4ull * n_), im(4ull * n_), lo;
-  Get("r", r.data(), st);
-  Get("v", v.data(), st);
-  Get("f", f.data(), st);
-  Get("w", w.data(), st);
-  Get("im", im.data(), st);
-  if (mixed_) {
-    lo.resize(4ull * n_);
-    Get("rlo", lo.data(), st);
-  }
-  std::vector<uint32_t> id(nvp_);
-  std::iota(id.begin(), id.end(), 0u);
-  d_unsorted_index.upload(id.data(), nvp_, st);
-  sorted_ = false;
-  auto put = [&](DeviceArray<float>& d, std::vector<float>& h) {
-    h.resize(4ull * nvp_, 0.f);
-    d.upload(h.data(), h.size(), st);
-  };
-  put(d_r, r);
-  put(d_v, v);
-  put(d_f, f);
-  put(d_w, w);
-  put(d_im, im);
-  if (mixed_) put(d_rlo, lo);
-}

@@ -239,9 +239,10 @@ class NeighborList {
   void NoteFusedCheck() { fused_check_pending_ = true; }
   void ResetFusedCheck() { fused_check_pending_ = false; }
   bool FusedCheckPending() const { return fused_check_pending_; }
-  // True when the next sorted rebuild must be a full one (rumdx_nblist_build_sorted).
-  // Whether the next update leaves a slot index current that was so before.
+  // Whether the next update leaves a slot index current that was so before: no
+  // sorted list, or one whose next rebuild is the tile re-sort.
   bool KeepsSlotIndex() const { return GetResolvedMethod() != SORT || (UseTileResort() && !force_full_sort_); }
+  // True when the next sorted rebuild must be a full one (rumdx_nblist_build_sorted).
   bool NeedsFullSort() const { return GetResolvedMethod() == SORT && !UseTileResort(); }
   bool UseTileResort() const { return sort_valid_ && last_max_tile_ <= RUMDX_RESORT_TILE_MAX / 2; }
   void InvalidateSortOrder();
@@ -893,7 +894,6 @@ class ParticleData {
   // The slots may be in another order than the particles' from now on.
   void NoteSorted() { sorted_ = true; }
   void GetTypes(int32_t* out, hipStream_t st);
-  void ResetSorting(hipStream_t st);
   rumdx_particles* Descriptor() { return &desc_; }
   std::vector<uint32_t> UnsortedIndex(hipStream_t st);
   // The second position array of fused steps (rumdx_pair_lj_nvt writes the
