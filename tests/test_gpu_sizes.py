@@ -110,6 +110,21 @@ def test_fp64_tiles_at_each_split(n, cutoff, stress):
             np.testing.assert_allclose(sts[:, :3], sts_ref[:, :3], rtol=0, atol=2e-7 * np.abs(sts_ref).max())
 
 
+# all six components, kept in sts and in the middle of w, at each split and list kind
+@pytest.mark.parametrize("method,n,cutoff", [("sorted", 2500, SP), ("sorted", 19001, SF), ("sorted", 95003, NS),
+                                             ("n2", 1003, SF), ("none", 333, SP)])
+def test_fp64_stress_components(method, n, cutoff):
+    s, pos4 = _ka(n)
+    g = _gpu(s, pos4, method, with_sts=True, **({"max_nbrs": 200} if method != "none" else {}))
+    print(f"[case] fp64 stress {method} n={n} cutoff={cutoff}", flush=True)
+    g.calc_f(cutoff, fp64=True, stress=True)
+    uidx = g.unsorted_index()
+    sts, w = unsort(g.get("sts"), uidx), unsort(g.get("w"), uidx)
+    ref = oracle.stress_brute(pos4, s.box, 2, ka_table(), cutoff)
+    # the output's rounding (2^-24) and the float parameters the oracle shares, as for the forces
+    np.testing.assert_allclose(np.column_stack([sts, w[:, 1:3]]), ref, rtol=0, atol=2e-7 * np.abs(ref).max())
+
+
 # list lanes and the all-pairs wave of the FP64 slot kernel
 @pytest.mark.parametrize("method,n", [("n2", 3), ("n2", 17), ("n2", 1003), ("none", 3), ("none", 333)])
 def test_fp64_slots_with_shared_lanes(method, n):
@@ -359,6 +374,53 @@ def test_bonded_steps_equal_the_separate_calls(golden_dir, chains, copies, metho
         assert itg_a.GetKineticEnergy() == itg_b.GetKineticEnergy()
     if method != "none":
         assert keep_a[0].GetNumberOfNbListBuilds() == keep_b[0].GetNumberOfNbListBuilds() > 1
+
+
+# the fused bonded step, the slot index that rebuilds keep and exclusions struck
+# out by the build, together in captured blocks
+@pytest.mark.parametrize("chains,copies,method,kinds", [
+    (200, 1, "n2", ("BondHarmonic", "AngleCosSq", "DihedralRyckaert")),
+    (200, 2, "sort", ("BondHarmonic", "AngleSq", "PeriodicDihedral")),
+    (199, 3, "sort", ("BondHarmonic", "AngleCosSq"))])
+def test_bonded_steps_with_exclusions_equal_the_separate_calls(golden_dir, chains, copies, method, kinds):
+    print(f"[case] bonded steps with exclusions {5 * chains * copies ** 3} {method} {kinds}", flush=True)
+    both = []
+    for _ in range(2):
+        s, itg, (pot, md) = _melt(golden_dir, chains, copies, method, kinds)
+        for p in s.GetPotentials():
+            if isinstance(p, rumd.BondHarmonic):
+                p.SetParams(bond_type=0, bond_length=1.0, stiffness=100.0, exclude=True)
+                p.SetParams(bond_type=1, bond_length=1.0, stiffness=100.0, exclude=True)
+            if hasattr(p, "SetExclusions"):
+                p.SetExclusions(pot)
+        both.append((s, itg, pot, md))
+    (a, itg_a, pot_a, _), (b, itg_b, pot_b, _) = both
+    total = chains * copies ** 3
+    gone = {(k, k + 1) for k in range(4)} | {(k, k + 2) for k in range(3)}  # bonds and the ends of angles
+    ends = {(k, k + 3) for k in range(2)} if len(kinds) == 3 else set()     # and of every other chain's dihedrals
+    assert pot_a.GetNumberOfExclusions() == total * len(gone) + (total + 1) // 2 * len(ends)
+    i = 0
+    for steps, block in ((7, 7), (1, 5), (24, 8), (16, 16)):
+        a.RunSteps(i, steps, block, 20)
+        for k in range(i, i + steps):
+            if k % 20 == 0:
+                itg_b.SetMomentumToZero()
+            b.CalcF()
+            itg_b.Integrate()
+        i += steps
+        b.Synchronize()
+        for get in ("GetPositions", "GetVelocities", "GetImages", "GetForcesAndEnergies", "GetVirials"):
+            np.testing.assert_array_equal(getattr(a, get)(), getattr(b, get)(), err_msg=f"{get} after {i} steps")
+        assert itg_a.GetThermostatState() == itg_b.GetThermostatState()
+    assert pot_a.GetNumberOfNbListBuilds() == pot_b.GetNumberOfNbListBuilds() > 1
+    off, ids = pot_a.GetNeighborListCSR(a)
+    first = np.repeat(np.arange(off.size - 1), np.diff(off))
+    same = first // 5 == ids // 5
+    lo, hi = np.minimum(first, ids)[same] % 5, np.maximum(first, ids)[same] % 5
+    near = {(int(x), int(y)) for x, y in zip(lo, hi)}
+    assert not near & gone
+    even = (first[same] // 5) % 2 == 0
+    assert not {(int(x), int(y)) for x, y in zip(lo[even], hi[even])} & ends
 
 
 # the FP64 tile kernel's two workgroup sizes (small tiles and 4x4x4 cells)
