@@ -313,9 +313,17 @@ __device__ __forceinline__ void tile_particles(const PP& pp, uint32_t slot0, uin
                                                const CellFallback& fb, uint32_t nvp, uint32_t max_nbrs,
                                                uint32_t lgp, uint32_t longest) {
   const uint32_t np = slot1 - slot0;
-  // a small tile's lists are spread over as many lanes as its workgroup has,
-  // while the longest still gives each lane a group
-  while (lgp < 3u && (np << (lgp + 1u)) <= kBlock && (8u << lgp) < longest) ++lgp;
+  // A small tile's lists are spread over as many lanes as its workgroup has,
+  // while the longest still gives each lane a group, where the launch is too
+  // small for other workgroups to use them: up to eight lanes with at most four
+  // workgroups per CU, two with at most sixteen.  Beyond, lanes that share a short
+  // list only wait for its last group, and two serve tiles of 65 to 128 particles
+  // alone.  us a step with 1 / 2 / 4 lanes, LJ cut at 1.5: 20.5 / 19.8 / 20.1 at
+  // n = 45,000 (1,331 tiles of 34 particles), 35.6 / 36.4 / 37.8 at 130,000 (3,375),
+  // 76.5 / 81.0 / 86.5 at 400,000 (10,648); cut at 2.0, 73 to 82 particles a tile,
+  // fused steps: 59.8 / 52.3 at 200,000 and 186 / 174 at 1,000,000.
+  const uint32_t most = gridDim.x <= 1024u ? 3u : gridDim.x <= 4096u || np > 64u ? 1u : 0u;
+  while (lgp < most && (np << (lgp + 1u)) <= kBlock && (8u << lgp) < longest) ++lgp;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t per_wave = 64u >> lgp;  // particles per wave and chunk: 2^lgp lanes each
   for (uint32_t c0 = (threadIdx.x >> 6) * per_wave; c0 < np; c0 += (kBlock / 64) * per_wave) {

@@ -246,6 +246,45 @@ def test_one_kernel_steps_with_an_overflowed_list():
     assert pot_a.GetActualMaxNumNbrs() > 40
 
 
+def _short_ranged(n, rcut, temperature=0.8):
+    """An LJ liquid at density 0.8442 cut off at rcut, sorted lists, constant energy."""
+    rng = np.random.default_rng(n)
+    k = int(np.ceil(n ** (1.0 / 3.0)))
+    box = (n / 0.8442) ** (1.0 / 3.0)
+    site = np.sort(rng.permutation(k ** 3)[:n])
+    pos = (np.stack([site // (k * k), site // k % k, site % k], axis=1) + 0.5) * (box / k) - 0.5 * box
+    pos = (pos + rng.uniform(-0.1, 0.1, size=pos.shape)).astype(np.float32)
+    sample = rumd.Sample(0, 0)
+    sample.SetVerbose(False)
+    sample.SetConfiguration(conf_io.Configuration(
+        n=n, box=np.full(3, box), types=np.zeros(n, np.int32), positions=pos, masses=np.ones(1),
+        velocities=rng.normal(size=(n, 3)) * np.sqrt(temperature), images=np.zeros((n, 3))))
+    pot = rumd.Pot_LJ_12_6(cutoff_method=rumd.ShiftedForce)
+    pot.SetVerbose(False)
+    pot.SetParams(0, 0, Sigma=1.0, Epsilon=1.0, Rcut=rcut)
+    pot.SetNbListSkin(0.3)
+    pot.SetNB_Method("sort")
+    sample.SetPotential(pot)
+    itg = rumd.IntegratorNVE(timeStep=0.002)
+    sample.SetIntegrator(itg)
+    return sample, pot, itg, configs.pack_pos4(sample.GetPositions(), np.zeros(n, np.int32)), np.full(3, box)
+
+
+# tiles of few particles: up to eight, two and one lane per list (1,331, 3,375 and
+# 4,913 tiles of 34 to 41), two lanes for the larger ones of many (4,913 of 66 to 81)
+@pytest.mark.parametrize("n,rcut,tiles", [(30001, 1.5, 729), (45001, 1.5, 1331), (130001, 1.5, 3375),
+                                          (200001, 1.5, 4913), (90001, 2.0, 1331), (400001, 2.0, 4913)])
+def test_forces_at_each_number_of_lanes(n, rcut, tiles):
+    s, pot, _itg, pos4, box = _short_ranged(n, rcut)
+    print(f"[case] lanes n={n} rcut={rcut}", flush=True)
+    s.CalcF()
+    assert pot.GetNbTileStats()["tiles"] == tiles
+    f = s.GetForcesAndEnergies()
+    table = configs.lj_param_table([(0, 0, 1.0, 1.0, rcut)], 1)
+    f_ref, _ = oracle.forces_cells(pos4, box, 1, table, SF)
+    assert force_errors(f[:, :3], f_ref[:, :3])["guarded_max"] <= FORCE_TOL_GUARDED
+
+
 # tiles of 2x2x2, 4x2x2, 4x4x2 and 4x4x4 cells
 @pytest.mark.parametrize("n", [9001, 33001, 66001, 130001])
 def test_sorted_lists_and_steps_at_each_tile_shape(n):
