@@ -642,13 +642,23 @@ void PairPotential::LaunchForce(const rumdx_particles* p, bool initialize, bool 
   rumdx_check(rc, GetID_String().c_str(), method);
 }
 
+// Fused steps advance a tile's particles with its workgroup: most of it idles
+// where a tile holds few.  They pay for tiles of 64 particles and more, and while
+// the tiles are few enough (four per CU) for the launch saved to count.  us a step,
+// fused / separate launches, LJ: cut at 2^(1/6), 16.5 to 20 particles a tile,
+// 14.4 / 15.5 at 12,000 (729 tiles), 15.5 / 16.3 at 20,000 (1,000), 23.5 / 19.9 at
+// 30,000 (1,728), 111 / 86 at 260,000 (13,824); cut at 2.5, density 0.3, 31.0 / 28.7
+// at 65,000 (1,331 tiles of 49).
+constexpr unsigned kFusedTiles = 1024;
+
 bool PairPotential::CanFuseStep() {
   if (!sample || GetPotentialForm() != 0 || fp64_forces_) return false;
   if (neighborList.GetResolvedMethod() != NeighborList::SORT) return false;
   const rumdx_nblist* nb = neighborList.Descriptor();
   if (nb->nbl16_dev == nullptr || nb->ntiles == 0) return false;
-  // the sample's workspace holds a partial sum per tile
-  return 256 + sizeof(double) * static_cast<size_t>(nb->ntiles) <= rumdx_workspace_bytes(sample->GetNumberOfParticles());
+  const unsigned n = sample->GetNumberOfParticles();
+  return nb->ntiles <= std::max(kFusedTiles, 4 * ((n + 255) / 256)) &&
+         256 + sizeof(double) * static_cast<size_t>(nb->ntiles) <= rumdx_workspace_bytes(n);  // a partial sum per tile
 }
 
 unsigned PairPotential::CalcFIntegrateNVT(const rumdx_nh_state* nh_dev, float dt, unsigned thermostat_on_mask,

@@ -285,6 +285,24 @@ def test_forces_at_each_number_of_lanes(n, rcut, tiles):
     assert force_errors(f[:, :3], f_ref[:, :3])["guarded_max"] <= FORCE_TOL_GUARDED
 
 
+# both sides of the fused steps' rule: at most 1,024 tiles, or 64 particles a tile;
+# the same bits either way
+@pytest.mark.parametrize("n,rcut,fused", [(20000, 2.0 ** (1.0 / 6.0), True), (30000, 2.0 ** (1.0 / 6.0), False),
+                                          (65000, 1.7, False), (90000, 2.0, True)])
+def test_fused_steps_on_both_sides_of_their_rule(n, rcut, fused):
+    print(f"[case] fused rule n={n} rcut={rcut:.3f}", flush=True)
+    a, pot_a, _ia, _, _ = _short_ranged(n, rcut)
+    b, _pb, _ib, _, _ = _short_ranged(n, rcut)
+    b.SetFusedSteps(False)
+    a.RunSteps(0, 40, 10, 0)  # rebuilds inside
+    b.RunSteps(0, 40, 10, 0)
+    tiles = pot_a.GetNbTileStats()["tiles"]
+    assert a.UsesFusedSteps() == fused == (tiles <= 1024 or 64 * tiles <= n)
+    assert pot_a.GetNumberOfNbListBuilds() > 1
+    for get in ("GetPositions", "GetVelocities", "GetImages", "GetForcesAndEnergies", "GetVirials"):
+        np.testing.assert_array_equal(getattr(a, get)(), getattr(b, get)(), err_msg=get)
+
+
 # tiles of 2x2x2, 4x2x2, 4x4x2 and 4x4x4 cells
 @pytest.mark.parametrize("n", [9001, 33001, 66001, 130001])
 def test_sorted_lists_and_steps_at_each_tile_shape(n):
