@@ -240,13 +240,23 @@ __device__ __forceinline__ void list_f64(const PosD& pi, uint32_t i, uint32_t nn
 // close behind (64 bytes a pair).  At KA N = 32,768 56.5 -> 20.6 us in 216 tiles
 // against one lane per particle walking 2-byte entries (19.3 in the 726 smaller
 // tiles a sample of this size has); 24.4 us with 32-byte records in LDS.
-constexpr uint32_t kBlockF64 = 512;
-// Tiles of up to 128 particles on average fill fewer lanes (eight to a particle
-// at most), and the smaller workgroup lets one more share a CU.  384 against 512
-// lanes: 14.0 / 16.0 us at 18 particles a tile (n = 9,000), 19.3 / 22.4 at 45
-// (32,768), 28.2 / 28.3 at 87 (60,000), but 36.4 / 30.9 at 215 (110,000).
-constexpr uint32_t kBlockF64Small = 384;
-constexpr uint32_t kSmallTileF64 = 128;
+//
+// The workgroup's size goes by the mean number of particles in a tile.  Where
+// the tiles are few (four workgroups per CU), 384 lanes for up to 128 particles,
+// else 512.  384 against 512 lanes: 14.0 / 16.0 us at 18 particles a tile (KA n =
+// 9,000), 19.3 / 22.4 at 45 (32,768), 28.2 / 28.3 at 87 (60,000), but 36.4 / 30.9 at
+// 215 (110,000); 256 lanes 13.6 for 11.5 at 23 (12,000).  Where they are many, lanes
+// without a particle only hold back other workgroups: the smallest power of two
+// with two lanes for each.  Such a workgroup against 384 lanes, LJ: 98 / 392 us at
+// 1,000,000 particles cut at 1.2 (46,656 tiles of 21), 23 / 57 at 200,000 cut at 1.5
+// (4,913 of 41), 129 / 197 at 1,000,000 cut at 2.0 (12,167 of 82).
+constexpr uint32_t kFewTilesF64 = 1024;
+
+uint32_t block_f64(uint32_t n, uint32_t ntiles) {
+  const auto holds = [&](uint32_t per_tile) { return n <= static_cast<uint64_t>(per_tile) * ntiles; };
+  if (ntiles <= kFewTilesF64) return holds(128) ? 384u : 512u;
+  return holds(32) ? 64u : holds(64) ? 128u : holds(128) ? 256u : 512u;
+}
 
 template <int CUT, bool STR, bool INIT, uint32_t BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_lj_tiles_f64(
@@ -400,10 +410,13 @@ int launch_f64(const rumdx_particles* p, const rumdx_nblist* nb, const float* pa
                          reinterpret_cast<const uint4*>(nb->tile_info_dev), nb->tile_halo_dev, nb->halo_cap, cap, fb,
                          p->nvp, nb->max_nbrs, split);
     };
-    if (p->n <= static_cast<uint64_t>(kSmallTileF64) * nb->ntiles)
-      launch(k_lj_tiles_f64<CUT, STR, INIT, kBlockF64Small>, kBlockF64Small);
-    else
-      launch(k_lj_tiles_f64<CUT, STR, INIT, kBlockF64>, kBlockF64);
+    switch (block_f64(p->n, nb->ntiles)) {
+      case 64: launch(k_lj_tiles_f64<CUT, STR, INIT, 64>, 64); break;
+      case 128: launch(k_lj_tiles_f64<CUT, STR, INIT, 128>, 128); break;
+      case 256: launch(k_lj_tiles_f64<CUT, STR, INIT, 256>, 256); break;
+      case 384: launch(k_lj_tiles_f64<CUT, STR, INIT, 384>, 384); break;
+      default: launch(k_lj_tiles_f64<CUT, STR, INIT, 512>, 512); break;
+    }
   } else {
     // a wave per particle over all pairs; 16 lanes over a list (some 90
     // entries), so that a sample of a thousand particles fills the CUs

@@ -303,6 +303,22 @@ def test_fused_steps_on_both_sides_of_their_rule(n, rcut, fused):
         np.testing.assert_array_equal(getattr(a, get)(), getattr(b, get)(), err_msg=get)
 
 
+# the FP64 tile kernel's workgroups of 64 to 512 lanes: few tiles (864, 729 and 512)
+# and many (1,331 or more), by the particles in a tile
+@pytest.mark.parametrize("n,rcut,tiles", [(9000, 1.5, 864), (30001, 1.5, 729), (130001, 2.5, 1000),
+                                          (30001, 1.2, 1331), (45001, 1.5, 1331), (90001, 2.0, 1331),
+                                          (200001, 2.5, 1331)])
+def test_fp64_forces_at_each_number_of_lanes(n, rcut, tiles):
+    s, pot, _itg, pos4, box = _short_ranged(n, rcut)
+    pot.SetFP64Forces(True)
+    print(f"[case] fp64 lanes n={n} rcut={rcut}", flush=True)
+    s.CalcF()
+    assert pot.GetNbTileStats()["tiles"] == tiles
+    table = configs.lj_param_table([(0, 0, 1.0, 1.0, rcut)], 1)
+    f_ref, _ = oracle.forces_cells(pos4, box, 1, table, SF)
+    assert force_errors(s.GetForces(), f_ref[:, :3])["guarded_max"] <= 2e-7  # as for all FP64 forces
+
+
 # tiles of 2x2x2, 4x2x2, 4x4x2 and 4x4x4 cells
 @pytest.mark.parametrize("n", [9001, 33001, 66001, 130001])
 def test_sorted_lists_and_steps_at_each_tile_shape(n):
