@@ -76,9 +76,9 @@ __device__ __forceinline__ double rsqrt_f64(double x) {
 // One pair; WRAP: the displacement needs the minimum image.  The pair term is
 // formed for every pair, so that a group's pairs overlap, and added only inside
 // rc: a masked factor of zero would still carry an infinite or undefined
-// coordinate into the sums (0 x NaN).  19.7 us at KA N = 32,768 (19.3 masked,
-// 20.0 with the displacements masked as well).  Below kTinyD2 (coincident
-// particles) the iteration of rsqrt_f64 has no start; r^-12 is infinite there.
+// coordinate into the sums (0 x NaN).  19.0 us at KA N = 32,768 either way (20.0
+// with the displacements masked as well).  kTinyD2 is added in d2's first product:
+// the iteration of rsqrt_f64 has no start at zero, and r^-12 is infinite there.
 constexpr double kTinyD2 = 1e-300;
 
 template <int CUT, bool STR, bool WRAP>
@@ -90,9 +90,9 @@ __device__ __forceinline__ void pair_f64(const PosD& pi, const PosD& pj, const d
     dy -= bx.Ld[1] * rint(dy * bx.iLd[1]);
     dz -= bx.Ld[2] * rint(dz * bx.iLd[2]);
   }
-  const double d2 = dx * dx + dy * dy + dz * dz;
+  const double d2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, kTinyD2)));
   const double* t = trow + kTabD * pj.t;
-  const double rinv = rsqrt_f64(fmax(d2, kTinyD2)), inv2 = rinv * rinv, inv6 = inv2 * inv2 * inv2;
+  const double rinv = rsqrt_f64(d2), inv2 = rinv * rinv, inv6 = inv2 * inv2 * inv2;
   const double x = t[1] * inv6;  // A12 / r^6
   double s = 6.0 * inv6 * inv2 * fma(2.0, x, t[2]);
   double u = inv6 * (x + t[2]);

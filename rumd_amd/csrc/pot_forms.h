@@ -48,30 +48,50 @@ RUMDX_HD double pf_rcp(double x) { return 1.0 / x; }
 RUMDX_HD double pf_sqrt(double x) { return sqrt(x); }
 // On the device 1/x and sqrt(x) are the hardware estimates refined by one
 // Newton step: as close to the exact value as a correctly rounded result but
-// for cases within a few 1e-3 of a tie, at 4 and 6 operations instead of the
-// 10 and more of the divide and square root sequences.  One operation of each
-// is for the values the step cannot refine, which coincident particles bring
-// about: v_div_fixup sets 1/0 and 1/infinity, and a root's estimate held finite
-// gives sqrt(0) = 0; forces of Buckingham N = 30,011 take 17.8 us with them, 17.3
-// without.  pf_sqrt takes a finite x (pf_finite makes it so).
-RUMDX_HD float pf_rcp(float x) {
+// for cases within a few 1e-3 of a tie, at 3 and 5 operations instead of the
+// 10 and more of the divide and square root sequences, for a positive finite x
+// (pf_rcp_pos, pf_sqrt_pos).  pf_rcp and pf_sqrt take one operation more for
+// the values the step cannot refine, which coincident particles bring about:
+// v_div_fixup sets 1/0 and 1/infinity, and a root's estimate held finite gives
+// sqrt(0) = 0.  pf_finite keeps the reciprocal of such a distance finite.
+RUMDX_HD double pf_rcp_pos(double x) { return 1.0 / x; }
+RUMDX_HD double pf_sqrt_pos(double x) { return sqrt(x); }
+RUMDX_HD double pf_finite(double x) { return x; }
+constexpr float kPfMax = 3.402823466e+38f;
+RUMDX_HD float pf_finite(float x) { return fminf(x, kPfMax); }
+RUMDX_HD float pf_rcp_pos(float x) {
 #ifdef __HIP_DEVICE_COMPILE__
   const float y = __builtin_amdgcn_rcpf(x);
-  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-x, y, 1.f), y, y), x, 1.f);
+  return fmaf(fmaf(-x, y, 1.f), y, y);
 #else
   return 1.f / x;
 #endif
 }
-RUMDX_HD float pf_sqrt(float x) {
+RUMDX_HD float pf_rcp(float x) {
 #ifdef __HIP_DEVICE_COMPILE__
-  const float y = fminf(__builtin_amdgcn_rsqf(x), 3.402823466e+38f), q = x * y;
+  return __builtin_amdgcn_div_fixupf(pf_rcp_pos(x), x, 1.f);
+#else
+  return 1.f / x;
+#endif
+}
+RUMDX_HD float pf_sqrt_from(float x, float y) {  // y: the estimate of 1/sqrt(x)
+  const float q = x * y;
   return fmaf(fmaf(-q, q, x), 0.5f * y, q);
+}
+RUMDX_HD float pf_sqrt_pos(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return pf_sqrt_from(x, __builtin_amdgcn_rsqf(x));
 #else
   return sqrtf(x);
 #endif
 }
-RUMDX_HD float pf_finite(float x) { return fminf(x, 3.402823466e+38f); }
-RUMDX_HD double pf_finite(double x) { return x; }
+RUMDX_HD float pf_sqrt(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return pf_sqrt_from(x, fminf(__builtin_amdgcn_rsqf(x), kPfMax));
+#else
+  return sqrtf(x);
+#endif
+}
 
 // Every form, for code that instantiates or dispatches over them.
 #define RUMDX_ALL_FORMS(X)                                                                                        \
@@ -112,8 +132,8 @@ RUMDX_HD T pot_form_of(T d2, const T* p, T& u) {
     case RUMDX_POT_BUCKINGHAM: {
       // v = eps (6/(alpha-6) exp(alpha (1 - r/rm)) - alpha/(alpha-6) (rm/r)^6)
       const T i2 = pf_rcp(d2 * p[1]), i6 = i2 * i2 * i2;
-      const T i1 = pf_sqrt(pf_finite(i2));
-      const T e = pf_exp(p[2] * (one - pf_rcp(i1)));
+      const T i1 = pf_sqrt_pos(pf_finite(i2));
+      const T e = pf_exp(p[2] * (one - pf_rcp_pos(i1)));
       u = p[3] * e - p[4] * i6;
       return p[1] * p[5] * (i1 * e - i6 * i2);
     }
@@ -157,7 +177,7 @@ RUMDX_HD T pot_form_of(T d2, const T* p, T& u) {
         in = i6 * i6;
       } else if (FORM == RUMDX_POT_IPL_9) {
         const T i4 = i2 * i2;
-        in = i4 * i4 * pf_sqrt(pf_finite(i2));
+        in = i4 * i4 * pf_sqrt_pos(pf_finite(i2));
       } else {
         const T i6 = i2 * i2 * i2;
         in = i6 * i6 * i6;
