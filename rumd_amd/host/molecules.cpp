@@ -118,13 +118,10 @@ void MoleculeData::SetDihedrals(const std::vector<uint32_t>& abcdt) {
   UploadDihedrals();
 }
 
-unsigned MoleculeData::GetNumberOfDihedralTypes() const {
-  unsigned t = 0;
-  for (size_t k = 4; k < dihedrals_.size(); k += 5) t = std::max(t, dihedrals_[k] + 1);
-  return t;
-}
-
 void MoleculeData::UploadDihedrals() {
+  num_dihedral_types_ = 0;
+  for (size_t k = 4; k < dihedrals_.size(); k += 5)
+    num_dihedral_types_ = std::max(num_dihedral_types_, dihedrals_[k] + 1);
   const unsigned n = sample_->GetNumberOfParticles();
   std::vector<std::vector<uint32_t>> per(n);
   for (size_t k = 0; k < dihedrals_.size(); k += 5)
@@ -143,12 +140,6 @@ void MoleculeData::UploadDihedrals() {
 unsigned MoleculeData::GetNumberOfBondTypes() const {
   unsigned t = 0;
   for (size_t k = 2; k < bonds_.size(); k += 3) t = std::max(t, bonds_[k] + 1);
-  return t;
-}
-
-unsigned MoleculeData::GetNumberOfAngleTypes() const {
-  unsigned t = 0;
-  for (size_t k = 3; k < angles_.size(); k += 4) t = std::max(t, angles_[k] + 1);
   return t;
 }
 
@@ -175,6 +166,8 @@ void MoleculeData::UploadBonds() {
 }
 
 void MoleculeData::UploadAngles() {
+  num_angle_types_ = 0;
+  for (size_t k = 3; k < angles_.size(); k += 4) num_angle_types_ = std::max(num_angle_types_, angles_[k] + 1);
   const unsigned n = sample_->GetNumberOfParticles();
   std::vector<std::vector<uint32_t>> per(n);
   for (size_t k = 0; k < angles_.size(); k += 4) {

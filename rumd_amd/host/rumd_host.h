@@ -618,7 +618,8 @@ class MoleculeData {
   // Replaces the dihedrals: flat (a, b, c, d, type) quintuples.
   void SetDihedrals(const std::vector<uint32_t>& abcdt);
   unsigned GetNumberOfDihedrals() const { return static_cast<unsigned>(dihedrals_.size() / 5); }
-  unsigned GetNumberOfDihedralTypes() const;
+  // (asked for at every step: counted when the terms are set)
+  unsigned GetNumberOfDihedralTypes() const { return num_dihedral_types_; }
   const std::vector<uint32_t>& GetDihedrals() const { return dihedrals_; }
   const uint32_t* DihedralStart() const { return dihedral_start_.get(); }
   const uint32_t* DihedralAtoms() const { return dihedral_atoms_.get(); }
@@ -626,7 +627,7 @@ class MoleculeData {
   unsigned GetNumberOfAngles() const { return static_cast<unsigned>(angles_.size() / 4); }
   unsigned GetNumberOfMolecules() const { return num_mol_; }
   unsigned GetNumberOfBondTypes() const;
-  unsigned GetNumberOfAngleTypes() const;
+  unsigned GetNumberOfAngleTypes() const { return num_angle_types_; }
   const std::vector<uint32_t>& GetBonds() const { return bonds_; }
   const std::vector<uint32_t>& GetAngles() const { return angles_; }
   // Refreshes slot_of from the particles' unsorted index (on the sample's stream).
@@ -646,6 +647,7 @@ class MoleculeData {
   Sample* sample_;
   unsigned num_mol_ = 0;
   std::vector<uint32_t> bonds_, angles_, dihedrals_;
+  uint32_t num_angle_types_ = 0, num_dihedral_types_ = 0;
   uint64_t slot_epoch_ = 0;  // sample epoch of the last slot index
   DeviceArray<uint32_t> bond_start_, bond_other_, bond_type_, angle_start_, angle_atoms_, slot_of_;
   DeviceArray<uint32_t> dihedral_start_, dihedral_atoms_;
