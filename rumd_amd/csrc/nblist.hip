@@ -1244,7 +1244,7 @@ __global__ __launch_bounds__(kBuildBlock) void k_build_tiles(uint32_t* __restric
     const bool small_box = (tg.origin[t] >> 30) != 0u && min(min(nc[0], nc[1]), nc[2]) < kShiftMinCells;
     bool shiftable = !small_box;
     for (int a = 0; a < 3; ++a) {
-      const bool below = h.base[a] < 0, above = h.base[a] + h.ext[a] > nc[a];
+      const bool below = h.base[a] < 0, above = h.base[a] + h.own[a] + 4 > nc[a];
       if (below) fl |= kTileShiftDown << (2 * a);
       if (above) fl |= kTileShiftUp << (2 * a);
       shiftable = shiftable && ((!below && !above) || (nc[a] >= kShiftMinCells && h.ext[a] < nc[a] &&

@@ -88,7 +88,7 @@ struct Halo {
   int base[3];   // first halo cell coordinate (may be negative: periodic)
   int ext[3];    // halo cells per axis (<= 8, <= nc)
   int own[3];    // the tile's own cells per axis (<= 4); they sit at halo index 2..2+own-1
-  bool wraps;    // some halo cell lies across the periodic boundary
+  bool wraps;    // some halo cell lies across the periodic boundary from a cell of the tile
   uint32_t ncell;
   uint32_t npart;  // particles in the halo
   uint32_t slot0, slot1;  // the tile's own slots
@@ -172,7 +172,9 @@ __device__ __forceinline__ void stage_halo(uint32_t t, const TileGeom& g, const 
       L.h.base[a] = c0[a] - 2;
       L.h.ext[a] = ext;
       L.h.own[a] = bw;
-      wraps = wraps || (c0[a] - 2 < 0) || (c0[a] - 2 + ext > nc[a]);
+      // (a halo of the whole axis holds each cell once, and a stencil of its own
+      // cells reaches some of them across the boundary: two cells of an axis of five)
+      wraps = wraps || (c0[a] - 2 < 0) || (c0[a] - 2 + ext > nc[a]) || bw + 4 > nc[a];
       ncell *= static_cast<uint32_t>(ext);
     }
     L.h.wraps = wraps;

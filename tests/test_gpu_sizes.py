@@ -285,6 +285,47 @@ def test_forces_at_each_number_of_lanes(n, rcut, tiles):
     assert force_errors(f[:, :3], f_ref[:, :3])["guarded_max"] <= FORCE_TOL_GUARDED
 
 
+# axes of five cells, where a tile's halo holds the box once and its stencils still
+# wrap, of six and seven, alone and with long ones, in every shape of tile
+@pytest.mark.parametrize("box", [(6.9, 6.9, 6.9), (8.5, 8.5, 8.5), (9.9, 9.9, 9.9), (7.0, 8.5, 9.9),
+                                 (56.0, 56.0, 7.0), (56.0, 7.0, 56.0), (7.0, 56.0, 56.0), (56.0, 56.0, 8.5),
+                                 (30.0, 7.0, 7.5), (140.0, 140.0, 7.0), (17.0, 17.0, 7.0)])
+def test_sorted_lists_and_forces_in_boxes_of_few_cells(box):
+    rng = np.random.default_rng(17)
+    box = np.array(box)
+    k = np.floor(box / 1.12).astype(int)
+    n = int(k.prod())
+    site = np.stack(np.meshgrid(*[np.arange(m) for m in k], indexing="ij"), axis=-1).reshape(-1, 3)
+    pos = ((site + 0.5) * (box / k) - 0.5 * box + rng.uniform(-0.15, 0.15, size=(n, 3))).astype(np.float32)
+    sample = rumd.Sample(0, 0)
+    sample.SetVerbose(False)
+    sample.SetConfiguration(conf_io.Configuration(
+        n=n, box=box, types=np.zeros(n, np.int32), positions=pos, masses=np.ones(1),
+        velocities=rng.normal(size=(n, 3)), images=np.zeros((n, 3))))
+    pot = rumd.Pot_LJ_12_6(cutoff_method=rumd.ShiftedForce)
+    pot.SetVerbose(False)
+    pot.SetParams(0, 0, Sigma=1.0, Epsilon=1.0, Rcut=2.5)
+    pot.SetNbListSkin(0.3)
+    pot.SetNB_Method("sort")
+    sample.SetPotential(pot)
+    itg = rumd.IntegratorNVE(timeStep=0.002)
+    sample.SetIntegrator(itg)
+    table = configs.lj_param_table([(0, 0, 1.0, 1.0, 2.5)], 1)
+    b8 = configs.box8(box)
+    print(f"[case] few cells {box.tolist()} n={n}", flush=True)
+    for steps in (0, 12):  # the full sort and, with a rebuild asked for, the tile re-sort
+        sample.RunSteps(0, steps, 6, 0)
+        if steps:
+            sample.SortParticles()
+        sample.CalcF()
+        pos4 = configs.pack_pos4(sample.GetPositions(), np.zeros(n, np.int32))
+        off, idx = oracle.nblist_brute_f32(pos4, b8, 1, configs.cut_skin2_table(table, 0.3))
+        got_off, got_idx = pot.GetNeighborListCSR(sample)
+        assert np.array_equal(sorted_rows(got_off, got_idx), sorted_rows(off, idx))
+        f_ref, _ = oracle.forces_nl(pos4, box, 1, table, SF, off, idx)
+        assert force_errors(sample.GetForces(), f_ref[:, :3])["guarded_max"] <= FORCE_TOL_GUARDED
+
+
 # both sides of the fused steps' rule: at most 1,024 tiles, or 64 particles a tile;
 # the same bits either way
 @pytest.mark.parametrize("n,rcut,fused", [(20000, 2.0 ** (1.0 / 6.0), True), (30000, 2.0 ** (1.0 / 6.0), False),
