@@ -271,6 +271,7 @@ rumdx_replica ReplicaBatch::HostReplica(unsigned r) const {
 // Thermostat states restart at Ps = 0.
 void ReplicaBatch::Allocate() {
   flags_changed_ = true;
+  lists_grown_ = false;
   if (reps_.empty()) throw RUMD_Error("ReplicaBatch", "Allocate", "no replicas");
   if (table_.empty()) throw RUMD_Error("ReplicaBatch", "Allocate", "no potential set");
   const unsigned nrep = static_cast<unsigned>(reps_.size());
@@ -437,6 +438,7 @@ void ReplicaBatch::Allocate() {
 void ReplicaBatch::CalcF() {
   flags_changed_ = true;
   if (!allocated_) Allocate();
+  lists_grown_ = false;
   rumdx_check(rumdx_batch_update_lists(&desc_, stream_), "ReplicaBatch", "CalcF");
   rumdx_check(rumdx_batch_forces(&desc_, params_.get(), cutoff_method_, stream_), "ReplicaBatch", "CalcF");
 }
@@ -458,6 +460,7 @@ float ReplicaBatch::TimeForceKernel(unsigned reps) {
   flags_changed_ = true;
   if (!allocated_) Allocate();
   if (reps == 0) reps = 1;
+  lists_grown_ = false;
   rumdx_check(rumdx_batch_update_lists(&desc_, stream_), "ReplicaBatch", "TimeForceKernel");
   hipEvent_t a, b;
   hip_check(hipEventCreate(&a), "ReplicaBatch", "TimeForceKernel");
@@ -499,6 +502,7 @@ void ReplicaBatch::RunSteps(unsigned nsteps, unsigned block) {
   flags_changed_ = true;
   if (!allocated_) Allocate();
   if (block == 0) block = 1;
+  if (nsteps) lists_grown_ = false;  // the first step brings the lists up to date
   unsigned done = 0;
   while (done < nsteps) {
     if (block == 1 || done + block > nsteps) {
@@ -555,6 +559,7 @@ void ReplicaBatch::Synchronize() {
   nbl_.resize(static_cast<size_t>(max_nbrs_) * nslots_);
   desc_.nbl_dev = nbl_.get();
   desc_.max_nbrs = max_nbrs_;
+  lists_grown_ = true;
   for (size_t r = 0; r < reps_.size(); ++r) {
     fl[RUMDX_BATCH_FLAGS * r] = 1u;  // rebuild
     fl[RUMDX_BATCH_FLAGS * r + 1] = 0u;
@@ -623,6 +628,10 @@ void ReplicaBatch::GetNeighborList(unsigned replica, std::vector<uint32_t>& offs
   if (!allocated_) Allocate();
   if (replica >= reps_.size()) throw RUMD_Error("ReplicaBatch", "GetNeighborList", "replica index out of range");
   Synchronize();
+  while (lists_grown_) {  // the lengths on the device are those of the lists before
+    CalcF();
+    Synchronize();
+  }
   const unsigned n = GetNumberOfParticles(replica);
   const uint32_t s0 = slot0_[replica];
   std::vector<uint32_t> cnt(n);

@@ -89,6 +89,8 @@ class ReplicaBatch {
   // {mean, longest} list length over the real particles of every replica.
   std::vector<double> GetNeighborListStats();
   // Neighbour list of one replica in replica-local ids: CSR (offsets n + 1, ids).
+  // After an overflow has grown the lists, those are built first, and the
+  // forces of the current positions with them.
   void GetNeighborList(unsigned replica, std::vector<uint32_t>& offsets, std::vector<uint32_t>& ids);
   hipStream_t GetStream() const { return stream_; }
 
@@ -117,6 +119,7 @@ class ReplicaBatch {
   unsigned user_max_nbrs_ = 0, max_nbrs_ = 0, lanes_per_particle_ = 1;
   bool saved_ = false;
   bool flags_changed_ = true;  // work that may change the flags was launched since they were read
+  bool lists_grown_ = false;   // the lists were reallocated after an overflow and not built since
   OriginalOrderReader reader_;
   bool allocated_ = false;
   bool staged_forces_ = true;

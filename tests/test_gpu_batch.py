@@ -153,6 +153,25 @@ def test_batch_overflowed_lists_still_exact():
     assert err["guarded_max"] <= FORCE_TOL_GUARDED, err
 
 
+def test_batch_lists_read_after_an_overflow():
+    """Lists read right after an overflow has grown them are the whole lists,
+    not what the new memory holds under the old lengths."""
+    systems = _systems([1000, 1500], seed0=720)
+    b = make_batch(systems, [0.5, 0.5], max_nbrs=24)
+    print("[case] batch lists after an overflow", flush=True)
+    b.CalcF()
+    cut2 = configs.cut_skin2_table(ka_table(), 0.3)
+    for r, s in enumerate(systems):
+        off, ids = b.GetNeighborListCSR(r)
+        b8 = configs.box8(s.box)
+        o2, i2 = oracle.nblist_cells_f32(configs.pack_pos4(s.positions, s.types), b8, 2, cut2,
+                                         oracle.cell_grid(b8, 2.5, 0.3))
+        assert np.array_equal(off, o2), r
+        for i in range(s.n):
+            assert set(ids[off[i]:off[i + 1]].tolist()) == set(i2[o2[i]:o2[i + 1]].tolist()), (r, i)
+    assert b.GetMaxNumNbrs() > 24
+
+
 def test_batch_hot_replicas_rebuild_more_often():
     systems = _systems([2000, 2000], seed0=100)
     b = make_batch(systems, [0.4, 2.0])
