@@ -848,11 +848,12 @@ __global__ __launch_bounds__(kBlock) void k_b_force(BatchArgs a, const uint32_t*
 // with more lanes the forces go through memory first.  kStepInner leaves
 // forces, energies and virials out, for a step whose forces the next one
 // replaces before anything can read them.
-// VALU issue bounds the pair terms (76 % of cycles measured).  512 replicas of
-// 261 to 8,186 particles (2.15 million), shifted forces: 291 us a step for
-// kStepInner and 315 for kStepStore, the thermostats included; 355 before, as
-// two launches with rounded displacements, energies always computed and the
-// update after all of a replica's pair terms.
+// VALU issue bounds the pair terms (busy 71 % of a kStepInner launch, 79 % with
+// kStepStore and 89 % for the forces alone).  512 replicas of 261 to 8,186
+// particles (2.15 million), shifted forces: 282 us a step for kStepInner and
+// 308 for kStepStore, the thermostats included; 355 before, as two launches
+// with rounded displacements, energies always computed and the update after all
+// of a replica's pair terms.
 constexpr uint32_t kStagedBlock = 1024;
 static_assert(kStagedBlock <= kMaxWorkgroup, "staged force workgroup");
 static_assert(kStagedBlock % kBlock == 0, "whole integrator blocks per pass");

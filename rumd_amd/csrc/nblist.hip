@@ -148,7 +148,7 @@ __global__ void k_request_rebuild(uint32_t* flags) {
 // waves; the next ones are read while these are tested.  Bound by the VALU
 // work of the n^2 tests; with a thread per particle it was the serial walk of
 // n / 256 workgroups over all n candidates (207 -> 10 us at n = 1000,
-// 845 -> 36 us at n = 5001).  Two or four particles per wave share each LDS
+// 845 -> 38 us at n = 5001).  Two or four particles per wave share each LDS
 // read but leave too few waves in flight (47 and 80 us at n = 5001).
 //
 // Arrivals are counted at the block's start, after its request read, so the
@@ -1240,7 +1240,8 @@ __global__ __launch_bounds__(kBuildBlock) void k_build_tiles(uint32_t* __restric
     uint32_t fl = 0;
     // A small box in small tiles (shape above 0) keeps FP64 displacements for
     // every tile: in 4^3 tiles nearly all of them wrapped and had them, and at
-    // these sizes they are not what the force kernel's time goes into.
+    // these sizes they are not what the force kernel's time goes into (KA at
+    // n = 9,000 in 14^3 cells: 12.6 us a fused step kernel with and without).
     const bool small_box = (tg.origin[t] >> 30) != 0u && min(min(nc[0], nc[1]), nc[2]) < kShiftMinCells;
     bool shiftable = !small_box;
     for (int a = 0; a < 3; ++a) {
@@ -1691,8 +1692,8 @@ extern "C" int rumdx_tile_shape(const int32_t nc[3]) {
   // The smallest tiles that do not exceed kTilesWanted.  The re-sort, build and
   // force kernels run one workgroup per tile, up to five to a CU (256 CUs):
   // with fewer tiles CUs idle and a tile's serial work is the kernel's time,
-  // with more the halo staged per particle grows (2.1 times the tile's own
-  // cells per halved axis at worst).  us per step at N = 12,000, shapes 0-3: 36
+  // with more the halo staged per particle grows (8, 12, 18 and 27 halo cells
+  // per own cell for shapes 0-3).  us per step at N = 12,000, shapes 0-3: 36
   // (64 tiles), 26, 24, 22 (512); 32,768: 40 (216), 34, 30 (726), 33 (1331);
   // 65,536: 37 (343), 32 (686), 36 (1372), 45; 200,000: 51 (1000), 58 (2000), 71.
   constexpr uint64_t kTilesWanted = 900;

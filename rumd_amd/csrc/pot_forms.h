@@ -58,8 +58,8 @@ RUMDX_HD double pf_rcp_pos(double x) { return 1.0 / x; }
 RUMDX_HD double pf_sqrt_pos(double x) { return sqrt(x); }
 // pf_mul_nonzero adds the smallest normal number to a product of squares: at no
 // cost, and without effect above 1e-30, its reciprocal stays finite at zero and
-// the powers of that overflow as those of 1/0 would (1.2 % of a Buckingham step
-// at n = 30,011 against v_div_fixup and pf_finite).
+// the powers of that overflow as those of 1/0 would (30 Buckingham steps at
+// n = 30,011: 1,066 us with v_div_fixup and pf_finite, 1,057 so).
 RUMDX_HD double pf_mul_nonzero(double x, double y) { return x * y; }
 RUMDX_HD float pf_mul_nonzero(float x, float y) { return fmaf(x, y, 1.175494351e-38f); }
 RUMDX_HD double pf_finite(double x) { return x; }

@@ -11,7 +11,10 @@
 // A small sample's step is bound by launches and by the chain of dependent
 // reads, not by work: four kernels (build, forces, integrator, thermostat) took
 // 13 us a step at n = 500 without a list, 18 at n = 1000 and 19 at n = 4099,
-// most of it between them; one takes 7.5, 8.4 and 12 (rebuilds included).
+// most of it between them; one takes 7.5, 8.4 and 12 (rebuilds included).  The
+// host class takes it over N2 lists of at most 5,000 particles: above, the
+// build's O(n^2) scan is the step's time and the four kernels' build is faster
+// at it.
 // None of the four needs a grid-wide barrier inside a step:
 //  - a list of the N2 method belongs to one particle and is built from the
 //    positions alone, so the workgroup that owns the particle rebuilds it when
